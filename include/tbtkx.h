@@ -316,7 +316,8 @@ int tbtkx_multi_moments(tbtkx_handle handle, const int *num_sites,
 
 /* Device time of the last recurrence call: total milliseconds between the
  * first and last step launch (HIP events on the handle's stream) and the
- * number of step launches in it. */
+ * number of steps in it (one launch each, or all in one launch where the
+ * recurrence ran resident, TBTKX_OPT_RESIDENT). */
 int tbtkx_last_timing(tbtkx_handle handle, double *milliseconds,
                       int64_t *launches);
 
@@ -406,7 +407,14 @@ enum {
 	                           outside 64-row chunks of one shared pattern
 	                           (the rows whose pattern byte the step reads
 	                           with TBTKX_OPT_ROW_PATTERNS = 1); -1 when the
-	                           model has no row patterns */
+	                           model has no row patterns */,
+	TBTKX_OPT_RESIDENT = 21 /* 1 = the plain recurrence runs all its steps in
+	                           one launch with the vectors resident on the
+	                           chip, where the model fits and that is faster
+	                           (default; not with TBTKX_OPT_GRAPH or options
+	                           that choose a form of the per-step kernel):
+	                           same moments; 0 = a launch per step. Reading it
+	                           gives 1 when the last plain call ran resident */
 };
 int tbtkx_set_option(tbtkx_handle handle, int option, int64_t value);
 

@@ -22,6 +22,7 @@
 // Algorithmic HBM bytes per step (FP32 vectors, FP32 H):
 //   12 Z (value + column) + 4 N (row pointer) + 24 B N (read Phi_n, read
 //   Phi_{n-1}, write Phi_{n+1}, 8 B each per element).
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <cstring>
@@ -1475,6 +1476,61 @@ int run_exact(tbtkx_context *h, int nvec, const int64_t *from, const std::vector
 	return TBTKX_OK;
 }
 
+// tbtkx_moments_multi with the model in one workgroup's LDS (resident.hip): a
+// workgroup per start vector, in launches whose moments take at most 512 MiB.
+// Entry l of the gather list (ordered by vector, rows ascending) is output row
+// gslot[l] of T; rows without an entry are zero.
+int run_resident(tbtkx_context *h, const ResidentPlan &plan, int nvec, const int64_t *from,
+                 const std::vector<int64_t> &grow, const std::vector<int> &gvec,
+                 const std::vector<int> &gslot, int T, int M, double *out) {
+	const size_t row = (size_t)M * 16, most = std::max<size_t>(1, ((size_t)512 << 20) / row);
+	const size_t L = grow.size();
+	const bool direct = L == (size_t)T && std::is_sorted(gslot.begin(), gslot.end());
+	if (!direct) memset(out, 0, (size_t)T * row);
+	std::vector<double2> buf;
+	std::vector<int> toff;
+	double ms_all = 0;
+	size_t l = 0;
+	for (int v = 0; v < nvec;) {
+		const int v0 = v;
+		const size_t l0 = l;
+		toff.assign(1, 0);
+		// At least one vector, then as many as fit.
+		do {
+			while (l < L && gvec[l] == v) l++;
+			toff.push_back((int)(l - l0));
+			v++;
+			size_t e = l;
+			while (v < nvec && e < L && gvec[e] == v) e++;
+			if (e - l0 > most) break;
+		} while (v < nvec && v - v0 < 65535);
+		if (l == l0) continue;
+		TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
+		int rc = resident_moments(h, plan, v - v0, from + v0, toff.data(), grow.data() + l0, M);
+		if (rc) return rc;
+		TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
+		void *dst = out + l0 * M * 2;
+		if (!direct) {
+			buf.resize((l - l0) * M);
+			dst = buf.data();
+		}
+		TBTKX_CHECK_HIP(hipMemcpyAsync(dst, h->coef.ptr, (l - l0) * row, hipMemcpyDeviceToHost,
+		                               h->stream));
+		TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
+		if (!direct)
+			for (size_t e = l0; e < l; e++)
+				memcpy(out + (size_t)gslot[e] * M * 2, buf.data() + (e - l0) * M, row);
+		float ms = 0;
+		TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
+		ms_all += ms;
+	}
+	h->last_ms = ms_all;
+	h->last_launches = M > 1 ? M - 1 : 0;
+	h->last_real = h->real_path && h->h_real;
+	h->last_resident = 1;
+	return TBTKX_OK;
+}
+
 // Algorithmic HBM bytes of the whole call: plain recurrences (one per start
 // vector, in the plain kernel's current form) or exact FP64 blocks of width
 // B (20 Z + 4 N for FP64 H and row pointers, 48 B N for the three block
@@ -1607,6 +1663,7 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 	if (T == 0) return TBTKX_OK;
 	int rc = set_device(h);
 	if (!rc) rc = build_plain_forms(h);
+	if (!rc && h->plain_kernel == 2 && !(h->use_palette && h->slot_pal)) rc = build_slot_values(h);
 	if (rc) return rc;
 	const int packed = h->real_path && h->h_real;
 	int B = 64;
@@ -1616,7 +1673,11 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 	bool blocks = h->multi_mode == 2 ||
 	              (h->multi_mode == 0 &&
 	               block_call_bytes(h, num_from, B, packed) < plain_call_bytes(h, num_from));
-	if (!blocks) {
+	// A model that fits one workgroup runs a workgroup per start vector, all
+	// in one launch: bitwise the same moments, and no vector in memory at all.
+	const ResidentPlan plan = resident_plan(h, h->num_cus);
+	const bool resident = h->multi_mode == 0 && num_from > 1 && plan.C == h->N;
+	if (!blocks && !resident) {
 		for (int j = 0; j < num_from; j++) {
 			const int k0 = to_offsets[j], k1 = to_offsets[j + 1];
 			if (k1 == k0) continue;
@@ -1639,6 +1700,11 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 			gvec.push_back(j);
 			gslot.push_back(kv.second);
 		}
+	}
+	if (resident) {
+		if ((rc = run_resident(h, plan, num_from, from, grow, gvec, gslot, T, M, out))) return rc;
+		h->last_multi_blocks = blocks;
+		return TBTKX_OK;
 	}
 	std::vector<double2> mu;
 	if (B == 64) rc = run_exact<64>(h, num_from, from, grow, gvec, M, packed, mu);

@@ -138,6 +138,7 @@ struct tbtkx_context {
 	// (slot_pal) or H/s, 2H/s values (complex, and real for a real H).
 	tbtkx::DevBuf scol, scode, sv1, sv2, sv1r, sv2r;
 	int slot_ok = 0, slot_pal = 0, slot_vals = 0, slot_W = 0;
+	int slot_half = 0;   // most entries on either side of a row's diagonal
 	// Row patterns of the slot form (pat_ok): one byte per row (ppid) into
 	// pat_count patterns of 8 offsets (ptoff) and 8 palette codes (ptcode).
 	tbtkx::DevBuf ppid, ptoff, ptcode;
@@ -154,6 +155,15 @@ struct tbtkx_context {
 
 	// Plain path vectors and moment output.
 	tbtkx::DevBuf vec_a, vec_b, coef, to;
+
+	// Resident recurrence (resident.hip): start vectors and to-lists, exchanged
+	// halo rows and the first unused tag, give-up flag.
+	tbtkx::DevBuf res_in, res_xg, res_err;
+	std::vector<int64_t> res_host;   // host copy of res_in, alive during its upload
+	uint32_t res_epoch = 0;
+	int use_resident = 1;
+	int last_resident = 0;   // the last plain call ran resident
+	int num_cus = 0;
 
 	// Lookup table L[n*E + e], complex double.
 	tbtkx::DevBuf lut;
@@ -262,7 +272,7 @@ int build_col16(tbtkx_context *h);
 
 // Builds the slot-major ELL form of the plain kernel from the resident CSR
 // and palette (plain.hip); `rowptr` is a host copy of the row pointer.
-int build_slots(tbtkx_context *h, const uint32_t *rowptr);
+int build_slots(tbtkx_context *h, const uint32_t *rowptr, const uint32_t *col);
 // Adds H/s and 2H/s values to the slots (for calls without the palette).
 int build_slot_values(tbtkx_context *h);
 // Builds the palette, the row patterns and the slot form of a device-built
@@ -298,6 +308,24 @@ inline PlainForm plain_form(const tbtkx_context *h) {
 		f.bytes = (e + (f.c16 ? 2 : 4)) * Z + N * (4 + 3 * e);
 	return f;
 }
+
+// The plain recurrence in one launch, the vectors resident on the chip
+// (resident.hip): C rows per workgroup (the whole model: one workgroup per start
+// vector), k steps between exchanges, estimated time of a step. C = 0: the
+// model does not fit or per-step launches are faster.
+struct ResidentPlan {
+	int C = 0, k = 1;
+	double us = 0;
+};
+ResidentPlan resident_plan(const tbtkx_context *h, int cus);
+// Enqueues the moments of V start vectors (V = 1 unless plan.C covers the
+// model) into h->coef, one row of M per entry of `to`; vector v's entries are
+// toff[v] .. toff[v + 1], ascending.
+int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *from,
+                     const int *toff, const int64_t *to, int M);
+// Whether the last launch gave up a wait (its moments are then incomplete);
+// waits for the stream.
+int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up);
 
 // Builds the plain kernel's value palette from host copies of the CSR
 // (v1 = H/s, v2 = 2H/s, interleaved complex); sets palette_ok when the

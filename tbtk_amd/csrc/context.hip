@@ -175,6 +175,8 @@ int tbtkx_create(int device, tbtkx_handle *handle) {
 	h->device = device;
 	hipError_t e = hipSetDevice(device);
 	if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
+	if (e == hipSuccess)
+		e = hipDeviceGetAttribute(&h->num_cus, hipDeviceAttributeMultiprocessorCount, device);
 	if (e == hipSuccess) e = hipEventCreate(&h->ev_start);
 	if (e == hipSuccess) e = hipEventCreate(&h->ev_stop);
 	if (e != hipSuccess) {
@@ -197,6 +199,7 @@ int tbtkx_destroy(tbtkx_handle h) {
 	                  &h->v1r, &h->v2r, &h->lat_terms, &h->lat_onsite, &h->lat_count,
 	                  &h->lat_part, &h->lat_tmp, &h->rblk, &h->col16, &h->col16_flag,
 	                  &h->pcode, &h->pal, &h->palr, &h->pdiag, &h->pdiagr, &h->scol, &h->scode, &h->sv1, &h->sv2, &h->sv1r, &h->sv2r, &h->ppid, &h->ptoff, &h->ptcode, &h->pchunk, &h->vec_a, &h->vec_b, &h->coef, &h->to,
+	                  &h->res_in, &h->res_xg, &h->res_err,
 	                  &h->lut, &h->gf_in, &h->gf_out, &h->dfac, &h->dden, &h->blk_x, &h->blk_y,
 	                  &h->blk_mu, &h->blk_sites, &h->blk_part, &h->blk_grow, &h->blk_gvec, &h->cplanes,
 	                  &h->lplanes, &h->gf_mfma_out, &h->ell_col, &h->ell_v1f,
@@ -364,7 +367,7 @@ int tbtkx_set_csr(tbtkx_handle h, int64_t N, int64_t Z, const uint32_t *rowptr,
 	if ((rc = build_col16(h))) return rc;
 	h->forms_pending = 0;
 	if ((rc = build_palette(h, N, Z, rowptr, col, v1.data(), v2.data()))) return rc;
-	return build_slots(h, rowptr);
+	return build_slots(h, rowptr, col);
 }
 
 int tbtkx_last_timing(tbtkx_handle h, double *ms, int64_t *launches) {
@@ -472,6 +475,11 @@ int tbtkx_set_option(tbtkx_handle h, int option, int64_t value) {
 		h->use_patterns = (int)value;
 		h->plain_graph.reset();
 		return TBTKX_OK;
+	case TBTKX_OPT_RESIDENT:
+		TBTKX_REQUIRE(value == 0 || value == 1, TBTKX_ERR_ARG,
+		              "tbtkx_set_option: resident recurrence option must be 0 or 1");
+		h->use_resident = (int)value;
+		return TBTKX_OK;
 	case TBTKX_OPT_MULTI:
 		TBTKX_REQUIRE(value >= 0 && value <= 2, TBTKX_ERR_ARG,
 		              "tbtkx_set_option: multi-vector mode must be 0, 1 or 2");
@@ -500,6 +508,7 @@ int tbtkx_get_option(tbtkx_handle h, int option, int64_t *value) {
 	case TBTKX_OPT_ELL: *value = h->use_ell && h->ell_W > 0; return TBTKX_OK;
 	case TBTKX_OPT_AUTOTUNE: *value = h->autotune; return TBTKX_OK;
 	case TBTKX_OPT_MFMA_PIPE: *value = h->mfma_pipe; return TBTKX_OK;
+	case TBTKX_OPT_RESIDENT: *value = h->last_resident; return TBTKX_OK;
 	case TBTKX_OPT_MULTI: *value = h->last_multi_blocks ? 2 : 1; return TBTKX_OK;
 	case TBTKX_OPT_ROW_PATTERNS: *value = h->last_patterns; return TBTKX_OK;
 	case TBTKX_OPT_SLOT_ROWS: *value = h->slot_rows; return TBTKX_OK;

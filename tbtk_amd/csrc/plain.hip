@@ -631,16 +631,26 @@ static int make_slot_arrays(tbtkx_context *h, bool codes, bool values) {
 	return TBTKX_OK;
 }
 
-int build_slots(tbtkx_context *h, const uint32_t *rowptr) {
+int build_slots(tbtkx_context *h, const uint32_t *rowptr, const uint32_t *col) {
 	h->slot_ok = 0;
 	h->slot_pal = 0;
 	h->slot_vals = 0;
 	h->slot_W = 0;
 	int64_t maxrow = 0;
-	for (int64_t r = 0; r < h->N; r++)
+	int half = 0;
+	for (int64_t r = 0; r < h->N; r++) {
+		int before = 0, after = 0;
+		bool diag = false;
+		for (uint32_t k = rowptr[r]; k < rowptr[r + 1]; k++) {
+			if ((int64_t)col[k] == r && !diag) diag = true;
+			else ++(diag ? after : before);
+		}
 		maxrow = std::max<int64_t>(maxrow, rowptr[r + 1] - rowptr[r]);
+		half = std::max(half, std::max(before, after));
+	}
 	if (h->N <= 0 || maxrow > 8) return TBTKX_OK;
 	h->slot_W = maxrow < 4 ? 4 : (int)maxrow;
+	h->slot_half = half;
 	h->slot_ok = 1;
 	const bool pal = h->palette_ok != 0;
 	int rc = make_slot_arrays(h, pal, !pal);
@@ -664,7 +674,7 @@ int build_plain_forms(tbtkx_context *h) {
 	}
 	int rc = build_palette(h, N, Z, hrp.data(), hcol.data(), hv1.data(), hv2.data());
 	if (rc) return rc;
-	if ((rc = build_slots(h, hrp.data()))) return rc;
+	if ((rc = build_slots(h, hrp.data(), hcol.data()))) return rc;
 	h->forms_pending = 0;
 	return TBTKX_OK;
 }
@@ -896,6 +906,70 @@ static int noalloc_scratch(tbtkx_context *h, unsigned char **ptr) {
 	return TBTKX_OK;
 }
 
+// The plain recurrence with a launch per step: enqueues the moments of the
+// unit vector `from` at the indices of `uniq` into h->coef.
+static int stream_moments(tbtkx_context *h, int64_t from, const std::vector<int64_t> &uniq, int M,
+                          const PlainForm &pform) {
+	const int U = (int)uniq.size();
+	int rc;
+	if ((rc = h->to.reserve((size_t)U * 8))) return rc;
+	if ((rc = h->coef.reserve((size_t)U * M * 16))) return rc;
+	TBTKX_CHECK_HIP(hipMemcpyAsync(h->to.ptr, uniq.data(), (size_t)U * 8,
+	                               hipMemcpyHostToDevice, h->stream));
+	const bool real = h->real_path && h->h_real;
+	const bool c16 = pform.c16, usepal = pform.pal;
+	if (real)
+		init_unit<double><<<grid_for(h->N), kThreads, 0, h->stream>>>(
+		    h->vec_a.as<double>(), h->N, from);
+	else
+		init_unit<double2><<<grid_for(h->N), kThreads, 0, h->stream>>>(
+		    h->vec_a.as<double2>(), h->N, from);
+	TBTKX_CHECK_HIP(hipGetLastError());
+	auto enqueue = [&]() {
+		double2 *coef = h->coef.as<double2>();
+		const int64_t *tod = h->to.as<int64_t>();
+		return real ? enqueue_steps<double>(h, U, M, h->vec_a.as<double>(),
+		                                    h->vec_b.as<double>(), coef, tod)
+		            : enqueue_steps<double2>(h, U, M, h->vec_a.as<double2>(),
+		                                     h->vec_b.as<double2>(), coef, tod);
+	};
+
+	TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
+	if (h->use_graph) {
+		GraphCache &gc = h->plain_graph;
+		int64_t key[GraphCache::kKey];
+		const bool key_ok = GraphCache::make_key(
+		    key, {U, M, h->plain_kernel * 4 + pform.slot * 2 + pform.pat + 16 * h->slot_rows +
+		                    256 * h->use_patterns,
+		          h->xcd_remap, h->N,
+		          real, c16, usepal},
+		    {h->vec_a.ptr, h->vec_b.ptr, h->coef.ptr, h->to.ptr, h->rowptr.ptr, h->col.ptr,
+		     h->v1.ptr, h->v2.ptr, h->v1r.ptr, h->v2r.ptr, h->rblk.ptr, h->col16.ptr,
+		     h->pcode.ptr, h->pal.ptr, h->palr.ptr, h->pdiag.ptr, h->pdiagr.ptr, h->scol.ptr,
+		     h->scode.ptr, h->sv1.ptr, h->sv2.ptr, h->sv1r.ptr, h->sv2r.ptr, h->ppid.ptr,
+		     h->pchunk.ptr,
+		     h->ptoff.ptr, h->ptcode.ptr});
+		TBTKX_REQUIRE(key_ok, TBTKX_ERR_STATE, "tbtkx_moments: graph key too long");
+		if (!gc.matches(key)) {
+			gc.reset();
+			TBTKX_CHECK_HIP(hipStreamBeginCapture(h->stream,
+			                                      hipStreamCaptureModeThreadLocal));
+			int erc = enqueue();
+			hipError_t ec = hipStreamEndCapture(h->stream, &gc.graph);
+			if (erc) return erc;
+			TBTKX_CHECK_HIP(ec);
+			TBTKX_CHECK_HIP(hipGraphInstantiate(&gc.exec, gc.graph, nullptr,
+			                                    nullptr, 0));
+			memcpy(gc.key, key, sizeof key);
+		}
+		TBTKX_CHECK_HIP(hipGraphLaunch(gc.exec, h->stream));
+	} else {
+		if ((rc = enqueue())) return rc;
+	}
+	TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
+	return TBTKX_OK;
+}
+
 }  // namespace tbtkx
 
 using namespace tbtkx;
@@ -969,6 +1043,7 @@ extern "C" int tbtkx_moments_noalloc(tbtkx_handle h, int64_t from, int K,
 	h->last_palette = usepal;
 	h->last_plain_kernel = pform.slot ? 2 : h->plain_kernel == 1 ? 1 : 0;
 	h->last_patterns = pform.pat;
+	h->last_resident = 0;
 	// A repeated to-index keeps only its last position (as tbtkx_moments).
 	for (int k = 0; k < K; k++)
 		for (int l = k + 1; l < K; l++)
@@ -1017,68 +1092,30 @@ extern "C" int tbtkx_moments(tbtkx_handle h, int64_t from, int K,
 	if (h->plain_kernel == 2 && !(h->use_palette && h->slot_pal) &&
 	    (rc = build_slot_values(h)))
 		return rc;
-	if ((rc = h->to.reserve((size_t)U * 8))) return rc;
-	if ((rc = h->coef.reserve((size_t)U * M * 16))) return rc;
-	TBTKX_CHECK_HIP(hipMemcpyAsync(h->to.ptr, uniq.data(), (size_t)U * 8,
-	                               hipMemcpyHostToDevice, h->stream));
 	// Real arithmetic when every value of H is real (the start vector is a
 	// unit vector).
 	const bool real = h->real_path && h->h_real;
 	const PlainForm pform = plain_form(h);
 	const bool c16 = pform.c16, usepal = pform.pal;
-	if (real)
-		init_unit<double><<<grid_for(h->N), kThreads, 0, h->stream>>>(
-		    h->vec_a.as<double>(), h->N, from);
-	else
-		init_unit<double2><<<grid_for(h->N), kThreads, 0, h->stream>>>(
-		    h->vec_a.as<double2>(), h->N, from);
-	TBTKX_CHECK_HIP(hipGetLastError());
-	auto enqueue = [&]() {
-		double2 *coef = h->coef.as<double2>();
-		const int64_t *tod = h->to.as<int64_t>();
-		return real ? enqueue_steps<double>(h, U, M, h->vec_a.as<double>(),
-		                                    h->vec_b.as<double>(), coef, tod)
-		            : enqueue_steps<double2>(h, U, M, h->vec_a.as<double2>(),
-		                                     h->vec_b.as<double2>(), coef, tod);
-	};
-
-	TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
-	if (h->use_graph) {
-		GraphCache &gc = h->plain_graph;
-		int64_t key[GraphCache::kKey];
-		const bool key_ok = GraphCache::make_key(
-		    key, {U, M, h->plain_kernel * 4 + pform.slot * 2 + pform.pat + 16 * h->slot_rows +
-		                    256 * h->use_patterns,
-		          h->xcd_remap, h->N,
-		          real, c16, usepal},
-		    {h->vec_a.ptr, h->vec_b.ptr, h->coef.ptr, h->to.ptr, h->rowptr.ptr, h->col.ptr,
-		     h->v1.ptr, h->v2.ptr, h->v1r.ptr, h->v2r.ptr, h->rblk.ptr, h->col16.ptr,
-		     h->pcode.ptr, h->pal.ptr, h->palr.ptr, h->pdiag.ptr, h->pdiagr.ptr, h->scol.ptr,
-		     h->scode.ptr, h->sv1.ptr, h->sv2.ptr, h->sv1r.ptr, h->sv2r.ptr, h->ppid.ptr,
-		     h->pchunk.ptr,
-		     h->ptoff.ptr, h->ptcode.ptr});
-		TBTKX_REQUIRE(key_ok, TBTKX_ERR_STATE, "tbtkx_moments: graph key too long");
-		if (!gc.matches(key)) {
-			gc.reset();
-			TBTKX_CHECK_HIP(hipStreamBeginCapture(h->stream,
-			                                      hipStreamCaptureModeThreadLocal));
-			int erc = enqueue();
-			hipError_t ec = hipStreamEndCapture(h->stream, &gc.graph);
-			if (erc) return erc;
-			TBTKX_CHECK_HIP(ec);
-			TBTKX_CHECK_HIP(hipGraphInstantiate(&gc.exec, gc.graph, nullptr,
-			                                    nullptr, 0));
-			memcpy(gc.key, key, sizeof key);
-		}
-		TBTKX_CHECK_HIP(hipGraphLaunch(gc.exec, h->stream));
-	} else {
-		if ((rc = enqueue())) return rc;
-	}
-	TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
-
 	std::vector<double> dense((size_t)U * M * 2);
-	TBTKX_CHECK_HIP(hipMemcpyAsync(dense.data(), h->coef.ptr, dense.size() * 8,
-	                               hipMemcpyDeviceToHost, h->stream));
+	const ResidentPlan plan = resident_plan(h, h->num_cus);
+	bool resident = plan.C > 0;
+	if (resident) {
+		const int toff[2] = {0, U};
+		TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
+		if ((rc = resident_moments(h, plan, 1, &from, toff, uniq.data(), M))) return rc;
+		TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
+		TBTKX_CHECK_HIP(hipMemcpyAsync(dense.data(), h->coef.ptr, dense.size() * 8,
+		                               hipMemcpyDeviceToHost, h->stream));
+		bool given_up = false;
+		if ((rc = resident_given_up(h, plan, &given_up))) return rc;
+		resident = !given_up;
+	}
+	if (!resident) {
+		if ((rc = stream_moments(h, from, uniq, M, pform))) return rc;
+		TBTKX_CHECK_HIP(hipMemcpyAsync(dense.data(), h->coef.ptr, dense.size() * 8,
+		                               hipMemcpyDeviceToHost, h->stream));
+	}
 	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
 	float ms = 0;
 	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
@@ -1089,6 +1126,7 @@ extern "C" int tbtkx_moments(tbtkx_handle h, int64_t from, int K,
 	h->last_palette = usepal;
 	h->last_plain_kernel = pform.slot ? 2 : h->plain_kernel == 1 ? 1 : 0;
 	h->last_patterns = pform.pat;
+	h->last_resident = resident;
 
 	for (int k = 0; k < K; k++) {
 		double *o = out + (size_t)k * M * 2;
