@@ -27,6 +27,7 @@
 // 32 staged in LDS.
 // Executed MFMA flops per launch: 2 * K * E * M * 12 (Retarded/Advanced)
 // or * 6 (Principal/NonPrincipal).
+#include <algorithm>
 #include <cstring>
 
 #include "common.hpp"
@@ -71,6 +72,12 @@ __global__ __launch_bounds__(kThreads) void split_planes(
 	planes[1 * plane + i] = rl;
 	planes[2 * plane + i] = ih;
 	planes[3 * plane + i] = il;
+}
+
+__global__ __launch_bounds__(kThreads) void widen(const float2 *__restrict__ in,
+                                                  double2 *__restrict__ out, int64_t n) {
+	const int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+	if (i < n) out[i] = make_double2((double)in[i].x, (double)in[i].y);
 }
 
 __device__ __forceinline__ bf16x8 neg(bf16x8 a) {
@@ -468,12 +475,21 @@ int tbtkx_contract_mfma(tbtkx_handle h, int type, double *out) {
 	h->last_ms = ms;
 	h->last_launches = 1;
 	if (out) {
-		std::vector<float2> g((size_t)K * E);
-		TBTKX_CHECK_HIP(hipMemcpy(g.data(), G, g.size() * 8, hipMemcpyDeviceToHost));
-		for (size_t i = 0; i < g.size(); i++) {
-			out[2 * i] = g[i].x;
-			out[2 * i + 1] = g[i].y;
+		// Widened to doubles on the device and copied straight into the
+		// caller's array, 256 MiB at a time (a host loop over the floats took
+		// several times the copy).
+		const int64_t n = (int64_t)K * E;
+		const int64_t part = std::min<int64_t>(n, ((int64_t)256 << 20) / 16);
+		if ((rc = h->gf_out.reserve((size_t)part * 16))) return rc;
+		for (int64_t i = 0; i < n; i += part) {
+			const int64_t m = std::min(part, n - i);
+			widen<<<(unsigned)((m + kThreads - 1) / kThreads), kThreads, 0, h->stream>>>(
+			    G + i, h->gf_out.as<double2>(), m);
+			TBTKX_CHECK_HIP(hipGetLastError());
+			TBTKX_CHECK_HIP(hipMemcpyAsync(out + 2 * i, h->gf_out.ptr, (size_t)m * 16,
+			                               hipMemcpyDeviceToHost, h->stream));
 		}
+		TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
 	}
 	return TBTKX_OK;
 }
