@@ -207,16 +207,7 @@ __global__ __launch_bounds__(kThreads) void block_init(
 		if (mode == 0) {
 			if (sites[b] == row) v.x = 1.0;
 		} else {
-			uint64_t c = (uint64_t)(col0 + b) * (uint64_t)N + (uint64_t)row;
-			uint64_t z = seed * 0x9E3779B97F4A7C15ull + c * 0xD1B54A32D192ED03ull +
-			             0x632BE59BD9B4E019ull;
-			z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-			z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-			z = z ^ (z >> 31);
-			const double u = (double)(z >> 11) * (1.0 / 9007199254740992.0);
-			double sn, cs;
-			sincos(2.0 * M_PI * u, &sn, &cs);
-			v = make_double2(cs, sn);
+			v = random_phase(seed, (uint64_t)(col0 + b) * (uint64_t)N + (uint64_t)row);
 		}
 	}
 	X[i] = C2<VT>::store(v);
@@ -1545,11 +1536,9 @@ double block_call_bytes(const tbtkx_context *h, int nvec, int B, int packed) {
 	return blocks * (20 * Z + 4 * N + 48.0 * B * N);
 }
 
-int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
-                uint64_t seed, int M, int flags, std::vector<double2> &mu) {
-	int rc = set_device(h);
-	if (rc) return rc;
-	if (flags & TBTKX_VEC_FP64) flags |= TBTKX_H_FP64;
+int wide_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
+               uint64_t seed, int M, int flags, std::vector<double2> &mu) {
+	int rc;
 	int B = h->block_width;
 	if (B == 32) B = 0;
 	// Unit start vectors on a real H: two real vectors per complex column.
@@ -1606,6 +1595,47 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 		                                     packed, mu);
 	return dispatch_width<float2, float2>(h, B, total, sites, mode, seed, M, flags,
 	                                      packed, mu);
+}
+
+// Columns in blocks of 64, 128 or 256 (wide_entry), except that up to
+// kNarrowRest columns, alone or left over by blocks of 128, run at their own
+// width (narrow_moments).
+constexpr int kNarrowRest = 96;
+
+int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
+                uint64_t seed, int M, int flags, std::vector<double2> &mu) {
+	int rc = set_device(h);
+	if (rc) return rc;
+	if (flags & TBTKX_VEC_FP64) flags |= TBTKX_H_FP64;
+	// Unit start vectors on a real H: two real vectors per complex column.
+	const int packed = mode == 0 && h->real_path && h->h_real;
+	const int per = packed ? 2 : 1, cols = (total + per - 1) / per;
+	const int rest = cols % 128;
+	const int parts = rest > 64 ? 2 : 1, w = (rest + parts - 1) / parts;
+	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w))
+		return wide_entry(h, total, sites, mode, seed, M, flags, mu);
+	const int wide = (cols - rest) * per;
+	mu.clear();
+	double ms = 0;
+	if (wide > 0) {
+		if ((rc = wide_entry(h, wide, sites, mode, seed, M, flags, mu))) return rc;
+		ms = h->last_ms;
+	}
+	mu.resize((size_t)total * M);
+	for (int v = wide; v < total; v += w * per) {
+		const int n = std::min(total - v, w * per);
+		if ((rc = narrow_moments(h, n, mode == 0 ? sites + v : nullptr, mode != 0, seed, v, M, flags,
+		                         packed, reinterpret_cast<double *>(mu.data() + (size_t)v * M))))
+			return rc;
+		ms += h->last_ms;
+	}
+	h->last_ms = ms;
+	const int S = (flags & TBTKX_DOUBLING) ? (M + 1) / 2 : M - 1;
+	h->last_launches = (int64_t)(wide / (128 * per) + parts) * S;
+	h->last_block_width = 64;
+	h->last_strip = -1;
+	h->last_rmul = 1;
+	return TBTKX_OK;
 }
 
 }  // namespace

@@ -209,6 +209,8 @@ struct tbtkx_context {
 	tbtkx::DevBuf mm_desc, mm_tab, mm_x, mm_y, mm_part, mm_seg, mm_D, mm_cols;
 	int64_t mm_tune_key[3] = {-1, -1, -1};    // (generation, flags, widths hash)
 	int mm_tune_g = 0, mm_tune_occ = 0;       // tuned tile groups, grid share
+	int64_t nb_tune_key[3] = {-1, -1, -1};    // the same of narrow blocks of the
+	int nb_tune_g = 0, nb_tune_occ = 0;       // single model (narrow_moments)
 	std::vector<tbtkx::GraphCache> mm_graphs;   // the run in bounded chunks
 	void reset_mm_graphs() {
 		for (tbtkx::GraphCache &g : mm_graphs) g.reset();
@@ -326,6 +328,26 @@ int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const in
 // Whether the last launch gave up a wait (its moments are then incomplete);
 // waits for the stream.
 int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up);
+
+// Up to 64 columns of the single model through the uneven batch's step kernel
+// (multi.hip), which stores and moves just these columns where a block is at
+// least 64 wide. out: total x M moments. narrow_fits: the launch shape is
+// free, the vectors FP32 and the model in ELL form.
+bool narrow_fits(const tbtkx_context *h, int flags, int cols);
+int narrow_moments(tbtkx_context *h, int total, const int64_t *sites, bool phases, uint64_t seed,
+                   int64_t col0, int M, int flags, int packed, double *out);
+
+// Random phase exp(2 pi i u), u the 53-bit splitmix64 uniform of (seed, c).
+__device__ __forceinline__ double2 random_phase(uint64_t seed, uint64_t c) {
+	uint64_t z = seed * 0x9E3779B97F4A7C15ull + c * 0xD1B54A32D192ED03ull + 0x632BE59BD9B4E019ull;
+	z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+	z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+	z = z ^ (z >> 31);
+	const double u = (double)(z >> 11) * (1.0 / 9007199254740992.0);
+	double sn, cs;
+	sincos(2.0 * M_PI * u, &sn, &cs);
+	return make_double2(cs, sn);
+}
 
 // Builds the plain kernel's value palette from host copies of the CSR
 // (v1 = H/s, v2 = 2H/s, interleaved complex); sets palette_ok when the

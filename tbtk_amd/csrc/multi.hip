@@ -66,6 +66,8 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kRpi = 2;          // row groups in flight per lane
 constexpr int kSegSlots = 64;    // dot slots summed per group in pass 1
 constexpr int kMaxWidth = 64;    // start vectors per model
+constexpr int kRing = 16;        // steps between two reductions of the dot slots,
+constexpr int64_t kRingBytes = (int64_t)256 << 20;   // as many as fit this
 constexpr int64_t kMaxSlotBytes = (int64_t)1 << 30;   // dot slots of a one-tile-per-wavefront plan
 
 struct MDesc {
@@ -161,17 +163,36 @@ __global__ __launch_bounds__(kThreads) void multi_units(float2 *__restrict__ X,
 	e[c.comp == 2 ? 1 : 0] = 1.0f;
 }
 
-// Gather mode: mu_n of every column whose model has more than n moments.
-__global__ __launch_bounds__(kThreads) void multi_gather(
-    const GCol *__restrict__ cols, int ncols, const float2 *__restrict__ X,
-    double2 *__restrict__ mu, int n) {
-	const int g = blockIdx.x * kThreads + threadIdx.x;
-	if (g >= ncols) return;
+// Gather mode: mu_n of column g, when its model has more than n moments.
+__device__ __forceinline__ void gather_col(const GCol *__restrict__ cols, int g,
+                                           const float2 *__restrict__ X,
+                                           double2 *__restrict__ mu, int n) {
 	const GCol c = cols[g];
 	if (n < c.M) {
 		const float2 x = X[c.xoff];
 		if (c.comp == 0) mu[c.out + n] = make_double2((double)x.x, (double)x.y);
 		else mu[c.out + n] = make_double2((double)(c.comp == 2 ? x.y : x.x), 0.0);
+	}
+}
+
+__global__ __launch_bounds__(kThreads) void multi_gather(
+    const GCol *__restrict__ cols, int ncols, const float2 *__restrict__ X,
+    double2 *__restrict__ mu, int n) {
+	const int g = blockIdx.x * kThreads + threadIdx.x;
+	if (g < ncols) gather_col(cols, g, X, mu, n);
+}
+
+// Random-phase start vectors of a single model (stored columns past w are 0).
+__global__ __launch_bounds__(kThreads) void multi_phases(float2 *__restrict__ X, int64_t N, int w,
+                                                         int wp, uint64_t seed, int64_t col0) {
+	const int64_t n = N * wp;
+	for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
+	     i += (int64_t)gridDim.x * kThreads) {
+		const int64_t row = i / wp;
+		const int b = (int)(i - row * wp);
+		double2 v = make_double2(0.0, 0.0);
+		if (b < w) v = random_phase(seed, (uint64_t)(col0 + b) * (uint64_t)N + (uint64_t)row);
+		X[i] = make_float2((float)v.x, (float)v.y);
 	}
 }
 
@@ -457,7 +478,7 @@ __device__ __forceinline__ void model_rows_w(
 }
 
 // Dispatch on the model's ELL width (4, 5, 6 or 8, at most the batch's
-// widest, WMAX, which fixes the kernel's registers).
+// widest, WMAX, which fixes the kernel's registers; 7: a single model).
 template <int WMAX, bool FIRST, bool DOTS, bool REALH>
 __device__ __forceinline__ void model_rows(
     const MDesc &d, int &t, int tend, int nwx, int toff_m, int G, int Q, int qc, bool act,
@@ -476,7 +497,7 @@ __device__ __forceinline__ void model_rows(
 #define TBTKX_MR(WW)                                                                 \
 	model_rows_w<WW, FIRST, DOTS, REALH>(d, t, tend, nwx, toff_m, G, Q, qc, act, b, tr, lane, \
 	                                     ecol, ev, X, Y, packed, dd)
-	if (d.W == WMAX) {
+	if (WMAX == 7 || d.W == WMAX) {
 		TBTKX_MR(WMAX);
 	} else if constexpr (WMAX > 4) {
 		if (d.W == 4) {
@@ -516,7 +537,13 @@ __attribute__((amdgpu_waves_per_eu(WMAX <= 5 ? 4 : 1))) void multi_step(
     const int *__restrict__ xpart, const int *__restrict__ pbase,
     const int *__restrict__ pstart, int G, const uint32_t *__restrict__ ecol,
     const float2 *__restrict__ ev, const float2 *__restrict__ X,
-    float2 *__restrict__ Y, double2 *__restrict__ part, int packed) {
+    float2 *__restrict__ Y, double2 *__restrict__ part, int packed,
+    const GCol *__restrict__ cols, int ncols, double2 *__restrict__ mu, int nprev) {
+	// The moments of X (step nprev) ride on the launch that reads it; X is not
+	// written here.
+	if (!DOTS)
+		for (int g = blockIdx.x * kThreads + threadIdx.x; g < ncols; g += gridDim.x * kThreads)
+			gather_col(cols, g, X, mu, nprev);
 	const int lane = threadIdx.x & 63;
 	const int x = blockIdx.x & 7;
 	const int nwx = (gridDim.x >> 3) * kWaves;                  // wavefronts per XCD
@@ -574,10 +601,15 @@ __attribute__((amdgpu_waves_per_eu(WMAX <= 5 ? 4 : 1))) void multi_step(
 }
 
 // Pass 1: segment s = (model, slot_lo, slot_hi) of <= 64 slots; one
-// wavefront per (segment, which), lane = column (the model's w columns).
+// wavefront per (segment, which), lane = column (the model's w columns);
+// blockIdx.y: the step, of those whose slots the ring holds (max_slots each).
+// The two passes run once per ring, not per step: they are launch and latency
+// bound (8.1 and 5.1 us per step of 16 models of up to 100,000 states).
 __global__ __launch_bounds__(kThreads) void multi_reduce_slots(
     const MDesc *__restrict__ md, const int *__restrict__ seg, int nseg,
-    const double2 *__restrict__ part, double2 *__restrict__ segsum) {
+    const double2 *__restrict__ part, double2 *__restrict__ segsum, int max_slots, int max_seg) {
+	part += (int64_t)blockIdx.y * max_slots * 2 * kMaxWidth;
+	segsum += (int64_t)blockIdx.y * max_seg * 2 * kMaxWidth;
 	const int lane = threadIdx.x & 63;
 	const int gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
 	if (gw >= 2 * nseg) return;
@@ -606,7 +638,9 @@ __global__ __launch_bounds__(kThreads) void multi_reduce_slots(
 // order, into D[dof + (n * 2 + which) * w + b].
 __global__ __launch_bounds__(kThreads) void multi_reduce_models(
     const MDesc *__restrict__ md, const int *__restrict__ mseg, int kact,
-    const double2 *__restrict__ segsum, double2 *__restrict__ D, int n) {
+    const double2 *__restrict__ segsum, double2 *__restrict__ D, int n, int max_seg) {
+	segsum += (int64_t)blockIdx.y * max_seg * 2 * kMaxWidth;
+	n += blockIdx.y;
 	const int lane = threadIdx.x & 63;
 	const int gw = blockIdx.x * kWaves + (threadIdx.x >> 6);
 	if (gw >= 2 * kact) return;
@@ -650,6 +684,7 @@ struct Plan {
 	std::vector<Phase> phases;
 	std::vector<int> tab;        // all phase tables
 	int nwg = 0, G = 8, Smax = 0, max_slots = 0, max_seg = 0;
+	int ring = 1;                // steps whose dot slots are kept between reductions
 	int64_t vec_elems = 0, d_elems = 0;
 };
 
@@ -756,6 +791,7 @@ int grid_size(tbtkx_context *h, bool dots, int share, int *nwg) {
 	if (h->mm_W == 4) TBTKX_FN(4);
 	else if (h->mm_W == 5) TBTKX_FN(5);
 	else if (h->mm_W == 6) TBTKX_FN(6);
+	else if (h->mm_W == 7) TBTKX_FN(7);
 	else TBTKX_FN(8);
 #undef TBTKX_FN
 	int per_cu = 0, cus = 0;
@@ -842,20 +878,23 @@ int make_plan(tbtkx_context *h, const std::vector<int> &width, const std::vector
 		p.phases.push_back(ph);
 		n = n_hi;
 	}
+	p.ring = (int)std::min<int64_t>(
+	    kRing, std::max<int64_t>(1, kRingBytes / ((int64_t)std::max(1, p.max_slots) * 2 * kMaxWidth * 16)));
 	return TBTKX_OK;
 }
 
 template <int W, bool REALH>
 void launch_step_w(tbtkx_context *h, const Plan &p, const Phase &ph, bool first,
-                   bool dots, const float2 *X, float2 *Y) {
+                   bool dots, const float2 *X, float2 *Y, int ring, int ncols, int n) {
 	const int *tab = h->mm_tab.as<int>();
 	const MDesc *md = h->mm_desc.as<MDesc>();
 	const float2 *ev = first ? h->mm_ev1.as<float2>() : h->mm_ev2.as<float2>();
-	double2 *part = h->mm_part.as<double2>();
+	double2 *part = h->mm_part.as<double2>() + (int64_t)ring * p.max_slots * 2 * kMaxWidth;
 #define TBTKX_MS(F, D)                                                          \
 	multi_step<W, F, D, REALH><<<ph.nwg, kThreads, 0, h->stream>>>(           \
 	    md, tab + ph.toff, ph.kact, tab + ph.xpart, tab + ph.pbase,            \
-	    tab + ph.pstart, p.G, h->mm_ecol.as<uint32_t>(), ev, X, Y, part, h->mm_packed)
+	    tab + ph.pstart, p.G, h->mm_ecol.as<uint32_t>(), ev, X, Y, part, h->mm_packed, \
+	    h->mm_cols.as<GCol>(), ncols, h->mm_D.as<double2>(), n)
 	if (first && dots) TBTKX_MS(true, true);
 	else if (first) TBTKX_MS(true, false);
 	else if (dots) TBTKX_MS(false, true);
@@ -863,17 +902,20 @@ void launch_step_w(tbtkx_context *h, const Plan &p, const Phase &ph, bool first,
 #undef TBTKX_MS
 }
 
+// One step; ring: where its dot slots go; without dots, ncols columns' moments n
+// of X.
 void launch_step(tbtkx_context *h, const Plan &p, const Phase &ph, bool first,
-                 bool dots, const float2 *X, float2 *Y) {
+                 bool dots, const float2 *X, float2 *Y, int ring, int ncols, int n) {
 	const bool R = h->mm_real;
 #define TBTKX_LS(WW)                                                  \
 	do {                                                          \
-		if (R) launch_step_w<WW, true>(h, p, ph, first, dots, X, Y);  \
-		else launch_step_w<WW, false>(h, p, ph, first, dots, X, Y);   \
+		if (R) launch_step_w<WW, true>(h, p, ph, first, dots, X, Y, ring, ncols, n);  \
+		else launch_step_w<WW, false>(h, p, ph, first, dots, X, Y, ring, ncols, n);   \
 	} while (0)
 	if (h->mm_W == 4) TBTKX_LS(4);
 	else if (h->mm_W == 5) TBTKX_LS(5);
 	else if (h->mm_W == 6) TBTKX_LS(6);
+	else if (h->mm_W == 7) TBTKX_LS(7);
 	else TBTKX_LS(8);
 #undef TBTKX_LS
 }
@@ -884,10 +926,10 @@ int reserve_plan(tbtkx_context *h, const Plan &p, int ncols, int64_t mu_elems) {
 	if ((rc = h->mm_tab.reserve(p.tab.size() * 4))) return rc;
 	if ((rc = h->mm_x.reserve((size_t)p.vec_elems * 8))) return rc;
 	if ((rc = h->mm_y.reserve((size_t)p.vec_elems * 8))) return rc;
-	if ((rc = h->mm_part.reserve((size_t)(p.max_slots > 0 ? p.max_slots : 1) * 2 *
+	if ((rc = h->mm_part.reserve((size_t)(p.max_slots > 0 ? p.max_slots : 1) * p.ring * 2 *
 	                             kMaxWidth * 16)))
 		return rc;
-	if ((rc = h->mm_seg.reserve((size_t)(p.max_seg > 0 ? p.max_seg : 1) * 2 *
+	if ((rc = h->mm_seg.reserve((size_t)(p.max_seg > 0 ? p.max_seg : 1) * p.ring * 2 *
 	                            kMaxWidth * 16)))
 		return rc;
 	if ((rc = h->mm_D.reserve((size_t)(mu_elems > 0 ? mu_elems : 1) * 16))) return rc;
@@ -902,44 +944,54 @@ int reserve_plan(tbtkx_context *h, const Plan &p, int ncols, int64_t mu_elems) {
 }
 
 // The two ordered reduction passes of the doubling dots of step n.
-void launch_reduce(tbtkx_context *h, const Phase &ph, double2 *D, int n) {
+// The dots of steps n .. n + count - 1, from the ring's first `count` places.
+void launch_reduce(tbtkx_context *h, const Plan &p, const Phase &ph, double2 *D, int n, int count) {
 	const int *tab = h->mm_tab.as<int>();
-	multi_reduce_slots<<<(2 * ph.nseg + kWaves - 1) / kWaves, kThreads, 0, h->stream>>>(
+	multi_reduce_slots<<<dim3((2 * ph.nseg + kWaves - 1) / kWaves, count), kThreads, 0, h->stream>>>(
 	    h->mm_desc.as<MDesc>(), tab + ph.seg, ph.nseg, h->mm_part.as<double2>(),
-	    h->mm_seg.as<double2>());
-	multi_reduce_models<<<(2 * ph.kact + kWaves - 1) / kWaves, kThreads, 0, h->stream>>>(
-	    h->mm_desc.as<MDesc>(), tab + ph.mseg, ph.kact, h->mm_seg.as<double2>(), D, n);
+	    h->mm_seg.as<double2>(), p.max_slots, p.max_seg);
+	multi_reduce_models<<<dim3((2 * ph.kact + kWaves - 1) / kWaves, count), kThreads, 0, h->stream>>>(
+	    h->mm_desc.as<MDesc>(), tab + ph.mseg, ph.kact, h->mm_seg.as<double2>(), D, n, p.max_seg);
 }
+
+// Start vectors of a run: unit vectors (the columns' sites), or random phases of
+// a single model, columns col0, col0 + 1, ... of the sequence of `seed`.
+struct Start {
+	bool phases = false;
+	uint64_t seed = 0;
+	int64_t col0 = 0;
+};
 
 // Everything from the initial vectors to the last step, on h->stream.
 // Enqueue steps s_lo .. s_hi - 1 of the run (all phases' steps counted in
 // order; the vectors' roles alternate with the step's parity), with the
 // start vectors before step 0 and, without the doubling dots, the final
 // gather after the last step.
-int enqueue_run(tbtkx_context *h, const Plan &p, bool dots, int ncols, int64_t s_lo,
-                int64_t s_hi) {
+int enqueue_run(tbtkx_context *h, const Plan &p, bool dots, int ncols, const Start &start,
+                int64_t s_lo, int64_t s_hi) {
 	const GCol *cols = h->mm_cols.as<GCol>();
 	double2 *D = h->mm_D.as<double2>();
-	const int *tab = h->mm_tab.as<int>();
 	float2 *X = h->mm_x.as<float2>(), *Y = h->mm_y.as<float2>();
 	if (s_lo & 1) std::swap(X, Y);
-	if (s_lo == 0) {
+	if (s_lo == 0 && start.phases) {
+		const MDesc &d = p.desc[0];
+		multi_phases<<<4096, kThreads, 0, h->stream>>>(X, d.N, d.w, d.wp, start.seed, start.col0);
+	} else if (s_lo == 0) {
 		multi_fill<<<2048, kThreads, 0, h->stream>>>(X, p.vec_elems);
 		multi_units<<<grid_for(ncols), kThreads, 0, h->stream>>>(X, cols, ncols);
 	}
 	int64_t launches = 0, step = 0;
 	for (const Phase &ph : p.phases) {
+		int held = 0;   // steps whose dots wait in the ring
 		for (int n = ph.n_lo; n < ph.n_hi; n++, step++) {
 			if (step < s_lo || step >= s_hi) continue;
-			if (!dots)
-				multi_gather<<<grid_for(ncols), kThreads, 0, h->stream>>>(
-				    cols, ncols, X, D, n);
-			launch_step(h, p, ph, n == 0, dots, X, Y);
+			launch_step(h, p, ph, n == 0, dots, X, Y, held, ncols, n);
 			launches++;
-			if (dots) launch_reduce(h, ph, D, n);
-			float2 *tmp = X;
-			X = Y;
-			Y = tmp;
+			if (dots && (++held == p.ring || n + 1 == ph.n_hi || step + 1 == s_hi)) {
+				launch_reduce(h, p, ph, D, n + 1 - held, held);
+				held = 0;
+			}
+			std::swap(X, Y);
 		}
 	}
 	if (!dots && s_hi >= step)
@@ -987,14 +1039,17 @@ int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<
 			const Phase &ph = p.phases[0];
 			float2 *X = h->mm_x.as<float2>(), *Y = h->mm_y.as<float2>();
 			multi_fill<<<2048, kThreads, 0, h->stream>>>(X, p.vec_elems);
-			launch_step(h, p, ph, true, dots, X, Y);
+			launch_step(h, p, ph, true, dots, X, Y, 0, 0, 0);
 			TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
+			int held = 0;
 			for (int i = 0; i < kTrial; i++) {
-				launch_step(h, p, ph, false, dots, Y, X);
-				if (dots) launch_reduce(h, ph, h->mm_D.as<double2>(), 0);
-				float2 *tmp = X;
-				X = Y;
-				Y = tmp;
+				launch_step(h, p, ph, false, dots, Y, X, held, 0, 0);
+				// (the run has at least one step: moments 0 are overwritten by it)
+				if (dots && (++held == p.ring || i + 1 == kTrial)) {
+					launch_reduce(h, p, ph, h->mm_D.as<double2>(), 0, std::min(held, ph.n_hi));
+					held = 0;
+				}
+				std::swap(X, Y);
 			}
 			TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
 			TBTKX_CHECK_HIP(hipEventSynchronize(h->ev_stop));
@@ -1013,7 +1068,243 @@ int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<
 	return TBTKX_OK;
 }
 
+// Moments of the batch (the mm_* model fields): num_sites[m] start vectors and
+// num_moments[m] moments of model m, doubling dots or gathers, packed real
+// vectors or complex columns.
+int run_batch(tbtkx_context *h, const int *num_sites, const int64_t *sites, const int *num_moments,
+              bool dots, int packed, const Start &start, double *out) {
+	const int K = h->mm_K;
+	h->mm_packed = packed;
+	std::vector<int> width(K), S(K);
+	std::vector<int64_t> out_off(K + 1, 0);
+	int ncols = 0;
+	for (int m = 0; m < K; m++) {
+		width[m] = packed ? (num_sites[m] + 1) / 2 : num_sites[m];
+		S[m] = dots ? (num_moments[m] + 1) / 2 : num_moments[m] - 1;
+		out_off[m + 1] = out_off[m] + (int64_t)num_sites[m] * num_moments[m];
+		if (!start.phases) ncols += num_sites[m];
+	}
+	int rc = set_device(h);
+	if (rc) return rc;
+	const int Smax = *std::max_element(S.begin(), S.end());
+
+	// Launch shape: explicit (TBTKX_OPT_TILE_ROWS = row groups per tile, with
+	// TBTKX_OPT_GRID_SHARE: 0 = one tile per wavefront, s > 0 = persistent
+	// grid of occupancy x CUs / s workgroups) or autotuned once per (batch,
+	// mode, widths).
+	int64_t hw = 1469598103934665603ll;
+	for (int m = 0; m < K; m++) hw = (hw ^ (width[m] * 131 + S[m])) * 1099511628211ll;
+	const int64_t key[3] = {h->mm_gen, (int)dots + (packed << 16), hw};
+	int G = 8, share = 1;
+	if (h->tile_rows > 0) {
+		G = std::max(kRpi, (h->tile_rows + kRpi - 1) / kRpi * kRpi);
+		share = h->grid_share;
+	} else if (h->autotune && Smax > 0) {
+		if (memcmp(key, h->mm_tune_key, sizeof key) != 0) {
+			// Output sizes are needed to reserve buffers for the trial runs.
+			int64_t mu_elems = 0;
+			for (int m = 0; m < K; m++)
+				mu_elems += dots ? (int64_t)S[m] * 2 * width[m] : out_off[m + 1] - out_off[m];
+			if ((rc = autotune(h, width, S, dots, ncols, mu_elems))) return rc;
+			memcpy(h->mm_tune_key, key, sizeof key);
+		}
+		G = h->mm_tune_g;
+		share = h->mm_tune_occ;
+	}
+	h->last_share = share;
+	h->last_tile_groups = G;
+	Plan p;
+	if (Smax > 0) {
+		if ((rc = make_plan(h, width, S, dots, G, share, p))) return rc;
+	} else {
+		// One moment per model: only the initial gather.
+		p.order.resize(K);
+		std::iota(p.order.begin(), p.order.end(), 0);
+		p.desc.resize(K);
+		int64_t vec = 0;
+		for (int m = 0; m < K; m++) {
+			MDesc &d = p.desc[m];
+			d = MDesc{};
+			d.N = h->mm_N[m];
+			d.e0 = h->mm_e0[m];
+			d.W = h->mm_Wm[m];
+		d.realh = h->mm_realm[m];
+			d.vec0 = vec;
+			d.w = width[m];
+			d.wp = width[m];
+			d.Q = kMaxWidth / width[m];
+			vec += h->mm_N[m] * width[m];
+		}
+		p.vec_elems = vec;
+	}
+	// Columns: X offset of each unit start vector and its output row.
+	std::vector<int> pos(K);
+	for (int k = 0; k < K; k++) pos[p.order[k]] = k;
+	std::vector<GCol> cols(std::max(ncols, 1));
+	for (int m = 0, c = 0; m < K; m++) {
+		const MDesc &d = p.desc[pos[m]];
+		for (int b = 0; b < num_sites[m] && !start.phases; b++, c++) {
+			cols[c].xoff = d.vec0 + sites[c] * d.wp + (packed ? b >> 1 : b);
+			cols[c].out = out_off[m] + (int64_t)b * num_moments[m];
+			cols[c].M = num_moments[m];
+			cols[c].comp = packed ? 1 + (b & 1) : 0;
+		}
+	}
+	const int64_t mu_elems = dots ? p.d_elems : out_off[K];
+	if ((rc = reserve_plan(h, p, (int)cols.size(), mu_elems))) return rc;
+	TBTKX_CHECK_HIP(hipMemcpyAsync(h->mm_cols.ptr, cols.data(), cols.size() * sizeof(GCol),
+	                               hipMemcpyHostToDevice, h->stream));
+
+	TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
+	const int64_t nsteps = run_steps(p);
+	if (h->use_graph) {
+		// The run is captured as graphs of at most kGraphSteps steps each (a
+		// few hundred kernel nodes per graph rather than one graph of three
+		// launches per step), all cached under one key and replayed in order.
+		const int64_t nchunk = nsteps > 0 ? (nsteps + kGraphSteps - 1) / kGraphSteps : 1;
+		int64_t mh = hw;
+		for (int m = 0; m < K; m++) mh = (mh ^ num_moments[m]) * 1099511628211ll;
+		int64_t gkey[GraphCache::kKey];
+		const bool key_ok = GraphCache::make_key(
+		    gkey, {h->mm_gen, (int)dots, mh, G * 16 + share, p.nwg, packed, nchunk},
+		    {h->mm_desc.ptr, h->mm_tab.ptr, h->mm_x.ptr, h->mm_y.ptr, h->mm_part.ptr,
+		     h->mm_seg.ptr, h->mm_D.ptr, h->mm_cols.ptr, h->mm_ecol.ptr, h->mm_ev1.ptr,
+		     h->mm_ev2.ptr});
+		TBTKX_REQUIRE(key_ok, TBTKX_ERR_STATE, "tbtkx_multi_moments: graph key too long");
+		bool cached = (int64_t)h->mm_graphs.size() == nchunk;
+		for (int64_t c = 0; cached && c < nchunk; c++)
+			cached = h->mm_graphs[c].matches(gkey);
+		if (!cached) {
+			for (GraphCache &g : h->mm_graphs) g.reset();
+			h->mm_graphs.clear();
+			h->mm_graphs.resize(nchunk);
+			for (int64_t c = 0; c < nchunk; c++) {
+				GraphCache &gc = h->mm_graphs[c];
+				TBTKX_CHECK_HIP(hipStreamBeginCapture(h->stream,
+				                                      hipStreamCaptureModeThreadLocal));
+				int erc = enqueue_run(h, p, dots, ncols, start, c * kGraphSteps,
+				                      std::min(nsteps, (c + 1) * kGraphSteps));
+				hipError_t ec = hipStreamEndCapture(h->stream, &gc.graph);
+				if (erc) return erc;
+				TBTKX_CHECK_HIP(ec);
+				TBTKX_CHECK_HIP(hipGraphInstantiate(&gc.exec, gc.graph, nullptr, nullptr, 0));
+				memcpy(gc.key, gkey, sizeof gkey);
+			}
+		}
+		for (GraphCache &gc : h->mm_graphs) TBTKX_CHECK_HIP(hipGraphLaunch(gc.exec, h->stream));
+		h->last_launches = Smax;
+	} else {
+		if ((rc = enqueue_run(h, p, dots, ncols, start, 0, nsteps))) return rc;
+	}
+	TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
+	std::vector<double2> buf(mu_elems > 0 ? mu_elems : 1);
+	TBTKX_CHECK_HIP(hipMemcpyAsync(buf.data(), h->mm_D.ptr, (size_t)mu_elems * 16,
+	                               hipMemcpyDeviceToHost, h->stream));
+	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
+	float ms = 0;
+	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
+	h->last_ms = ms;
+	h->last_real = packed;
+
+	double2 *o2 = reinterpret_cast<double2 *>(out);
+	if (!dots) {
+		memcpy(o2, buf.data(), (size_t)out_off[K] * 16);
+		return TBTKX_OK;
+	}
+	for (int m = 0; m < K; m++) {
+		const MDesc &d = p.desc[pos[m]];
+		const int M = num_moments[m], w = width[m];
+		for (int b = 0; b < num_sites[m]; b++) {
+			double2 *o = o2 + out_off[m] + (int64_t)b * M;
+			// Column of vector b; packed: its component.
+			const int c = packed ? b >> 1 : b;
+			auto Dv = [&](int n, int which) {
+				const double2 v = buf[d.dof + ((int64_t)n * 2 + which) * w + c];
+				if (!packed) return v;
+				return make_double2((b & 1) ? v.y : v.x, 0.0);
+			};
+			const double2 mu0 = Dv(0, 0), mu1 = Dv(0, 1);
+			o[0] = mu0;
+			if (M > 1) o[1] = mu1;
+			for (int n = 1; n < S[m]; n++) {
+				const double2 a = Dv(n, 0), c = Dv(n, 1);
+				if (2 * n < M) o[2 * n] = make_double2(2 * a.x - mu0.x, 2 * a.y - mu0.y);
+				if (2 * n + 1 < M)
+					o[2 * n + 1] = make_double2(2 * c.x - mu1.x, 2 * c.y - mu1.y);
+			}
+		}
+	}
+	return TBTKX_OK;
+}
+
+// The handle's single model takes the batch's place while this lives. Its
+// block ELL has the batch's layout (rows of W slots, diagonal first, 8 bytes a
+// value).
+struct SingleModel {
+	tbtkx_context *h;
+	int K, W, realH = 0;
+	bool real;
+	std::vector<int64_t> N, e0, band;
+	std::vector<int> Wm, realm;
+	int64_t gen;
+	explicit SingleModel(tbtkx_context *ctx) : h(ctx) {
+		const int r = h->h_real ? 1 : 0;
+		K = 1;
+		W = h->ell_W;
+		real = h->h_real;
+		N = {h->N};
+		e0 = {0};
+		band = {h->band};
+		Wm = {W};
+		realm = {r};
+		gen = h->csr_gen;
+		exchange();
+	}
+	~SingleModel() { exchange(); }
+	SingleModel(const SingleModel &) = delete;
+	void exchange() {
+		std::swap(K, h->mm_K);
+		std::swap(W, h->mm_W);
+		std::swap(real, h->mm_real);
+		std::swap(N, h->mm_N);
+		std::swap(e0, h->mm_e0);
+		std::swap(band, h->mm_band);
+		std::swap(Wm, h->mm_Wm);
+		std::swap(realm, h->mm_realm);
+		std::swap(gen, h->mm_gen);
+		std::swap(h->mm_ecol, h->ell_col);
+		std::swap(h->mm_ev1, h->ell_v1f);
+		std::swap(h->mm_ev2, h->ell_v2f);
+		std::swap(h->mm_tune_key, h->nb_tune_key);
+		std::swap(h->mm_tune_g, h->nb_tune_g);
+		std::swap(h->mm_tune_occ, h->nb_tune_occ);
+	}
+};
+
 }  // namespace
+
+bool narrow_fits(const tbtkx_context *h, int flags, int cols) {
+	return (flags & ~TBTKX_DOUBLING) == 0 && h->ell_W > 0 && h->use_ell && h->autotune &&
+	       !h->use_graph && h->block_width == 0 && h->strip_rows == 0 && h->grid_share == 0 &&
+	       h->rows_in_flight == 0 && h->tile_rows == 0 && h->strip_chunk == 0 && h->nt_stream &&
+	       !h->xcd_remap && cols >= 1 && cols <= kMaxWidth &&
+	       h->N * (cols + 1) * 8 < ((int64_t)1 << 32);
+}
+
+int narrow_moments(tbtkx_context *h, int total, const int64_t *sites, bool phases, uint64_t seed,
+                   int64_t col0, int M, int flags, int packed, double *out) {
+	int rc;
+	{
+		SingleModel view(h);
+		Start start;
+		start.phases = phases;
+		start.seed = seed;
+		start.col0 = col0;
+		rc = run_batch(h, &total, sites, &M, (flags & TBTKX_DOUBLING) != 0, packed, start, out);
+	}
+	return rc;
+}
+
 }  // namespace tbtkx
 
 using namespace tbtkx;
@@ -1160,183 +1451,26 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 	TBTKX_REQUIRE((flags & ~TBTKX_DOUBLING) == 0, TBTKX_ERR_ARG,
 	              "tbtkx_multi_moments: only TBTKX_DOUBLING is supported (FP32 storage)");
 	const int K = h->mm_K;
-	const bool dots = (flags & TBTKX_DOUBLING) != 0;
 	// Real H in every model (the start vectors are unit vectors): two real
 	// vectors per complex column.
 	const int packed = h->real_path && h->mm_real;
-	h->mm_packed = packed;
-	std::vector<int> width(K), S(K);
-	std::vector<int64_t> out_off(K + 1, 0);
-	int ncols = 0;
-	for (int m = 0; m < K; m++) {
+	for (int m = 0, c = 0; m < K; c += num_sites[m], m++) {
 		const std::string tag = "tbtkx_multi_moments: model " + std::to_string(m) + ": ";
 		TBTKX_REQUIRE(num_sites[m] >= 1 && num_sites[m] <= kMaxWidth, TBTKX_ERR_ARG,
 		              tag + "needs 1..64 sites");
 		TBTKX_REQUIRE(num_moments[m] >= 1, TBTKX_ERR_ARG,
 		              tag + "numCoefficients has to be larger than 0");
 		for (int b = 0; b < num_sites[m]; b++)
-			TBTKX_REQUIRE(sites[ncols + b] >= 0 && sites[ncols + b] < h->mm_N[m],
+			TBTKX_REQUIRE(sites[c + b] >= 0 && sites[c + b] < h->mm_N[m],
 			              TBTKX_ERR_ARG, tag + "site outside the basis");
-		width[m] = packed ? (num_sites[m] + 1) / 2 : num_sites[m];
 		// The step addresses a model's vectors with 32-bit byte offsets
 		// (stored columns: at most one past the model's).
-		TBTKX_REQUIRE(h->mm_N[m] * (width[m] + 1) * 8 < ((int64_t)1 << 32), TBTKX_ERR_ARG,
+		const int width = packed ? (num_sites[m] + 1) / 2 : num_sites[m];
+		TBTKX_REQUIRE(h->mm_N[m] * (width + 1) * 8 < ((int64_t)1 << 32), TBTKX_ERR_ARG,
 		              tag + "rows x (columns + 1) x 8 B must stay below 4 GiB");
-		S[m] = dots ? (num_moments[m] + 1) / 2 : num_moments[m] - 1;
-		out_off[m + 1] = out_off[m] + (int64_t)num_sites[m] * num_moments[m];
-		ncols += num_sites[m];
 	}
-	int rc = set_device(h);
-	if (rc) return rc;
-	const int Smax = *std::max_element(S.begin(), S.end());
-
-	// Launch shape: explicit (TBTKX_OPT_TILE_ROWS = row groups per tile, with
-	// TBTKX_OPT_GRID_SHARE: 0 = one tile per wavefront, s > 0 = persistent
-	// grid of occupancy x CUs / s workgroups) or autotuned once per (batch,
-	// mode, widths).
-	int64_t hw = 1469598103934665603ll;
-	for (int m = 0; m < K; m++) hw = (hw ^ (width[m] * 131 + S[m])) * 1099511628211ll;
-	const int64_t key[3] = {h->mm_gen, flags + (packed << 16), hw};
-	int G = 8, share = 1;
-	if (h->tile_rows > 0) {
-		G = std::max(kRpi, (h->tile_rows + kRpi - 1) / kRpi * kRpi);
-		share = h->grid_share;
-	} else if (h->autotune && Smax > 0) {
-		if (memcmp(key, h->mm_tune_key, sizeof key) != 0) {
-			// Output sizes are needed to reserve buffers for the trial runs.
-			int64_t mu_elems = 0;
-			for (int m = 0; m < K; m++)
-				mu_elems += dots ? (int64_t)S[m] * 2 * width[m] : out_off[m + 1] - out_off[m];
-			if ((rc = autotune(h, width, S, dots, ncols, mu_elems))) return rc;
-			memcpy(h->mm_tune_key, key, sizeof key);
-		}
-		G = h->mm_tune_g;
-		share = h->mm_tune_occ;
-	}
-	h->last_share = share;
-	h->last_tile_groups = G;
-	Plan p;
-	if (Smax > 0) {
-		if ((rc = make_plan(h, width, S, dots, G, share, p))) return rc;
-	} else {
-		// One moment per model: only the initial gather.
-		p.order.resize(K);
-		std::iota(p.order.begin(), p.order.end(), 0);
-		p.desc.resize(K);
-		int64_t vec = 0;
-		for (int m = 0; m < K; m++) {
-			MDesc &d = p.desc[m];
-			d = MDesc{};
-			d.N = h->mm_N[m];
-			d.e0 = h->mm_e0[m];
-			d.W = h->mm_Wm[m];
-		d.realh = h->mm_realm[m];
-			d.vec0 = vec;
-			d.w = width[m];
-			d.wp = width[m];
-			d.Q = kMaxWidth / width[m];
-			vec += h->mm_N[m] * width[m];
-		}
-		p.vec_elems = vec;
-	}
-	// Columns: X offset of each unit start vector and its output row.
-	std::vector<int> pos(K);
-	for (int k = 0; k < K; k++) pos[p.order[k]] = k;
-	std::vector<GCol> cols(ncols);
-	for (int m = 0, c = 0; m < K; m++) {
-		const MDesc &d = p.desc[pos[m]];
-		for (int b = 0; b < num_sites[m]; b++, c++) {
-			cols[c].xoff = d.vec0 + sites[c] * d.wp + (packed ? b >> 1 : b);
-			cols[c].out = out_off[m] + (int64_t)b * num_moments[m];
-			cols[c].M = num_moments[m];
-			cols[c].comp = packed ? 1 + (b & 1) : 0;
-		}
-	}
-	const int64_t mu_elems = dots ? p.d_elems : out_off[K];
-	if ((rc = reserve_plan(h, p, ncols, mu_elems))) return rc;
-	TBTKX_CHECK_HIP(hipMemcpyAsync(h->mm_cols.ptr, cols.data(), cols.size() * sizeof(GCol),
-	                               hipMemcpyHostToDevice, h->stream));
-
-	TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
-	const int64_t nsteps = run_steps(p);
-	if (h->use_graph) {
-		// The run is captured as graphs of at most kGraphSteps steps each (a
-		// few hundred kernel nodes per graph rather than one graph of three
-		// launches per step), all cached under one key and replayed in order.
-		const int64_t nchunk = nsteps > 0 ? (nsteps + kGraphSteps - 1) / kGraphSteps : 1;
-		int64_t mh = hw;
-		for (int m = 0; m < K; m++) mh = (mh ^ num_moments[m]) * 1099511628211ll;
-		int64_t gkey[GraphCache::kKey];
-		const bool key_ok = GraphCache::make_key(
-		    gkey, {h->mm_gen, flags, mh, G * 16 + share, p.nwg, packed, nchunk},
-		    {h->mm_desc.ptr, h->mm_tab.ptr, h->mm_x.ptr, h->mm_y.ptr, h->mm_part.ptr,
-		     h->mm_seg.ptr, h->mm_D.ptr, h->mm_cols.ptr, h->mm_ecol.ptr, h->mm_ev1.ptr,
-		     h->mm_ev2.ptr});
-		TBTKX_REQUIRE(key_ok, TBTKX_ERR_STATE, "tbtkx_multi_moments: graph key too long");
-		bool cached = (int64_t)h->mm_graphs.size() == nchunk;
-		for (int64_t c = 0; cached && c < nchunk; c++)
-			cached = h->mm_graphs[c].matches(gkey);
-		if (!cached) {
-			for (GraphCache &g : h->mm_graphs) g.reset();
-			h->mm_graphs.clear();
-			h->mm_graphs.resize(nchunk);
-			for (int64_t c = 0; c < nchunk; c++) {
-				GraphCache &gc = h->mm_graphs[c];
-				TBTKX_CHECK_HIP(hipStreamBeginCapture(h->stream,
-				                                      hipStreamCaptureModeThreadLocal));
-				int erc = enqueue_run(h, p, dots, ncols, c * kGraphSteps,
-				                      std::min(nsteps, (c + 1) * kGraphSteps));
-				hipError_t ec = hipStreamEndCapture(h->stream, &gc.graph);
-				if (erc) return erc;
-				TBTKX_CHECK_HIP(ec);
-				TBTKX_CHECK_HIP(hipGraphInstantiate(&gc.exec, gc.graph, nullptr, nullptr, 0));
-				memcpy(gc.key, gkey, sizeof gkey);
-			}
-		}
-		for (GraphCache &gc : h->mm_graphs) TBTKX_CHECK_HIP(hipGraphLaunch(gc.exec, h->stream));
-		h->last_launches = Smax;
-	} else {
-		if ((rc = enqueue_run(h, p, dots, ncols, 0, nsteps))) return rc;
-	}
-	TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
-	std::vector<double2> buf(mu_elems > 0 ? mu_elems : 1);
-	TBTKX_CHECK_HIP(hipMemcpyAsync(buf.data(), h->mm_D.ptr, (size_t)mu_elems * 16,
-	                               hipMemcpyDeviceToHost, h->stream));
-	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
-	float ms = 0;
-	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
-	h->last_ms = ms;
-	h->last_real = packed;
-
-	double2 *o2 = reinterpret_cast<double2 *>(out);
-	if (!dots) {
-		memcpy(o2, buf.data(), (size_t)out_off[K] * 16);
-		return TBTKX_OK;
-	}
-	for (int m = 0; m < K; m++) {
-		const MDesc &d = p.desc[pos[m]];
-		const int M = num_moments[m], w = width[m];
-		for (int b = 0; b < num_sites[m]; b++) {
-			double2 *o = o2 + out_off[m] + (int64_t)b * M;
-			// Column of vector b; packed: its component.
-			const int c = packed ? b >> 1 : b;
-			auto Dv = [&](int n, int which) {
-				const double2 v = buf[d.dof + ((int64_t)n * 2 + which) * w + c];
-				if (!packed) return v;
-				return make_double2((b & 1) ? v.y : v.x, 0.0);
-			};
-			const double2 mu0 = Dv(0, 0), mu1 = Dv(0, 1);
-			o[0] = mu0;
-			if (M > 1) o[1] = mu1;
-			for (int n = 1; n < S[m]; n++) {
-				const double2 a = Dv(n, 0), c = Dv(n, 1);
-				if (2 * n < M) o[2 * n] = make_double2(2 * a.x - mu0.x, 2 * a.y - mu0.y);
-				if (2 * n + 1 < M)
-					o[2 * n + 1] = make_double2(2 * c.x - mu1.x, 2 * c.y - mu1.y);
-			}
-		}
-	}
-	return TBTKX_OK;
+	return run_batch(h, num_sites, sites, num_moments, (flags & TBTKX_DOUBLING) != 0, packed, Start{},
+	                 out);
 }
 
 }  // extern "C"
