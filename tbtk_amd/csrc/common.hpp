@@ -94,6 +94,18 @@ struct GraphCache {
 	}
 };
 
+// The plain recurrence in one launch, the vectors resident on the chip
+// (resident.hip): C rows per workgroup (the whole model: one workgroup per start
+// vector), else G tiles of A layers x B rows with k steps between exchanges;
+// estimated time of a step. C = 0: the model does not fit or per-step launches
+// are faster.
+struct ResidentPlan {
+	int C = 0, k = 1, G = 1;
+	int L = 0, hq = 0, ds = 0, A = 0, B = 0;
+	bool wide = false;
+	double us = 0;
+};
+
 }  // namespace tbtkx
 
 struct tbtkx_context {
@@ -139,6 +151,9 @@ struct tbtkx_context {
 	tbtkx::DevBuf scol, scode, sv1, sv2, sv1r, sv2r;
 	int slot_ok = 0, slot_pal = 0, slot_vals = 0, slot_W = 0;
 	int slot_half = 0;   // most entries on either side of a row's diagonal
+	// Rows per layer of the slot form's lattice view and the farthest column
+	// within a layer (layer_stride; 0: none).
+	int tile_L = 0, tile_ds = 0;
 	// Row patterns of the slot form (pat_ok): one byte per row (ppid) into
 	// pat_count patterns of 8 offsets (ptoff) and 8 palette codes (ptcode).
 	tbtkx::DevBuf ppid, ptoff, ptcode;
@@ -162,6 +177,8 @@ struct tbtkx_context {
 	std::vector<int64_t> res_host;   // host copy of res_in, alive during its upload
 	uint32_t res_epoch = 0;
 	int use_resident = 1;
+	tbtkx::ResidentPlan res_plan;   // of res_plan_key (resident_plan)
+	int64_t res_plan_key[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
 	int last_resident = 0;   // the last plain call ran resident
 	int num_cus = 0;
 
@@ -311,15 +328,8 @@ inline PlainForm plain_form(const tbtkx_context *h) {
 	return f;
 }
 
-// The plain recurrence in one launch, the vectors resident on the chip
-// (resident.hip): C rows per workgroup (the whole model: one workgroup per start
-// vector), k steps between exchanges, estimated time of a step. C = 0: the
-// model does not fit or per-step launches are faster.
-struct ResidentPlan {
-	int C = 0, k = 1;
-	double us = 0;
-};
-ResidentPlan resident_plan(const tbtkx_context *h, int cus);
+// The resident recurrence of this model and form (made once per model).
+ResidentPlan resident_plan(tbtkx_context *h, int cus);
 // Enqueues the moments of V start vectors (V = 1 unless plan.C covers the
 // model) into h->coef, one row of M per entry of `to`; vector v's entries are
 // toff[v] .. toff[v + 1], ascending.

@@ -12,16 +12,22 @@
 // LDS round trip below. Measured per step, real H: 0.25 us at 600 states, 0.37
 // at 1800, 0.65 at 4042 (per-step launches: 3.7-3.9 us with the gaps).
 //
-// Models beyond one workgroup (MULTI): the rows are cut into G chunks of C
-// consecutive rows, one workgroup each, and a workgroup also computes a halo.
-// With D = max |column - row| and k steps between exchanges, the halo of x_n
-// is k D rows on either side; step s of a phase computes the rows within
-// (k - 1 - s) D of the chunk, so after k steps the chunk is exact and the
-// halo is taken from the two neighbours (C >= k D). The halo of x_{n-1} reaches
-// (k - 1) D; its rows are published one step early. An exchange costs about
-// 1.1 us of latency between two XCDs plus its bytes, hence several steps per
-// exchange where D is small against C. 73,006 states (D = 422, C = 1024, k = 2):
-// 1.31 us per step; 64,000 states (D = 64, C = 512, k = 8): 0.59 us.
+// Models beyond one workgroup (MULTI): the rows are seen as a grid of layers of L
+// consecutive rows, and every column of the matrix lies `hq` layers and at
+// most `ds` rows away from its row. The grid is cut into tiles of A layers x B
+// rows, one workgroup each, and a workgroup also computes a halo. With k
+// steps between exchanges the halo of x_n is k rings of hq layers and ds rows
+// around the tile; step s of a phase computes the tile and k - 1 - s rings, so
+// after k steps the tile is exact and the halo is taken from the neighbours
+// (A >= k hq, B >= k ds). The halo of x_{n-1} has k - 1 rings; its rows are
+// published one step early. L is a lattice's slowest stride (hq = 1), or the
+// whole model (hq = 0: chunks of consecutive rows, ds = max |column - row|). A
+// place of the window outside its layer is the row of that linear index, so
+// bonds that wrap around within a layer need nothing special. An exchange costs
+// about 1.3 us between two XCDs plus its bytes, hence several steps per exchange
+// where the rings are small against the tile. Measured per step: 73,006 states
+// (lattice 173 x 211 x 2) in 143 tiles of 16 x 33 rows, k = 4: 1.00 us; in chunks
+// of 1024 consecutive rows (halo 422 rows a step), k = 2: 1.31 us.
 //
 // Waiting: the launch is cooperative, so all workgroups are resident, and every
 // wait is bounded (one second, or another workgroup's give-up): the kernel
@@ -103,7 +109,9 @@ struct ResArgs {
 	const uint8_t *scode;          // palette codes, or null
 	const S *sv1, *sv2;            // slot values of H/s and 2H/s (no palette)
 	const S *pal, *diag;           // palette (256 + 256), diagonal (N + N)
-	int N, W, C, D, k, G;
+	int N, W, k, G;
+	int L, La, hq, ds;             // rows per layer, layers, reach in layers and in rows
+	int A, B, tb;                  // tile: layers, rows of each; tiles along a layer
 	const int64_t *from;           // per vector
 	const int *toff;               // per vector: first entry of its to-list
 	const int64_t *to;             // ascending per vector
@@ -114,6 +122,55 @@ struct ResArgs {
 	uint32_t epoch;
 	uint32_t *err;
 };
+
+// A workgroup's tile: first layer and row of it, extents.
+struct Tile {
+	int a, b, h, w;
+};
+template <typename S>
+__device__ __forceinline__ Tile tile_of(const ResArgs<S> &a, int g) {
+	Tile t;
+	t.a = g / a.tb * a.A;
+	t.b = g % a.tb * a.B;
+	t.h = t.a + a.A < a.La ? a.A : a.La - t.a;
+	t.w = t.b + a.B < a.L ? a.B : a.L - t.b;
+	return t;
+}
+struct Cell {
+	int a, b;   // layer, row in it; may lie outside the grid
+};
+// d-th place of the frame of rectangle t that is fh layers and fw rows thick.
+__device__ __forceinline__ Cell frame_cell(const Tile &t, int d, int fh, int fw) {
+	const int band = fh * t.w;
+	if (d < 2 * band) {
+		const int q = d / t.w;
+		return Cell{t.a + (q < fh ? q : t.h - 2 * fh + q), t.b + d - q * t.w};
+	}
+	const int q = (d - 2 * band) / (2 * fw), o = d - 2 * band - q * 2 * fw;
+	return Cell{t.a + fh + q, t.b + (o < fw ? o : t.w - 2 * fw + o)};
+}
+__device__ __forceinline__ Tile grown(const Tile &t, int h, int w) {
+	return Tile{t.a - h, t.b - w, t.h + 2 * h, t.w + 2 * w};
+}
+__device__ __forceinline__ int area(const Tile &t) { return t.h * t.w; }
+// Entries q0 .. q1 - 1 of the ascending list `to` that lie in layers a .. a + h - 1
+// of the tile's span of rows.
+template <typename S>
+__device__ __forceinline__ void span(const ResArgs<S> &a, const Tile &t, int *q0, int *q1) {
+	const int64_t r0 = (int64_t)t.a * a.L + t.b, r1 = (int64_t)(t.a + t.h - 1) * a.L + t.b + t.w;
+	auto first = [&](int64_t r) __attribute__((always_inline)) {
+		int lo = *q0, hi = *q1;
+		while (lo < hi) {
+			const int m = (lo + hi) >> 1;
+			if (a.to[m] < r) lo = m + 1;
+			else hi = m;
+		}
+		return lo;
+	};
+	const int f = first(r0);
+	*q1 = first(r1);
+	*q0 = f;
+}
 
 // A row's entries in CSR order: up to H before its (first) diagonal entry,
 // the diagonal, up to H after it. Unused places hold the value -0.0 and the
@@ -128,24 +185,37 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	__shared__ S buf[2 * kStride];
 	__shared__ int stop;
 	const int t = threadIdx.x;
+	const int wave = __builtin_amdgcn_readfirstlane(t & ~63);   // its first thread
 	const int g = MULTI ? (int)blockIdx.x : 0;
 	const int vec = MULTI ? 0 : (int)blockIdx.x;
-	const int N = a.N, D = MULTI ? a.D : 0, k = MULTI ? a.k : 1;
-	const int halo = k * D;
-	const int r0 = MULTI ? g * a.C : 0;
-	const int r1 = MULTI ? (r0 + a.C < N ? r0 + a.C : N) : N;
-	const int w0 = MULTI ? (r0 > halo ? r0 - halo : 0) : 0;
-	const int w1 = MULTI ? (r1 + halo < N ? r1 + halo : N) : N;
-	const int win = w1 - w0, own = r1 - r0;
-	// i-th row of the workgroup: its own rows first, then the halo in rings of
-	// D rows, left and right; -1 outside the matrix.
-	auto row_of = [&](int i) __attribute__((always_inline)) -> int {
-		if (i < own) return r0 + i;
-		if (!MULTI) return -1;
-		const int d = i - own, q = d / (2 * D), o = d - q * 2 * D;
-		if (q >= k) return -1;
-		const int r = o < D ? r0 - (q + 1) * D + o : r1 + q * D + (o - D);
-		return r < 0 || r >= N ? -1 : r;
+	const int N = a.N, k = MULTI ? a.k : 1, L = MULTI ? a.L : N;
+	const int hq = MULTI ? a.hq : 0, ds = MULTI ? a.ds : 0;
+	const Tile tile = MULTI ? tile_of(a, g) : Tile{0, 0, 1, N};
+	const Tile window = grown(tile, k * hq, k * ds);
+	const int win = area(window), own = area(tile), P = window.w;
+	// Rows within q rings of the tile.
+	auto within = [&](int q) __attribute__((always_inline)) {
+		return (tile.h + 2 * q * hq) * (tile.w + 2 * q * ds);
+	};
+	// Element of the window at a cell, and the row of an element (-1: none).
+	auto place = [&](Cell c) __attribute__((always_inline)) {
+		return (c.a - window.a) * P + c.b - window.b;
+	};
+	auto row_in = [&](int p) __attribute__((always_inline)) -> int {
+		if (!MULTI) return p;
+		const int q = p / P;
+		const int64_t r = (int64_t)(window.a + q) * L + window.b + p - q * P;
+		return r < 0 || r >= N ? -1 : (int)r;
+	};
+	// Element of the workgroup's i-th row: the tile, then the rings outwards;
+	// -1: none.
+	auto element = [&](int i) __attribute__((always_inline)) -> int {
+		if (!MULTI) return i < own ? i : -1;
+		if (i < own) return place(Cell{tile.a + i / tile.w, tile.b + i % tile.w});
+		for (int q = 1; q <= k; q++)
+			if (i < within(q))
+				return place(frame_cell(grown(tile, q * hq, q * ds), i - within(q - 1), hq, ds));
+		return -1;
 	};
 	// Byte offsets into a vector: pos of the row itself (0: no row), adr of
 	// entry s (low half) and s + H (high half).
@@ -154,11 +224,11 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	bool hasd[R];
 #pragma unroll
 	for (int j = 0; j < R; j++) {
-		const int r = row_of(t + T * j);
-		pos[j] = r < 0 ? 0u : (uint32_t)(r - w0 + 1) * (uint32_t)sizeof(S);
+		const int p = element(t + T * j);
+		pos[j] = p < 0 || row_in(p) < 0 ? 0u : (uint32_t)(p + 1) * (uint32_t)sizeof(S);
 	}
 	auto row_at = [&](int j) __attribute__((always_inline)) {
-		return (int)(pos[j] / (uint32_t)sizeof(S)) - 1 + w0;
+		return row_in((int)(pos[j] / (uint32_t)sizeof(S)) - 1);
 	};
 	auto at = [](const S *v, uint32_t o) __attribute__((always_inline)) -> const S & {
 		return *reinterpret_cast<const S *>(reinterpret_cast<const char *>(v) + o);
@@ -190,8 +260,10 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 					diag[j] = v;
 					continue;
 				}
-				int col = r + off - w0;
-				if (col < 0 || col >= win) col = r - w0;
+				const int here = (int)(pos[j] / (uint32_t)sizeof(S)) - 1;
+				const int lay = !MULTI || !hq ? 0 : 2 * off > L ? 1 : 2 * off < -L ? -1 : 0;
+				int col = here + off - lay * (L - P);
+				if (col < 0 || col >= win) col = here;
 				const int u = hd ? c++ : b++;
 				const uint32_t o = (uint32_t)(1 + col) * (uint32_t)sizeof(S);
 #pragma unroll
@@ -206,7 +278,7 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	load(true);
 	if (t < 2) buf[t * kStride] = A::num(1.0);
 	const int from = (int)a.from[vec];
-	for (int i = t; i < win; i += T) buf[1 + i] = A::num(w0 + i == from ? 1.0 : 0.0);
+	for (int i = t; i < win; i += T) buf[1 + i] = A::num(row_in(i) == from ? 1.0 : 0.0);
 #pragma unroll
 	for (int j = 0; j < R; j++) {
 		xo[j] = A::num(pos[j] != 0 && row_at(j) == from ? 1.0 : 0.0);
@@ -215,30 +287,23 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	if (t == 0) stop = 0;
 	// This workgroup's part of the to-list.
 	int q0 = a.toff[vec], q1 = a.toff[vec + 1];
-	if (MULTI) {
-		int lo = q0, hi = q1;
-		while (lo < hi) {
-			const int m = (lo + hi) >> 1;
-			if (a.to[m] < r0) lo = m + 1;
-			else hi = m;
-		}
-		const int first = lo;
-		hi = q1;
-		while (lo < hi) {
-			const int m = (lo + hi) >> 1;
-			if (a.to[m] < r1) lo = m + 1;
-			else hi = m;
-		}
-		q0 = first;
-		q1 = lo;
-	}
-	const int my = q0 + t < q1 ? (int)a.to[q0 + t] - w0 + 1 : -1;
+	if (MULTI) span(a, tile, &q0, &q1);
+	// Element of the to-list's entry q, -1: of another tile.
+	auto target = [&](int q) __attribute__((always_inline)) -> int {
+		const int r = (int)a.to[q];
+		if (!MULTI) return r;
+		const int b = hq ? r % L : r;
+		return b < tile.b || b >= tile.b + tile.w ? -1 : place(Cell{hq ? r / L : 0, b});
+	};
+	const int my = q0 + t < q1 ? target(q0 + t) : -1;
 	__syncthreads();
 
 	auto gather = [&](const S *cur, int n) __attribute__((always_inline)) {
-		if (my >= 0) a.coef[(int64_t)(q0 + t) * a.M + n] = A::moment(cur[my]);
-		for (int q = q0 + t + T; q < q1; q += T)
-			a.coef[(int64_t)q * a.M + n] = A::moment(cur[(int)a.to[q] - w0 + 1]);
+		if (my >= 0) a.coef[(int64_t)(q0 + t) * a.M + n] = A::moment(cur[1 + my]);
+		for (int q = q0 + t + T; q < q1; q += T) {
+			const int p = target(q);
+			if (p >= 0) a.coef[(int64_t)q * a.M + n] = A::moment(cur[1 + p]);
+		}
 	};
 	gather(buf, 0);
 
@@ -269,7 +334,8 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 		if constexpr (!MULTI) {
 			rows(std::integral_constant<int, R>{}, first, src, dst);
 		} else {
-			const int rn = (need + T - 1) / T;
+			// Rounds with rows of this wavefront.
+			const int rn = (need - wave + T - 1) / T;
 #define TBTKX_ROWS(Q)                                                                        \
 	if constexpr (R >= Q)                                                                \
 		if (rn == Q) rows(std::integral_constant<int, Q>{}, first, src, dst);
@@ -296,20 +362,32 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	auto slot_of = [&](int p, int v, int c, int r) __attribute__((always_inline)) {
 		return (uint32_t)((((p & 1) * 2 + v) * NC + c) * N + r);
 	};
-	// Publish the current vector of the rows within `ext` of the chunk's
+	// Publish the current vector of the tile's rows within `ext` rings of its
 	// edges, as vector v of phase p.
 	auto publish = [&](int p, int v, int ext) __attribute__((always_inline)) {
 #pragma unroll
 		for (int j = 0; j < R; j++) {
 			const int i = t + T * j;
 			if (i >= own) break;
-			if ((g > 0 && i < ext) || (g < a.G - 1 && i >= own - ext)) {
+			const int la = i / tile.w, lb = i - la * tile.w;
+			if (la < ext * hq || la >= tile.h - ext * hq || lb < ext * ds ||
+			    lb >= tile.w - ext * ds) {
+				const int r = (tile.a + la) * L + tile.b + lb;
 #pragma unroll
 				for (int c = 0; c < NC; c++)
-					put(xg, slot_of(p, v, c, r0 + i), A::part(xo[j], c), a.epoch + (uint32_t)p);
+					put(xg, slot_of(p, v, c, r), A::part(xo[j], c), a.epoch + (uint32_t)p);
 			}
 		}
 	};
+	// This thread's first rows of the inner rings and of the outermost.
+	const int inner = within(k - 1), outer = within(k);
+	int pa0 = -1, pb0 = -1, ra0 = -1, rb0 = -1;
+	if (MULTI) {
+		if (own + t < inner) pa0 = element(own + t);
+		if (inner + t < outer) pb0 = element(inner + t);
+		if (pa0 >= 0) ra0 = row_in(pa0);
+		if (pb0 >= 0) rb0 = row_in(pb0);
+	}
 	// Take the neighbours' rows of phase p. Returns false when the wait was
 	// given up.
 	auto exchange = [&](S *cur, S *oth, int p) __attribute__((always_inline)) -> bool {
@@ -317,11 +395,15 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 		const long long begin = wall_clock64();
 		// Per pass one row of the inner rings (x_n and x_{n-1}) and one of the
 		// outermost ring (x_n only), all in flight together.
-		const int inner = own + 2 * (k - 1) * D, outer = inner + 2 * D;
 		int spins = 0;
 		for (int i = t; own + i < inner || inner + i < outer; i += T) {
-			const int ra = own + i < inner ? row_of(own + i) : -1;
-			const int rb = inner + i < outer ? row_of(inner + i) : -1;
+			int pa = pa0, pb = pb0, ra = ra0, rb = rb0;
+			if (i != t) {
+				pa = own + i < inner ? element(own + i) : -1;
+				pb = inner + i < outer ? element(inner + i) : -1;
+				ra = pa < 0 ? -1 : row_in(pa);
+				rb = pb < 0 ? -1 : row_in(pb);
+			}
 			u32x4 wa[2 * NC], wb[NC];
 			const u32x4 none = {0, want, 0, want};
 			for (;;) {
@@ -353,10 +435,10 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 				return A::make(__hiloint2double(w[0].z, w[0].x), __hiloint2double(w[NC - 1].z, w[NC - 1].x));
 			};
 			if (ra >= 0) {
-				cur[1 + ra - w0] = value(wa);
-				oth[1 + ra - w0] = value(wa + NC);
+				cur[1 + pa] = value(wa);
+				oth[1 + pa] = value(wa + NC);
 			}
-			if (rb >= 0) cur[1 + rb - w0] = value(wb);
+			if (rb >= 0) cur[1 + pb] = value(wb);
 		}
 		__syncthreads();
 		if (stop) return false;
@@ -370,18 +452,18 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	};
 
 	S *const xa = buf, *const xb = buf + kStride;
-	int sub = 0, phase = 0, need = own + 2 * (k - 1) * D;
+	int sub = 0, phase = 0, need = inner;
 	auto after = [&](S *cur, S *oth, int n) __attribute__((always_inline)) -> bool {
 		gather(cur, n);
 		if (!MULTI) return true;
-		need -= 2 * D;
 		++sub;
+		if (sub < k) need = within(k - 1 - sub);
 		// x_{n-1} of the phase's end goes out one step ahead.
-		if (sub == k - 1) publish(phase + 1, 1, halo - D);
+		if (sub == k - 1) publish(phase + 1, 1, k - 1);
 		if (sub == k && n + 1 < a.M) {
 			sub = 0;
-			need = own + 2 * (k - 1) * D;
-			publish(++phase, 0, halo);
+			need = inner;
+			publish(++phase, 0, k);
 			return exchange(cur, oth, phase);
 		}
 		return true;
@@ -401,6 +483,212 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	if (n < a.M) {
 		step(std::false_type{}, xb, xa, need);
 		after(xa, xb, n);
+	}
+}
+
+// Measured per step: 2,097,152 states (1024 x 1024 x 2) in 256 tiles of 64 x 128
+// rows 2.7 us, where a launch per step took 11.9 (50 MB of vectors and 18 MB
+// of matrix from the cache beyond L2); 1,048,576 states (512 x 512 x 4) 1.9 us;
+// 864,000 states (96 x 100 x 90) 4.1 us, a frame of 2800 of 4000 rows there. Bound by
+// LDS reads (8 per row and step) and the exchange.
+// Large models (palette only): up to 8192 real rows per workgroup, one step per
+// exchange. LDS holds one window of x_n, which is overwritten after a
+// barrier; a row's entries are 16-bit window elements and 8-bit palette codes in
+// registers, the palette's values come from LDS. The tile's frame comes first
+// among its rows, so it is computed and published first and the exchange runs
+// while the rest is computed. Element 0 of the window holds 1 and code 255 the
+// value -0.0, for unused places.
+constexpr int kWideBytes = 159200;
+template <typename S, int H, int R>
+__global__ __launch_bounds__(kResThreads) void resident_wide(ResArgs<S> a) {
+#pragma clang fp contract(off)
+	typedef R64<S> A;
+	constexpr int T = kResThreads, NC = sizeof(S) / 8, CW = (2 * H + 3) / 4;
+	__shared__ S buf[kWideBytes / sizeof(S)];
+	__shared__ S pal[256];
+	__shared__ int stop;
+	const int t = threadIdx.x, N = a.N, L = a.L, hq = a.hq, ds = a.ds;
+	const Tile tile = tile_of(a, (int)blockIdx.x);
+	const Tile window = grown(tile, hq, ds), inside = grown(tile, -hq, -ds);
+	const int win = area(window), own = area(tile), P = window.w;
+	const int frame = own - area(inside), ring = win - own;
+	auto place = [&](Cell c) __attribute__((always_inline)) {
+		return (c.a - window.a) * P + c.b - window.b;
+	};
+	auto row_in = [&](int p) __attribute__((always_inline)) -> int {
+		const int q = p / P;
+		const int64_t r = (int64_t)(window.a + q) * L + window.b + p - q * P;
+		return r < 0 || r >= N ? -1 : (int)r;
+	};
+	S diag[R], xo[R], yo[R];
+	uint32_t adr[R][H], code[R][CW], pos[R], hasd = 0;
+#pragma unroll
+	for (int j = 0; j < R; j++) {
+		const int i = t + T * j;
+		pos[j] = 0;
+		if (i < frame) {
+			pos[j] = place(frame_cell(tile, i, hq, ds)) + 1;
+		} else if (i < own) {
+			const int q = (i - frame) / inside.w;
+			pos[j] = place(Cell{inside.a + q, inside.b + (i - frame) - q * inside.w}) + 1;
+		}
+	}
+	auto diagonals = [&](bool first) __attribute__((always_inline)) {
+#pragma unroll
+		for (int j = 0; j < R; j++) {
+			diag[j] = A::num(-0.0);
+			if (hasd >> j & 1) diag[j] = a.diag[(first ? 0 : N) + row_in((int)pos[j] - 1)];
+		}
+		if (t < 256) pal[t] = t == 255 ? A::num(-0.0) : a.pal[(first ? 0 : 256) + t];
+	};
+	const int from = (int)a.from[0];
+#pragma unroll
+	for (int j = 0; j < R; j++) {
+#pragma unroll
+		for (int s = 0; s < H; s++) adr[j][s] = 0;
+#pragma unroll
+		for (int s = 0; s < CW; s++) code[j][s] = 0xffffffffu;
+		const int here = (int)pos[j] - 1, r = pos[j] ? row_in(here) : -1;
+		bool hd = false;
+		int b = 0, c = H;
+		for (int s = 0; s < a.W && pos[j]; s++) {
+			const int64_t e = (int64_t)s * N + r;
+			const int off = a.scol[e];
+			if (off == kSlotPad) break;
+			const uint32_t q = a.scode[e];
+			if (off == 0 && !hd) {
+				hd = true;
+				continue;
+			}
+			const int lay = !hq ? 0 : 2 * off > L ? 1 : 2 * off < -L ? -1 : 0;
+			const uint32_t o = (uint32_t)(here + off - lay * (L - P) + 1);
+			const int u = hd ? c++ : b++;
+#pragma unroll
+			for (int z = 0; z < 2 * H; z++) {
+				adr[j][z % H] |= z == u ? (z < H ? o : o << 16) : 0u;
+				code[j][z / 4] ^= z == u ? (q ^ 255u) << 8 * (z % 4) : 0u;
+			}
+		}
+		hasd |= (uint32_t)hd << j;
+		xo[j] = A::num(pos[j] != 0 && r == from ? 1.0 : 0.0);
+		yo[j] = A::num(0.0);
+	}
+	diagonals(true);
+	if (t == 0) {
+		buf[0] = A::num(1.0);
+		stop = 0;
+	}
+	for (int i = t; i < win; i += T) buf[1 + i] = A::num(row_in(i) == from ? 1.0 : 0.0);
+	int q0 = a.toff[0], q1 = a.toff[1];
+	span(a, tile, &q0, &q1);
+	auto target = [&](int q) __attribute__((always_inline)) -> int {
+		const int r = (int)a.to[q], b = hq ? r % L : r;
+		return b < tile.b || b >= tile.b + tile.w ? -1 : place(Cell{hq ? r / L : 0, b});
+	};
+	const int my = q0 + t < q1 ? target(q0 + t) : -1;
+	auto gather = [&](int n) __attribute__((always_inline)) {
+		if (my >= 0) a.coef[(int64_t)(q0 + t) * a.M + n] = A::moment(buf[1 + my]);
+		for (int q = q0 + t + T; q < q1; q += T) {
+			const int p = target(q);
+			if (p >= 0) a.coef[(int64_t)q * a.M + n] = A::moment(buf[1 + p]);
+		}
+	};
+	const __amdgpu_buffer_rsrc_t xg = __builtin_amdgcn_make_buffer_rsrc(a.xg, 0, a.xg_bytes, 0x00027000);
+	auto slot_of = [&](int n, int c, int r) __attribute__((always_inline)) {
+		return (uint32_t)(((n & 1) * NC + c) * N + r);
+	};
+	const int r0 = t < frame ? row_in((int)pos[0] - 1) : -1;
+	const int ph0 = t < ring ? place(frame_cell(window, t, hq, ds)) : -1;
+	const int rh0 = ph0 < 0 ? -1 : row_in(ph0);
+	// Waits for row r of x_n; false when the wait was given up.
+	auto take = [&](int r, int n, S *x) __attribute__((always_inline)) {
+		const uint32_t want = a.epoch + (uint32_t)n;
+		const long long begin = wall_clock64();
+		int spins = 0;
+		for (;;) {
+			u32x4 w[NC];
+			bool ok = true;
+#pragma unroll
+			for (int c = 0; c < NC; c++) w[c] = get(xg, slot_of(n, c, r));
+#pragma unroll
+			for (int c = 0; c < NC; c++) ok = ok && w[c].y == want && w[c].w == want;
+			if (ok) {
+				*x = A::make(__hiloint2double(w[0].z, w[0].x),
+				             __hiloint2double(w[NC - 1].z, w[NC - 1].x));
+				return;
+			}
+			if ((++spins & 63) == 0 &&
+			    (wall_clock64() - begin > kWaitTicks ||
+			     __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+				__hip_atomic_store(a.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				stop = 1;
+				return;
+			}
+		}
+	};
+	auto step = [&](auto first, int n) __attribute__((always_inline)) {
+		constexpr bool FIRST = decltype(first)::value;
+#pragma unroll
+		for (int j = 0; j < R; j++) {
+			S x[2 * H], v[2 * H];
+			// The packed words stay packed: unpacked once for all steps, they would
+			// take more registers than there are.
+#pragma unroll
+			for (int s = 0; s < H; s++) asm volatile("" : "+v"(adr[j][s]));
+#pragma unroll
+			for (int s = 0; s < CW; s++) asm volatile("" : "+v"(code[j][s]));
+#pragma unroll
+			for (int s = 0; s < H; s++) {
+				x[s] = buf[adr[j][s] & 0xffffu];
+				x[s + H] = buf[adr[j][s] >> 16];
+			}
+#pragma unroll
+			for (int s = 0; s < 2 * H; s++) v[s] = pal[code[j][s / 4] >> 8 * (s % 4) & 255u];
+			S acc = FIRST ? A::num(0.0) : A::neg(yo[j]);
+#pragma unroll
+			for (int s = 0; s < H; s++) acc = A::add(acc, A::mul(v[s], x[s]));
+			acc = A::add(acc, A::mul(diag[j], A::pick(hasd >> j & 1, xo[j], A::num(1.0))));
+#pragma unroll
+			for (int s = H; s < 2 * H; s++) acc = A::add(acc, A::mul(v[s], x[s]));
+			yo[j] = xo[j];
+			xo[j] = acc;
+			if (T * j < frame && t + T * j < frame) {
+				const int r = j == 0 ? r0 : row_in((int)pos[j] - 1);
+#pragma unroll
+				for (int c = 0; c < NC; c++)
+					put(xg, slot_of(n, c, r), A::part(acc, c), a.epoch + (uint32_t)n);
+			}
+		}
+		const bool more = n + 1 < a.M;
+		S h0 = A::num(0.0);
+		if (more && rh0 >= 0) take(rh0, n, &h0);
+		__syncthreads();
+#pragma unroll
+		for (int j = 0; j < R; j++)
+			if (pos[j]) {
+				asm volatile("" : "+v"(pos[j]));
+				buf[pos[j]] = xo[j];
+			}
+		if (rh0 >= 0) buf[1 + ph0] = h0;
+		for (int i = t + T; more && i < ring; i += T) {
+			const int p = place(frame_cell(window, i, hq, ds)), r = row_in(p);
+			if (r >= 0) take(r, n, &buf[1 + p]);
+		}
+		__syncthreads();
+	};
+	__syncthreads();
+	gather(0);
+	if (a.M > 1) {
+		step(std::true_type{}, 1);
+		if (stop) return;
+		gather(1);
+		diagonals(false);
+		__syncthreads();
+	}
+	for (int n = 2; n < a.M; n++) {
+		step(std::false_type{}, n);
+		if (stop) return;
+		gather(n);
 	}
 }
 
@@ -442,8 +730,30 @@ int launch_res_r(tbtkx_context *h, const ResArgs<S> &a, unsigned grid, int r) {
 	return TBTKX_ERR_STATE;
 }
 
+// The same of the wide kernel: a row takes 3 values, H + (2 H + 3) / 4 words and
+// its element.
+template <typename S>
+constexpr int wide_rows(int H) {
+	if (std::is_same<S, double>::value) return H <= 2 ? 8 : H == 3 ? 7 : 5;
+	return H <= 2 ? 4 : H == 3 ? 3 : 2;
+}
+
+template <typename S, int H, int R>
+int launch_wide(tbtkx_context *h, ResArgs<S> a, unsigned grid, int r) {
+	if constexpr (R <= wide_rows<S>(H)) {
+		if (r > R) return launch_wide<S, H, R + 1>(h, a, grid, r);
+		void *p[] = {&a};
+		TBTKX_CHECK_HIP(hipLaunchCooperativeKernel((const void *)resident_wide<S, H, R>, dim3(grid),
+		                                           dim3(kResThreads), p, 0, h->stream));
+		return TBTKX_OK;
+	}
+	set_error("resident recurrence: too many rows per thread");
+	return TBTKX_ERR_STATE;
+}
+
 template <typename S, int H>
-int launch_res_h(tbtkx_context *h, const ResArgs<S> &a, unsigned grid, int r) {
+int launch_res_h(tbtkx_context *h, const ResArgs<S> &a, unsigned grid, int r, bool wide) {
+	if (wide) return launch_wide<S, H, 1>(h, a, grid, r);
 	return a.G > 1 ? launch_res_r<S, H, 1, true>(h, a, grid, r)
 	               : launch_res_r<S, H, 1, false>(h, a, grid, r);
 }
@@ -463,10 +773,15 @@ int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *fr
 	a.diag = real ? h->pdiagr.as<S>() : h->pdiag.as<S>();
 	a.N = (int)h->N;
 	a.W = h->slot_W;
-	a.D = (int)(h->band < h->N ? h->band : 0);
 	a.k = plan.k;
-	a.C = plan.C;
-	a.G = (int)((h->N + plan.C - 1) / plan.C);
+	a.G = plan.G;
+	a.L = plan.L;
+	a.La = (int)(h->N / plan.L);
+	a.hq = plan.hq;
+	a.ds = plan.ds;
+	a.A = plan.A;
+	a.B = plan.B;
+	a.tb = (plan.L + plan.B - 1) / plan.B;
 	a.M = M;
 	int rc;
 	// Start vectors, to-list and its offsets in one copy.
@@ -486,7 +801,7 @@ int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *fr
 	if (a.G > 1) {
 		// Tags are never used twice: a buffer starts all zero and the tags go on
 		// from launch to launch.
-		const size_t bytes = (size_t)h->N * sizeof(S) / 8 * 64;
+		const size_t bytes = (size_t)h->N * sizeof(S) / 8 * (plan.wide ? 32 : 64);
 		const uint32_t phases = (uint32_t)(M / plan.k + 2);
 		if (!h->res_xg.ptr || h->res_xg.bytes < bytes || h->res_epoch > 0xffffffffu - phases) {
 			if ((rc = h->res_xg.reserve(bytes))) return rc;
@@ -502,64 +817,118 @@ int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *fr
 		a.epoch = h->res_epoch;
 		h->res_epoch += phases;
 	}
-	const int rows = a.G > 1 ? a.C + 2 * (a.k - 1) * a.D : a.N;
+	const int q = 2 * (a.k - 1);
+	const int rows = a.G > 1 ? (a.A + q * a.hq) * (a.B + q * a.ds) : a.N;
 	const int r = (rows + kResThreads - 1) / kResThreads;
 	const unsigned grid = a.G > 1 ? (unsigned)a.G : (unsigned)V;
 	switch (h->slot_half) {
 	case 0:
-	case 1: return launch_res_h<S, 1>(h, a, grid, r);
-	case 2: return launch_res_h<S, 2>(h, a, grid, r);
-	case 3: return launch_res_h<S, 3>(h, a, grid, r);
-	default: return launch_res_h<S, 4>(h, a, grid, r);
+	case 1: return launch_res_h<S, 1>(h, a, grid, r, plan.wide);
+	case 2: return launch_res_h<S, 2>(h, a, grid, r, plan.wide);
+	case 3: return launch_res_h<S, 3>(h, a, grid, r, plan.wide);
+	default: return launch_res_h<S, 4>(h, a, grid, r, plan.wide);
 	}
 }
 
 }  // namespace
 
-// The model fits one workgroup's registers and LDS, or chunks of it fit and
-// their exchanges cost less than a launch per step. Times in us, from the
-// measurements in this file's head; a launch per step takes 3.8 us up to
-// 200,000 states and the slot step's bytes at 5.5 TB/s above.
-ResidentPlan resident_plan(const tbtkx_context *h, int cus) {
+// The model fits one workgroup's registers and LDS, or tiles of it fit and
+// their exchanges cost less than a launch per step. Times in us, fitted to
+// (model and measured, real H, H = 2 unless said): narrow, 73,006 states k = 1 1.9
+// 1.8, k = 2 1.3 1.4, k = 4 1.0 1.0, k = 8 1.1 1.1; 524,288 states k = 4 1.6 1.8;
+// wide, 73,006 states 1.6 1.6, 524,288 states 2.0 2.1, 2,097,152 states 3.0 2.7,
+// 1,048,576 states H = 3 2.8 1.9, 864,000 states H = 3 4.6 4.1. A launch per step
+// takes 2.7 us up to 200,000 states and the slot step's bytes at 5.5 TB/s above.
+static ResidentPlan make_plan(const tbtkx_context *h, const PlainForm &f, int cus) {
 	ResidentPlan best;
-	const PlainForm f = plain_form(h);
 	if (!h->use_resident || !f.slot || h->use_graph || h->slot_rows || h->use_patterns != 1 ||
 	    h->slot_half > 4)
 		return best;
 	const bool real = h->real_path && h->h_real;
 	const int H = h->slot_half;
-	const int64_t N = h->N, D = h->band;
-	const int window = (real ? R64<double>::kStride : R64<Z2>::kStride) - 1;
+	const int64_t N = h->N, T = kResThreads;
+	const int64_t window = (real ? R64<double>::kStride : R64<Z2>::kStride) - 1;
+	const int64_t wide_window = kWideBytes / (real ? 8 : 16) - 1;
 	const int one = real ? max_rows<double, false>(H) : max_rows<Z2, false>(H);
 	const int many = real ? max_rows<double, true>(H) : max_rows<Z2, true>(H);
+	const int wide = !f.pal ? 0 : real ? wide_rows<double>(H) : wide_rows<Z2>(H);
 	// One round of rows (1024), and what a step takes without any.
 	const double set = (real ? 0.025 : 0.06) * (2 * H + 1), base = 0.14;
-	if (N <= (int64_t)one * kResThreads && N <= window) {
-		best.C = (int)N;
-		best.k = 1;
-		best.us = base + set * (double)((N + kResThreads - 1) / kResThreads);
+	if (N <= (int64_t)one * T && N <= window) {
+		best.C = best.L = best.B = (int)N;
+		best.A = 1;
+		best.us = base + set * (double)((N + T - 1) / T);
 		return best;
 	}
-	if (D >= N) return best;
-	double limit = std::max(3.8, f.bytes / 5.5e6);
-	for (int k = 1; k <= 16; k++)
-		for (int q = 1; q <= many; q++) {
-			const int64_t C = (int64_t)q * kResThreads - 2 * (k - 1) * D;
-			if (C < k * D || C + 2 * k * D > window || C >= N) continue;
-			const int64_t G = (N + C - 1) / C;
-			if (G > cus) continue;
-			double us = 1.1 + (double)G * (2 * k - 1) * 2 * D * (real ? 32 : 64) / 8e6;
-			for (int s = 0; s < k; s++)
-				us += base + set * (double)((C + 2 * (k - 1 - s) * D + kResThreads - 1) / kResThreads);
-			us /= k;
-			if (us < limit) {
-				limit = us;
-				best.C = (int)C;
-				best.k = k;
-				best.us = us;
+	double limit = std::max(2.7, f.bytes / 5.5e6);
+	// Tiles of every form that fits and has no more of them than CUs.
+	auto tiles = [&](int64_t L, int64_t hq, int64_t ds) {
+		const int64_t La = N / L;
+		if (ds <= 0 || (int64_t)cus * T * std::max(many, wide) < N) return;
+		for (int64_t ta = 1; ta <= (hq ? std::min<int64_t>(La, cus) : 1); ta++) {
+			const int64_t A = (La + ta - 1) / ta, tb0 = cus / ta;
+			if ((La + A - 1) / A != ta) continue;
+			// As few tiles along a layer as fit cost no more than twice the rows.
+			for (int64_t tb = std::max<int64_t>(1, tb0 / 2); tb <= tb0; tb++) {
+				const int64_t B = (L + tb - 1) / tb;
+				if ((L + B - 1) / B != tb || ta * tb < 2) continue;
+				const int64_t low = std::min(La - (ta - 1) * A, A), narrow = L - (tb - 1) * B;
+				double steps = 0;                     // of a phase, without the exchange
+				for (int64_t k = 0; k <= 16; k++) {   // 0: the wide kernel
+					const int64_t q = k ? k : 1;
+					if (low < q * hq || narrow < q * ds) break;
+					if (k == 0 && (low < 2 * hq || narrow < 2 * ds)) continue;
+					auto rows = [&](int64_t i) { return (A + 2 * i * hq) * (B + 2 * i * ds); };
+					if (rows(q) > (k ? window : wide_window)) break;
+					if (rows(q - 1) > T * (k ? many : wide)) {
+						if (k) break;
+						continue;
+					}
+					const double bytes = (double)(ta * tb) * (real ? 32 : 64) *
+					                     ((double)(rows(q) - rows(0)) + (double)(rows(q - 1) - rows(0)));
+					double us;
+					if (k) {
+						const int64_t most = std::max(rows(q) - rows(q - 1), rows(q - 1) - rows(0));
+						steps += 0.5 + set * (double)rows(q - 1) / T;
+						us = (1.3 * (double)((most + T - 1) / T) + bytes / 8e6 + steps) / (double)k;
+					} else {
+						us = 1.5 + bytes / 8e6 + set * (double)((rows(0) + T - 1) / T);
+					}
+					if (us < limit) {
+						limit = us;
+						best.C = (int)std::min<int64_t>(A * B, N - 1);
+						best.k = (int)q;
+						best.G = (int)(ta * tb);
+						best.L = (int)L;
+						best.hq = (int)hq;
+						best.ds = (int)ds;
+						best.A = (int)A;
+						best.B = (int)B;
+						best.wide = k == 0;
+						best.us = us;
+					}
+				}
 			}
 		}
+	};
+	if (h->tile_L) tiles(h->tile_L, 1, h->tile_ds);
+	if (h->band < N) tiles(N, 0, h->band);
 	return best;
+}
+
+// The plan is made once per model and form.
+ResidentPlan resident_plan(tbtkx_context *h, int cus) {
+	const PlainForm f = plain_form(h);
+	const int64_t key[8] = {h->csr_gen, h->N, h->Z, h->slot_half + 16 * (int64_t)h->tile_L, h->band,
+	                        f.slot + 2 * f.pal + 4 * (h->real_path && h->h_real),
+	                        (int64_t)h->use_resident + 2 * h->use_graph + 4 * h->slot_rows +
+	                            64 * h->use_patterns,
+	                        cus};
+	if (memcmp(key, h->res_plan_key, sizeof key) != 0) {
+		h->res_plan = make_plan(h, f, cus);
+		memcpy(h->res_plan_key, key, sizeof key);
+	}
+	return h->res_plan;
 }
 
 int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *from,
@@ -570,7 +939,7 @@ int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const in
 
 int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up) {
 	*given_up = false;
-	if (plan.C >= h->N) return TBTKX_OK;
+	if (plan.G <= 1) return TBTKX_OK;
 	uint32_t err = 0;
 	TBTKX_CHECK_HIP(hipMemcpyAsync(&err, h->res_err.ptr, 4, hipMemcpyDeviceToHost, h->stream));
 	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));

@@ -159,3 +159,53 @@ def test_nan_and_infinite_entries(res):
             b = res.moments(n // 2, [n // 2, n // 2 + 60], 40)
             res.set_option(X.OPT_RESIDENT, 1)
             assert np.array_equal(a, b, equal_nan=True)
+
+
+def cylinder(la, lb, orb, seed):
+    """A square lattice that wraps within its layers of lb cells, with a
+    diagonal bond, of `orb` states per cell: bonds beyond the layer's end."""
+    rng = np.random.default_rng(seed)
+    a, b, o = (x.ravel() for x in np.meshgrid(np.arange(la), np.arange(lb), np.arange(orb),
+                                              indexing="ij"))
+    here = (a * lb + b) * orb + o
+    r, c, v = [here], [here], [rng.uniform(-1, 1, here.size).astype(np.complex128)]
+    for da, db, t in ((0, 1, -1.0), (1, 0, -0.75), (1, 1, 0.25)):
+        ok = a + da < la
+        there = ((a + da) * lb + (b + db) % lb) * orb + o
+        r += [here[ok], there[ok]]
+        c += [there[ok], here[ok]]
+        v += [np.full(ok.sum(), t, dtype=np.complex128)] * 2
+    n = la * lb * orb
+    return L.coo_to_csr(np.concatenate(r), np.concatenate(c), np.concatenate(v), n)
+
+
+@pytest.mark.parametrize("real", [1, 0], ids=["real", "complex"])
+@pytest.mark.parametrize("name,n,ran", [
+    ("square_spin", (173, 61), 1), ("square_spin", (40, 701), 1), ("square_spin", (7, 3001), None),
+    ("square_spin", (611, 613), 1), ("nambu", (97, 101), 1), ("nambu", (257, 260), 1),
+    ("honeycomb", (40, 997), 1), ("honeycomb", (5, 2003), None), ("cubic", (31, 29, 37), 1),
+    ("cubic", (93, 89, 71), None), ("square", (1021, 1019), None), ("cylinder", (61, 83), None),
+    ("cylinder", (3, 5000), None), ("cylinder", (301, 700), None)])
+def test_tiles(res, oracle_mod, name, n, ran, real):
+    """Tiles of a lattice's layers, narrow and wide, with short last tiles and
+    bonds that wrap: bitwise the per-step kernels; targets across the tiles."""
+    f = {"square_spin": L.square_spin, "nambu": L.nambu_swave, "honeycomb": L.honeycomb_ribbon,
+         "cubic": L.cubic, "square": L.square}
+    csr = cylinder(*n, 2, seed=3) if name == "cylinder" else f[name](*n, disorder=0.5, seed=2).csr()
+    N = csr[0].size - 1
+    res.set_option(X.OPT_REAL, real)
+    to = sorted({0, 1, N - 1, N // 2, N // 3, *range(N // 2, min(N, N // 2 + 3000), 2)})
+    for M in (2, 3, 41):
+        got = check(res, oracle_mod, csr, 9.2, N // 2 + 1, to, M, oracle=N < 100000 and M == 41)
+        assert ran is None or not real or got == ran
+
+
+def test_tiles_without_palette(res, oracle_mod):
+    """Distinct values: the narrow tiles, or a launch per step where only the
+    wide ones would fit."""
+    m = L.square(300, 211, disorder=0.5, seed=3, flux=0.013)
+    to = [0, 30000, 30001, 63299]
+    assert check(res, oracle_mod, m.csr(), 5.0, 30000, to, 60) == 1
+    csr = cylinder(211, 190, 1, seed=4)
+    res.set_option(X.OPT_PALETTE, 0)
+    assert check(res, oracle_mod, csr, 5.0, 9, [0, 9, 189, 190, 40089], 60) == 1
