@@ -1610,6 +1610,24 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 	// Unit start vectors on a real H: two real vectors per complex column.
 	const int packed = mode == 0 && h->real_path && h->h_real;
 	const int per = packed ? 2 : 1, cols = (total + per - 1) / per;
+	if (h->use_resident && h->real_path && h->h_real && narrow_fits(h, flags, 1)) {
+		const int real_cols = mode == 0 ? total : 2 * total;
+		const int64_t zero = 0;
+		BlockCall c{1, h->ell_col.as<uint32_t>(), h->ell_v2f.as<double>(), &h->N, &zero, &h->band,
+		            &h->ell_W, h->csr_gen, true, &real_cols, mode == 0 ? sites : nullptr, mode != 0,
+		            seed, &M, (flags & TBTKX_DOUBLING) != 0};
+		bool done = false;
+		mu.resize((size_t)total * M);
+		if ((rc = resident_block(h, c, reinterpret_cast<double *>(mu.data()), &done))) return rc;
+		if (done) {
+			h->last_block_width = 64;
+			h->last_strip = -1;
+			h->last_share = h->last_rmul = 1;
+			h->last_real = packed;
+			return TBTKX_OK;
+		}
+		mu.clear();
+	}
 	const int rest = cols % 128;
 	const int parts = rest > 64 ? 2 : 1, w = (rest + parts - 1) / parts;
 	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w))

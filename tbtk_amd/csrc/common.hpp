@@ -181,6 +181,14 @@ struct tbtkx_context {
 	int64_t res_plan_key[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
 	int last_resident = 0;   // the last plain call ran resident
 	int num_cus = 0;
+	// What the resident blocks need of the single model and of the batch: the
+	// scan's results and the palettes on the device.
+	struct BlockForms {
+		int64_t gen = -1;
+		std::vector<int> ne, layer, reach;   // per model; ne 0: not for this path
+		tbtkx::DevBuf scan;
+	} rb_single, rb_multi;
+	tbtkx::DevBuf rb_sites, rb_part, rb_D;
 
 	// Lookup table L[n*E + e], complex double.
 	tbtkx::DevBuf lut;
@@ -338,6 +346,10 @@ int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const in
 // Whether the last launch gave up a wait (its moments are then incomplete);
 // waits for the stream.
 int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up);
+// The tagged exchange's buffer for that many bytes and unused tags from
+// res_epoch on; and whether a launch since gave up a wait (waits for the stream).
+int exchange_buffer(tbtkx_context *h, size_t bytes, uint32_t phases);
+int exchange_given_up(tbtkx_context *h, bool *given_up);
 
 // Up to 64 columns of the single model through the uneven batch's step kernel
 // (multi.hip), which stores and moves just these columns where a block is at
@@ -346,6 +358,34 @@ int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up
 bool narrow_fits(const tbtkx_context *h, int flags, int cols);
 int narrow_moments(tbtkx_context *h, int total, const int64_t *sites, bool phases, uint64_t seed,
                    int64_t col0, int M, int flags, int packed, double *out);
+
+// The lattice view of a model with the column offsets seen (offset + 32768):
+// layers of L rows such that every offset is q L + s with |q| <= 1 and |s| <=
+// ds, ds as small as it goes. L divides N and lies within 64 of the largest
+// offset, which is a lattice's slowest stride plus a few orbitals or rows.
+void layer_stride(int64_t N, const std::vector<uint8_t> &seen, int *layer, int *reach);
+
+// FP32 blocks of a real H resident on the chip (resident_block.hip). A call's
+// models: K of them in ELL form (FP64 values), cols real columns each, M moments;
+// unit vectors at `sites` (all models' in order) or, for one model, the real and
+// imaginary parts of random-phase vectors. out: per column (per vector with
+// phases) M moments. *done is false when the call is not for this path.
+struct BlockCall {
+	int K;
+	const uint32_t *ecol;
+	const double *ev2;
+	const int64_t *N, *e0, *band;
+	const int *W;
+	int64_t gen;
+	bool single;         // the handle's single model, else the batch
+	const int *cols;
+	const int64_t *sites;
+	bool phases;
+	uint64_t seed;
+	const int *M;
+	bool doubling;
+};
+int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done);
 
 // Random phase exp(2 pi i u), u the 53-bit splitmix64 uniform of (seed, c).
 __device__ __forceinline__ double2 random_phase(uint64_t seed, uint64_t c) {

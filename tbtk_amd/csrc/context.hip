@@ -202,7 +202,8 @@ int tbtkx_destroy(tbtkx_handle h) {
 	                  &h->res_in, &h->res_xg, &h->res_err,
 	                  &h->lut, &h->gf_in, &h->gf_out, &h->dfac, &h->dden, &h->blk_x, &h->blk_y,
 	                  &h->blk_mu, &h->blk_sites, &h->blk_part, &h->blk_grow, &h->blk_gvec, &h->cplanes,
-	                  &h->lplanes, &h->gf_mfma_out, &h->ell_col, &h->ell_v1f,
+	                  &h->lplanes, &h->gf_mfma_out, &h->rb_single.scan, &h->rb_multi.scan,
+	                  &h->rb_sites, &h->rb_part, &h->rb_D, &h->ell_col, &h->ell_v1f,
 	                  &h->ell_v2f, &h->ell_v1d, &h->ell_v2d,
 	                  &h->mm_ecol, &h->mm_ev1, &h->mm_ev2, &h->mm_desc, &h->mm_tab,
 	                  &h->mm_x, &h->mm_y, &h->mm_part, &h->mm_seg, &h->mm_D,

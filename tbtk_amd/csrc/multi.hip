@@ -1469,6 +1469,20 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 		TBTKX_REQUIRE(h->mm_N[m] * (width + 1) * 8 < ((int64_t)1 << 32), TBTKX_ERR_ARG,
 		              tag + "rows x (columns + 1) x 8 B must stay below 4 GiB");
 	}
+	if (packed && h->use_resident && h->autotune && !h->use_graph && h->tile_rows == 0 &&
+	    h->grid_share == 0) {
+		int rc = set_device(h);
+		if (rc) return rc;
+		BlockCall c{K, h->mm_ecol.as<uint32_t>(), h->mm_ev2.as<double>(), h->mm_N.data(),
+		            h->mm_e0.data(), h->mm_band.data(), h->mm_Wm.data(), h->mm_gen, false, num_sites,
+		            sites, false, 0, num_moments, (flags & TBTKX_DOUBLING) != 0};
+		bool done = false;
+		if ((rc = resident_block(h, c, out, &done))) return rc;
+		if (done) {
+			h->last_real = packed;
+			return TBTKX_OK;
+		}
+	}
 	return run_batch(h, num_sites, sites, num_moments, (flags & TBTKX_DOUBLING) != 0, packed, Start{},
 	                 out);
 }

@@ -631,25 +631,21 @@ static int make_slot_arrays(tbtkx_context *h, bool codes, bool values) {
 	return TBTKX_OK;
 }
 
-// The lattice view of a model with the column offsets seen (offset + 32768):
-// layers of L rows such that every offset is q L + s with |q| <= 1 and |s| <=
-// ds, ds as small as it goes. L divides N and lies within 64 of the largest
-// offset, which is a lattice's slowest stride plus a few orbitals or rows.
-static void layer_stride(tbtkx_context *h, const std::vector<uint8_t> &seen) {
-	h->tile_L = h->tile_ds = 0;
+void layer_stride(int64_t N, const std::vector<uint8_t> &seen, int *layer, int *reach) {
+	*layer = *reach = 0;
 	std::vector<int> offs;
 	for (int o = 1; o < 32768; o++)
 		if (seen[32768 + o] || seen[32768 - o]) offs.push_back(o);
 	if (offs.size() < 2 || offs.size() > 64) return;
 	int best = offs.back() / 2;
 	for (int L = std::max(2, offs.back() - 64); L <= offs.back() + 64; L++) {
-		if (h->N % L) continue;
+		if (N % L) continue;
 		int ds = 1;
 		for (int o : offs) ds = std::max(ds, 2 * o > L ? std::abs(o - L) : o);
 		if (ds < best) {
 			best = ds;
-			h->tile_L = L;
-			h->tile_ds = ds;
+			*layer = L;
+			*reach = ds;
 		}
 	}
 }
@@ -679,7 +675,7 @@ int build_slots(tbtkx_context *h, const uint32_t *rowptr, const uint32_t *col) {
 	h->slot_W = maxrow < 4 ? 4 : (int)maxrow;
 	h->slot_half = half;
 	h->slot_ok = 1;
-	layer_stride(h, seen);
+	layer_stride(h->N, seen, &h->tile_L, &h->tile_ds);
 	const bool pal = h->palette_ok != 0;
 	int rc = make_slot_arrays(h, pal, !pal);
 	if (rc || !h->slot_ok) return rc;

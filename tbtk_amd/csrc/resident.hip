@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "tiles.hpp"
 
 namespace tbtkx {
 namespace {
@@ -89,19 +90,12 @@ template <> struct R64<double> {
 // with a 32-bit tag beside it, so both 8-byte halves say by themselves that
 // they have arrived. Stored and loaded at the device's coherence point (sc1);
 // the loads are volatile, as they are polled.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-constexpr int kCoherent = 16, kVolatile = (int)0x80000000;
 __device__ __forceinline__ void put(__amdgpu_buffer_rsrc_t b, uint32_t at, double v, uint32_t tag) {
 	const u32x4 w = {(uint32_t)__double2loint(v), tag, (uint32_t)__double2hiint(v), tag};
 	__builtin_amdgcn_raw_buffer_store_b128(w, b, at * 16u, 0, kCoherent | kVolatile);
 }
-__device__ __forceinline__ u32x4 get(__amdgpu_buffer_rsrc_t b, uint32_t at) {
-	return __builtin_amdgcn_raw_buffer_load_b128(b, at * 16u, 0, kCoherent | kVolatile);
-}
-
 constexpr int16_t kSlotPad = -32768;
 constexpr int kResThreads = 1024;
-constexpr long long kWaitTicks = 100000000ll;   // of the 100 MHz clock: one second
 
 template <typename S>
 struct ResArgs {
@@ -123,36 +117,6 @@ struct ResArgs {
 	uint32_t *err;
 };
 
-// A workgroup's tile: first layer and row of it, extents.
-struct Tile {
-	int a, b, h, w;
-};
-template <typename S>
-__device__ __forceinline__ Tile tile_of(const ResArgs<S> &a, int g) {
-	Tile t;
-	t.a = g / a.tb * a.A;
-	t.b = g % a.tb * a.B;
-	t.h = t.a + a.A < a.La ? a.A : a.La - t.a;
-	t.w = t.b + a.B < a.L ? a.B : a.L - t.b;
-	return t;
-}
-struct Cell {
-	int a, b;   // layer, row in it; may lie outside the grid
-};
-// d-th place of the frame of rectangle t that is fh layers and fw rows thick.
-__device__ __forceinline__ Cell frame_cell(const Tile &t, int d, int fh, int fw) {
-	const int band = fh * t.w;
-	if (d < 2 * band) {
-		const int q = d / t.w;
-		return Cell{t.a + (q < fh ? q : t.h - 2 * fh + q), t.b + d - q * t.w};
-	}
-	const int q = (d - 2 * band) / (2 * fw), o = d - 2 * band - q * 2 * fw;
-	return Cell{t.a + fh + q, t.b + (o < fw ? o : t.w - 2 * fw + o)};
-}
-__device__ __forceinline__ Tile grown(const Tile &t, int h, int w) {
-	return Tile{t.a - h, t.b - w, t.h + 2 * h, t.w + 2 * w};
-}
-__device__ __forceinline__ int area(const Tile &t) { return t.h * t.w; }
 // Entries q0 .. q1 - 1 of the ascending list `to` that lie in layers a .. a + h - 1
 // of the tile's span of rows.
 template <typename S>
@@ -190,7 +154,7 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 	const int vec = MULTI ? 0 : (int)blockIdx.x;
 	const int N = a.N, k = MULTI ? a.k : 1, L = MULTI ? a.L : N;
 	const int hq = MULTI ? a.hq : 0, ds = MULTI ? a.ds : 0;
-	const Tile tile = MULTI ? tile_of(a, g) : Tile{0, 0, 1, N};
+	const Tile tile = MULTI ? tile_of(a.L, a.La, a.A, a.B, a.tb, g) : Tile{0, 0, 1, N};
 	const Tile window = grown(tile, k * hq, k * ds);
 	const int win = area(window), own = area(tile), P = window.w;
 	// Rows within q rings of the tile.
@@ -508,7 +472,7 @@ __global__ __launch_bounds__(kResThreads) void resident_wide(ResArgs<S> a) {
 	__shared__ S pal[256];
 	__shared__ int stop;
 	const int t = threadIdx.x, N = a.N, L = a.L, hq = a.hq, ds = a.ds;
-	const Tile tile = tile_of(a, (int)blockIdx.x);
+	const Tile tile = tile_of(a.L, a.La, a.A, a.B, a.tb, (int)blockIdx.x);
 	const Tile window = grown(tile, hq, ds), inside = grown(tile, -hq, -ds);
 	const int win = area(window), own = area(tile), P = window.w;
 	const int frame = own - area(inside), ring = win - own;
@@ -758,6 +722,26 @@ int launch_res_h(tbtkx_context *h, const ResArgs<S> &a, unsigned grid, int r, bo
 	               : launch_res_r<S, H, 1, false>(h, a, grid, r);
 }
 
+}  // namespace
+
+// Tags are never used twice: a buffer starts all zero and the tags go on from
+// launch to launch.
+int exchange_buffer(tbtkx_context *h, size_t bytes, uint32_t phases) {
+	if (h->res_err.ptr && (bytes == 0 || (h->res_xg.ptr && h->res_xg.bytes >= bytes)) &&
+	    h->res_epoch <= 0xffffffffu - phases)
+		return TBTKX_OK;
+	int rc;
+	if ((rc = h->res_xg.reserve(std::max<size_t>(bytes, 64)))) return rc;
+	if ((rc = h->res_err.reserve(256))) return rc;
+	res_zero<<<1024, kThreads, 0, h->stream>>>(h->res_xg.as<uint32_t>(), (int64_t)(h->res_xg.bytes / 4));
+	res_zero<<<1, kThreads, 0, h->stream>>>(h->res_err.as<uint32_t>(), 64);
+	TBTKX_CHECK_HIP(hipGetLastError());
+	h->res_epoch = 1;
+	return TBTKX_OK;
+}
+
+namespace {
+
 template <typename S>
 int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *from,
             const int *toff, const int64_t *to, int M) {
@@ -799,18 +783,9 @@ int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *fr
 	a.toff = reinterpret_cast<const int *>(a.from + V + T);
 	a.coef = h->coef.as<double2>();
 	if (a.G > 1) {
-		// Tags are never used twice: a buffer starts all zero and the tags go on
-		// from launch to launch.
 		const size_t bytes = (size_t)h->N * sizeof(S) / 8 * (plan.wide ? 32 : 64);
 		const uint32_t phases = (uint32_t)(M / plan.k + 2);
-		if (!h->res_xg.ptr || h->res_xg.bytes < bytes || h->res_epoch > 0xffffffffu - phases) {
-			if ((rc = h->res_xg.reserve(bytes))) return rc;
-			if ((rc = h->res_err.reserve(256))) return rc;
-			res_zero<<<1024, kThreads, 0, h->stream>>>(h->res_xg.as<uint32_t>(),
-			                                           (int64_t)(h->res_xg.bytes / 4));
-			res_zero<<<1, kThreads, 0, h->stream>>>(h->res_err.as<uint32_t>(), 64);
-			h->res_epoch = 1;
-		}
+		if ((rc = exchange_buffer(h, bytes, phases))) return rc;
 		a.xg = h->res_xg.ptr;
 		a.xg_bytes = (uint32_t)bytes;
 		a.err = h->res_err.as<uint32_t>();
@@ -937,9 +912,8 @@ int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const in
 	                                 : run_res<Z2>(h, plan, V, from, toff, to, M);
 }
 
-int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up) {
+int exchange_given_up(tbtkx_context *h, bool *given_up) {
 	*given_up = false;
-	if (plan.G <= 1) return TBTKX_OK;
 	uint32_t err = 0;
 	TBTKX_CHECK_HIP(hipMemcpyAsync(&err, h->res_err.ptr, 4, hipMemcpyDeviceToHost, h->stream));
 	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
@@ -948,6 +922,11 @@ int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up
 	TBTKX_CHECK_HIP(hipGetLastError());
 	*given_up = true;
 	return TBTKX_OK;
+}
+
+int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up) {
+	*given_up = false;
+	return plan.G > 1 ? exchange_given_up(h, given_up) : TBTKX_OK;
 }
 
 }  // namespace tbtkx
