@@ -201,6 +201,7 @@ struct tbtkx_context {
 	double dfac_e0 = 0, dfac_de = 0, dfac_s = 0;
 	// Split-BF16 planes for the MFMA contraction.
 	tbtkx::DevBuf cplanes, lplanes, gf_mfma_out;
+	void *gf_stage = nullptr;   // pinned, two halves (tbtkx_contract_mfma)
 	int cplanes_K = 0, cplanes_M = 0;
 	int lplanes_valid = 0;   // the table planes match the current table
 

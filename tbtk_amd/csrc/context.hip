@@ -209,6 +209,7 @@ int tbtkx_destroy(tbtkx_handle h) {
 	                  &h->mm_x, &h->mm_y, &h->mm_part, &h->mm_seg, &h->mm_D,
 	                  &h->mm_cols})
 		b->release();
+	if (h->gf_stage) (void)hipHostFree(h->gf_stage);
 	if (h->ev_start) (void)hipEventDestroy(h->ev_start);
 	if (h->ev_stop) (void)hipEventDestroy(h->ev_stop);
 	if (h->stream) (void)hipStreamDestroy(h->stream);
