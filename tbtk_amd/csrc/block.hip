@@ -1620,6 +1620,9 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 		mu.resize((size_t)total * M);
 		if ((rc = resident_block(h, c, reinterpret_cast<double *>(mu.data()), &done))) return rc;
 		if (done) {
+			// Counted as steps of 64 columns, as the step kernels' launches.
+			h->last_launches =
+			    (int64_t)((cols + 63) / 64) * ((flags & TBTKX_DOUBLING) ? (M + 1) / 2 : M - 1);
 			h->last_block_width = 64;
 			h->last_strip = -1;
 			h->last_share = h->last_rmul = 1;

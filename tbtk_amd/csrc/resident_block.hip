@@ -577,6 +577,7 @@ int scan_models(tbtkx_context *h, const BlockCall &c, tbtkx_context::BlockForms 
 
 int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done) {
 	*done = false;
+	h->last_resident = 0;
 	int64_t vectors = 0;
 	std::vector<int> S(c.K);
 	for (int m = 0; m < c.K; m++) {
@@ -635,7 +636,7 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 		                               hipMemcpyHostToDevice, h->stream));
 	}
 	TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
-	int64_t site0 = 0, launches = 0;
+	int64_t site0 = 0;
 	for (int m = 0; m < c.K; m++) {
 		const Shape &s = sh[m];
 		RunArgs a{};
@@ -673,7 +674,6 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 			void *args[] = {&a};
 			TBTKX_CHECK_HIP(hipLaunchCooperativeKernel(k, dim3((unsigned)(teams * s.Gt)), dim3(kT), args, 0,
 			                                           h->stream));
-			launches++;
 			if (!c.doubling) continue;
 			const int64_t n = (int64_t)S[m] * teams * kDots;
 			block_dots<<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, h->stream>>>(
@@ -692,7 +692,8 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	float ms = 0;
 	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
 	h->last_ms = ms;
-	h->last_launches = launches;
+	h->last_launches = Smax;
+	h->last_resident = 1;
 	*done = true;
 	if (!c.doubling) {
 		memcpy(out, res.data(), res_bytes);
