@@ -745,6 +745,12 @@ def main():
         slot, patterns, uniform = form["slot"], form["patterns"], form["uniform"]
         byte_rows = form["byte_rows"]
         avg_kernel_s = kernel_ms * 1e-3 / launches
+        # All steps in one launch with the vectors on the chip: LDS bounds a step
+        # (per row 4 neighbours, 4 palette values and the row's own write).
+        resident = eng.get_option(X.OPT_RESIDENT) == 1
+        peak = 256 * 128 * 2.4 if resident else HBM_PEAK_GBPS
+        if resident:
+            step_bytes = 9 * (8 if real else 16) * N
         achieved = step_bytes / avg_kernel_s / 1e9
         dE = (WINDOW[1] - WINDOW[0]) / (E_PTS - 1)
         out.update({
@@ -770,7 +776,9 @@ def main():
             "physical_sites_per_s": value / 2,
             "spmv_GBps": achieved,
             "roofline": {
-                "kernel": ((("plain_step_slot<double> (real FP64 slot-major ELL SpMV "
+                "kernel": "resident_wide (all steps in one launch, vectors in LDS and "
+                          "registers; per-step figures)" if resident else
+                          ((("plain_step_slot<double> (real FP64 slot-major ELL SpMV "
                              "recurrence step, one thread per row; H is real)" if real else
                              "plain_step_slot<double2> (complex FP64 slot-major ELL SpMV "
                              "recurrence step)") if slot else
@@ -786,12 +794,12 @@ def main():
                               (("; 16-bit column offsets" if col16 else "; 32-bit columns")
                                + ("; 1-byte value codes (palette) + diagonal array"
                                   if palette else "")))),
-                "bound": "hbm",
+                "bound": "lds" if resident else "hbm",
                 "achieved": achieved,
-                "peak": HBM_PEAK_GBPS,
+                "peak": peak,
                 "unit": "GB/s",
-                "frac": achieved / HBM_PEAK_GBPS,
-                "traffic": load_traffic(("plain_step_slot" if slot else "plain_step_lds")
+                "frac": achieved / peak,
+                "traffic": None if resident else load_traffic(("plain_step_slot" if slot else "plain_step_lds")
                                         + ("_real" if real else "")
                                         + ("_col16" if col16 and not slot else "")
                                         + ("_palette" if palette else "")
