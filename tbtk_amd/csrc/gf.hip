@@ -109,7 +109,8 @@ struct Term {
 		else if constexpr (DIRECT) return t[at];
 		else return t[2 * at + (TYPE == TBTKX_PRINCIPAL ? 0 : 1)];
 	}
-	// The same of row `at / row bytes` through a buffer resource; 0 past its end.
+	// The same through a buffer resource. `row` is a scalar offset, which the
+	// resource's bounds check leaves out: it must lie inside the array.
 	static constexpr int kBytes = DIRECT && !kPair ? 8 : 16;   // of an array element
 	static constexpr int kPart = !DIRECT && TYPE == TBTKX_NONPRINCIPAL ? 8 : 0;
 	__device__ __forceinline__ static F load(__amdgpu_buffer_rsrc_t t, uint32_t lane, uint32_t row) {
@@ -190,15 +191,21 @@ __global__ __launch_bounds__(64) void contract_few(
 	const uint32_t rowb = (uint32_t)E * O::kBytes, off = (uint32_t)ec * O::kBytes;
 	for (int r0 = 0; r0 < rows; r0 += kFewChunk) {
 		const int n = rows - r0 < kFewChunk ? rows - r0 : kFewChunk;
-		// The chunk's rows (below 512 x 16384 x 16 B; rows past the end read 0): a
-		// row then takes one scalar add and one load, where a lone wavefront
-		// pays every instruction in full.
+		// The chunk's rows. A row takes a scalar add, a scalar minimum and one load,
+		// where a lone wavefront pays every instruction in full. Rows read ahead of
+		// the chunk's end repeat its last. Offsets stay in 32 bits: contract_launch
+		// comes here with at most 16 x 5 energies per CU (20,480), 16 B each, and r
+		// runs to 512 + 3 kAhead rows.
 		const __amdgpu_buffer_rsrc_t tab = __builtin_amdgcn_make_buffer_rsrc(
 		    const_cast<char *>(reinterpret_cast<const char *>(L)) + (int64_t)r0 * rowb, 0,
 		    (uint32_t)n * rowb, 0x00027000);
+		const uint32_t last = (uint32_t)(n - 1) * rowb;
 		auto load = [&](F (&f)[kAhead], int r) __attribute__((always_inline)) {
 #pragma unroll
-			for (int i = 0; i < kAhead; i++) f[i] = O::load(tab, off, (uint32_t)(r + i) * rowb);
+			for (int i = 0; i < kAhead; i++) {
+				const uint32_t row = (uint32_t)(r + i) * rowb;
+				f[i] = O::load(tab, off, row < last ? row : last);
+			}
 		};
 		F a[kAhead], b[kAhead];
 		load(a, 0);

@@ -29,3 +29,27 @@ def test_contraction_bitwise(engine, oracle_mod, K, M, E, gtype):
         assert np.array_equal(got[k], oracle_mod.gf_lookup(gtype, table, c[k])), k
         assert np.array_equal(direct[k], oracle_mod.gf_direct(gtype, c[k], lo, hi, E, s)), k
     engine.lut_destroy()
+
+
+@pytest.mark.parametrize("gtype", range(4))
+@pytest.mark.parametrize("K,M", [(1, 1), (2, 2), (1, 18), (2, 49), (1, 513), (1, 530)])
+def test_few_vectors_widest_rows(engine, oracle_mod, K, M, gtype):
+    """Few vectors at the most energies the few-vector kernel takes on 256 compute
+    units (16 x 5 x 256), where the rows it reads ahead of the last one would
+    lie farthest beyond the array: bitwise the oracle."""
+    E, s, lo, hi = 20480, 6.0, -5.7, 5.8
+    rng = np.random.default_rng(M)
+    c = rng.normal(size=(K, M)) + 1j * rng.normal(size=(K, M))
+    engine.lut_generate(M, E, lo, hi, s)
+    got = engine.contract(c, gtype)
+    direct = engine.contract_direct(c, gtype, E, lo, (hi - lo) / (E - 1), s)
+    table = oracle_mod.lookup_table(M, E, lo, hi, s)
+    engine.lut_upload(table)
+    uploaded = engine.contract(c, gtype)
+    engine.lut_destroy()
+    for k in range(K):
+        ref = oracle_mod.gf_lookup(gtype, table, c[k])
+        assert np.array_equal(uploaded[k], ref), k
+        assert np.array_equal(direct[k], oracle_mod.gf_direct(gtype, c[k], lo, hi, E, s)), k
+        # The generated table: a few ulp of acos, times n up to M, per term.
+        assert np.abs(got[k] - ref).max() <= 1e-13 * M * np.abs(ref).max()
