@@ -94,6 +94,13 @@ struct GraphCache {
 	}
 };
 
+// An autotuned launch shape of the uneven batch's step: tile groups and grid
+// share, of the model generation, mode and widths of `key`.
+struct TunedShape {
+	int64_t key[3] = {-1, -1, -1};
+	int g = 0, share = 0;
+};
+
 // The plain recurrence in one launch, the vectors resident on the chip
 // (resident.hip): C rows per workgroup (the whole model: one workgroup per start
 // vector), else G tiles of A layers x B rows with k steps between exchanges;
@@ -233,10 +240,9 @@ struct tbtkx_context {
 	std::vector<int64_t> mm_band;             // max |col - row| per model
 	tbtkx::DevBuf mm_ecol, mm_ev1, mm_ev2;
 	tbtkx::DevBuf mm_desc, mm_tab, mm_x, mm_y, mm_part, mm_seg, mm_D, mm_cols;
-	int64_t mm_tune_key[3] = {-1, -1, -1};    // (generation, flags, widths hash)
-	int mm_tune_g = 0, mm_tune_occ = 0;       // tuned tile groups, grid share
-	int64_t nb_tune_key[3] = {-1, -1, -1};    // the same of narrow blocks of the
-	int nb_tune_g = 0, nb_tune_occ = 0;       // single model (narrow_moments)
+	tbtkx::TunedShape mm_tuned;
+	std::map<int, tbtkx::TunedShape> nb_tuned;   // narrow blocks of the single
+	                                             // model, by class (narrow_class)
 	std::vector<tbtkx::GraphCache> mm_graphs;   // the run in bounded chunks
 	void reset_mm_graphs() {
 		for (tbtkx::GraphCache &g : mm_graphs) g.reset();

@@ -419,7 +419,8 @@ int tbtkx_set_option(tbtkx_handle h, int option, int64_t value) {
 		return TBTKX_OK;
 	case TBTKX_OPT_AUTOTUNE:
 		h->autotune = value != 0;
-		for (auto &k : h->mm_tune_key) k = -1;
+		h->mm_tuned = TunedShape{};
+		h->nb_tuned.clear();
 		return TBTKX_OK;
 	case TBTKX_OPT_MFMA_PIPE:
 		h->mfma_pipe = value != 0;

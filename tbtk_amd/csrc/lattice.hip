@@ -581,7 +581,7 @@ int tbtkx_multi_set_lattices(tbtkx_handle h, int K, const tbtkx_lattice *lats,
 	h->mm_real = real;
 	h->mm_realm = realm;
 	h->mm_gen++;
-	for (auto &k : h->mm_tune_key) k = -1;
+	h->mm_tuned = TunedShape{};
 	return TBTKX_OK;
 }
 

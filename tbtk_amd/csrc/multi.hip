@@ -1018,7 +1018,7 @@ int64_t run_steps(const Plan &p) {
 // (share 1 or 2) with tiles of 2-16 row groups, and one tile per wavefront
 // (share 0) with tiles of 8-64 row groups.
 int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<int> &S,
-             bool dots, int ncols, int64_t mu_elems) {
+             bool dots, int ncols, int64_t mu_elems, TunedShape &tuned) {
 	static const int kCand[][2] = {{1, 2}, {1, 4}, {1, 8}, {1, 16}, {2, 2},  {2, 4},
 	                               {2, 8}, {2, 16}, {0, 8}, {0, 16}, {0, 32}, {0, 64}};
 	constexpr int kTrial = 4;
@@ -1063,16 +1063,26 @@ int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<
 			}
 		}
 	}
-	h->mm_tune_g = bestG;
-	h->mm_tune_occ = bestShare;
+	tuned.g = bestG;
+	tuned.share = bestShare;
 	return TBTKX_OK;
+}
+
+// What the tuned shape of a narrow block depends on: the lanes of a row, which
+// set the rows of a row group, and whether a lane moves two columns; rows that
+// fill a group by themselves in two halves. The steps don't matter, and a class
+// per width would tune up to 64 times per model (about 12 x 5 steps each).
+int narrow_class(int w, int W) {
+	const int pairs = use_pairs(w, W) ? 1 : 0;
+	const int lanes = pairs ? (w + 1) / 2 : w;
+	return kMaxWidth / lanes * 4 + (lanes > 48 ? 2 : 0) + pairs;
 }
 
 // Moments of the batch (the mm_* model fields): num_sites[m] start vectors and
 // num_moments[m] moments of model m, doubling dots or gathers, packed real
-// vectors or complex columns.
+// vectors or complex columns. narrow: a single model's block (narrow_moments).
 int run_batch(tbtkx_context *h, const int *num_sites, const int64_t *sites, const int *num_moments,
-              bool dots, int packed, const Start &start, double *out) {
+              bool dots, int packed, const Start &start, bool narrow, double *out) {
 	const int K = h->mm_K;
 	h->mm_packed = packed;
 	std::vector<int> width(K), S(K);
@@ -1091,25 +1101,28 @@ int run_batch(tbtkx_context *h, const int *num_sites, const int64_t *sites, cons
 	// Launch shape: explicit (TBTKX_OPT_TILE_ROWS = row groups per tile, with
 	// TBTKX_OPT_GRID_SHARE: 0 = one tile per wavefront, s > 0 = persistent
 	// grid of occupancy x CUs / s workgroups) or autotuned once per (batch,
-	// mode, widths).
+	// mode, widths), narrow blocks once per class.
 	int64_t hw = 1469598103934665603ll;
 	for (int m = 0; m < K; m++) hw = (hw ^ (width[m] * 131 + S[m])) * 1099511628211ll;
-	const int64_t key[3] = {h->mm_gen, (int)dots + (packed << 16), hw};
+	const int mode = (int)dots + 2 * packed;
+	const int cls = narrow ? narrow_class(width[0], h->mm_W) : 0;
+	TunedShape &tuned = narrow ? h->nb_tuned[cls * 4 + mode] : h->mm_tuned;
+	const int64_t key[3] = {h->mm_gen, mode, narrow ? cls : hw};
 	int G = 8, share = 1;
 	if (h->tile_rows > 0) {
 		G = std::max(kRpi, (h->tile_rows + kRpi - 1) / kRpi * kRpi);
 		share = h->grid_share;
 	} else if (h->autotune && Smax > 0) {
-		if (memcmp(key, h->mm_tune_key, sizeof key) != 0) {
+		if (memcmp(key, tuned.key, sizeof key) != 0) {
 			// Output sizes are needed to reserve buffers for the trial runs.
 			int64_t mu_elems = 0;
 			for (int m = 0; m < K; m++)
 				mu_elems += dots ? (int64_t)S[m] * 2 * width[m] : out_off[m + 1] - out_off[m];
-			if ((rc = autotune(h, width, S, dots, ncols, mu_elems))) return rc;
-			memcpy(h->mm_tune_key, key, sizeof key);
+			if ((rc = autotune(h, width, S, dots, ncols, mu_elems, tuned))) return rc;
+			memcpy(tuned.key, key, sizeof key);
 		}
-		G = h->mm_tune_g;
-		share = h->mm_tune_occ;
+		G = tuned.g;
+		share = tuned.share;
 	}
 	h->last_share = share;
 	h->last_tile_groups = G;
@@ -1275,9 +1288,6 @@ struct SingleModel {
 		std::swap(h->mm_ecol, h->ell_col);
 		std::swap(h->mm_ev1, h->ell_v1f);
 		std::swap(h->mm_ev2, h->ell_v2f);
-		std::swap(h->mm_tune_key, h->nb_tune_key);
-		std::swap(h->mm_tune_g, h->nb_tune_g);
-		std::swap(h->mm_tune_occ, h->nb_tune_occ);
 	}
 };
 
@@ -1300,7 +1310,7 @@ int narrow_moments(tbtkx_context *h, int total, const int64_t *sites, bool phase
 		start.phases = phases;
 		start.seed = seed;
 		start.col0 = col0;
-		rc = run_batch(h, &total, sites, &M, (flags & TBTKX_DOUBLING) != 0, packed, start, out);
+		rc = run_batch(h, &total, sites, &M, (flags & TBTKX_DOUBLING) != 0, packed, start, true, out);
 	}
 	return rc;
 }
@@ -1437,7 +1447,7 @@ int tbtkx_multi_set(tbtkx_handle h, int K, const int64_t *num_rows,
 	h->mm_real = real;
 	h->mm_realm = realm;
 	h->mm_gen++;
-	for (auto &k : h->mm_tune_key) k = -1;
+	h->mm_tuned = TunedShape{};
 	return TBTKX_OK;
 }
 
@@ -1484,7 +1494,7 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 		}
 	}
 	return run_batch(h, num_sites, sites, num_moments, (flags & TBTKX_DOUBLING) != 0, packed, Start{},
-	                 out);
+	                 false, out);
 }
 
 }  // extern "C"
