@@ -188,6 +188,7 @@ struct tbtkx_context {
 	int64_t res_plan_key[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
 	int last_resident = 0;   // the last plain call ran resident
 	int num_cus = 0;
+	int cooperative = 0;     // cooperative launches supported and none refused yet
 	// What the resident blocks need of the single model and of the batch: the
 	// scan's results and the palettes on the device.
 	struct BlockForms {
@@ -343,18 +344,35 @@ inline PlainForm plain_form(const tbtkx_context *h) {
 	return f;
 }
 
+// Internal status: the resident path can't run now (a cooperative launch was
+// refused, or there is no memory for its scratch); the step kernels run instead.
+constexpr int kDeclined = -1;
+
+// Launches a resident kernel whose workgroups wait for each other; kDeclined, and
+// no further tries on this handle, when the runtime refuses it (fewer usable CUs
+// than the device reports).
+inline int launch_cooperative(tbtkx_context *h, const void *kernel, unsigned grid,
+                              unsigned threads, void **args) {
+	if (hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(threads), args, 0, h->stream) ==
+	    hipSuccess)
+		return TBTKX_OK;
+	(void)hipGetLastError();
+	h->cooperative = 0;
+	return kDeclined;
+}
+
 // The resident recurrence of this model and form (made once per model).
 ResidentPlan resident_plan(tbtkx_context *h, int cus);
 // Enqueues the moments of V start vectors (V = 1 unless plan.C covers the
 // model) into h->coef, one row of M per entry of `to`; vector v's entries are
-// toff[v] .. toff[v + 1], ascending.
+// toff[v] .. toff[v + 1], ascending. kDeclined: nothing was launched.
 int resident_moments(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *from,
                      const int *toff, const int64_t *to, int M);
 // Whether the last launch gave up a wait (its moments are then incomplete);
 // waits for the stream.
 int resident_given_up(tbtkx_context *h, const ResidentPlan &plan, bool *given_up);
 // The tagged exchange's buffer for that many bytes and unused tags from
-// res_epoch on; and whether a launch since gave up a wait (waits for the stream).
+// res_epoch on (kDeclined: no memory); and whether a launch since gave up a wait (waits for the stream).
 int exchange_buffer(tbtkx_context *h, size_t bytes, uint32_t phases);
 int exchange_given_up(tbtkx_context *h, bool *given_up);
 

@@ -177,6 +177,8 @@ int tbtkx_create(int device, tbtkx_handle *handle) {
 	if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
 	if (e == hipSuccess)
 		e = hipDeviceGetAttribute(&h->num_cus, hipDeviceAttributeMultiprocessorCount, device);
+	if (e == hipSuccess)
+		e = hipDeviceGetAttribute(&h->cooperative, hipDeviceAttributeCooperativeLaunch, device);
 	if (e == hipSuccess) e = hipEventCreate(&h->ev_start);
 	if (e == hipSuccess) e = hipEventCreate(&h->ev_stop);
 	if (e != hipSuccess) {

@@ -1127,7 +1127,11 @@ extern "C" int tbtkx_moments(tbtkx_handle h, int64_t from, int K,
 	if (resident) {
 		const int toff[2] = {0, U};
 		TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));
-		if ((rc = resident_moments(h, plan, 1, &from, toff, uniq.data(), M))) return rc;
+		rc = resident_moments(h, plan, 1, &from, toff, uniq.data(), M);
+		if (rc && rc != kDeclined) return rc;
+		resident = rc == TBTKX_OK;
+	}
+	if (resident) {
 		TBTKX_CHECK_HIP(hipEventRecord(h->ev_stop, h->stream));
 		TBTKX_CHECK_HIP(hipMemcpyAsync(dense.data(), h->coef.ptr, dense.size() * 8,
 		                               hipMemcpyDeviceToHost, h->stream));

@@ -665,13 +665,12 @@ int launch_res(tbtkx_context *h, ResArgs<S> a, unsigned grid) {
 	if constexpr (!MULTI) {
 		resident_recurrence<S, H, R, MULTI><<<grid, kResThreads, 0, h->stream>>>(a);
 		TBTKX_CHECK_HIP(hipGetLastError());
+		return TBTKX_OK;
 	} else {
 		void *p[] = {&a};
-		TBTKX_CHECK_HIP(hipLaunchCooperativeKernel(
-		    (const void *)resident_recurrence<S, H, R, MULTI>, dim3(grid), dim3(kResThreads), p, 0,
-		    h->stream));
+		return launch_cooperative(h, (const void *)resident_recurrence<S, H, R, MULTI>, grid,
+		                          kResThreads, p);
 	}
-	return TBTKX_OK;
 }
 
 // Most rows per thread: what 128 VGPRs hold (16 wavefronts per CU) without
@@ -707,9 +706,7 @@ int launch_wide(tbtkx_context *h, ResArgs<S> a, unsigned grid, int r) {
 	if constexpr (R <= wide_rows<S>(H)) {
 		if (r > R) return launch_wide<S, H, R + 1>(h, a, grid, r);
 		void *p[] = {&a};
-		TBTKX_CHECK_HIP(hipLaunchCooperativeKernel((const void *)resident_wide<S, H, R>, dim3(grid),
-		                                           dim3(kResThreads), p, 0, h->stream));
-		return TBTKX_OK;
+		return launch_cooperative(h, (const void *)resident_wide<S, H, R>, grid, kResThreads, p);
 	}
 	set_error("resident recurrence: too many rows per thread");
 	return TBTKX_ERR_STATE;
@@ -731,8 +728,10 @@ int exchange_buffer(tbtkx_context *h, size_t bytes, uint32_t phases) {
 	    h->res_epoch <= 0xffffffffu - phases)
 		return TBTKX_OK;
 	int rc;
-	if ((rc = h->res_xg.reserve(std::max<size_t>(bytes, 64)))) return rc;
-	if ((rc = h->res_err.reserve(256))) return rc;
+	if ((rc = h->res_xg.reserve(std::max<size_t>(bytes, 64))) || (rc = h->res_err.reserve(256))) {
+		(void)hipGetLastError();
+		return rc == TBTKX_ERR_OOM ? kDeclined : rc;
+	}
 	res_zero<<<1024, kThreads, 0, h->stream>>>(h->res_xg.as<uint32_t>(), (int64_t)(h->res_xg.bytes / 4));
 	res_zero<<<1, kThreads, 0, h->stream>>>(h->res_err.as<uint32_t>(), 64);
 	TBTKX_CHECK_HIP(hipGetLastError());
@@ -835,6 +834,7 @@ static ResidentPlan make_plan(const tbtkx_context *h, const PlainForm &f, int cu
 		best.us = base + set * (double)((N + T - 1) / T);
 		return best;
 	}
+	if (!h->cooperative) return best;
 	double limit = std::max(2.7, f.bytes / 5.5e6);
 	// Tiles of every form that fits and has no more of them than CUs.
 	auto tiles = [&](int64_t L, int64_t hq, int64_t ds) {
@@ -898,7 +898,7 @@ ResidentPlan resident_plan(tbtkx_context *h, int cus) {
 	                        f.slot + 2 * f.pal + 4 * (h->real_path && h->h_real),
 	                        (int64_t)h->use_resident + 2 * h->use_graph + 4 * h->slot_rows +
 	                            64 * h->use_patterns,
-	                        cus};
+	                        cus * 2 + (h->cooperative != 0)};
 	if (memcmp(key, h->res_plan_key, sizeof key) != 0) {
 		h->res_plan = make_plan(h, f, cus);
 		memcpy(h->res_plan_key, key, sizeof key);

@@ -586,8 +586,15 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 		vectors += c.cols[m];
 	}
 	int rc;
+	if (!h->cooperative) return TBTKX_OK;
+	// No memory for this path's own scratch: the step kernels need what it holds.
+	auto no_memory = [&]() {
+		(void)hipGetLastError();
+		for (tbtkx::DevBuf *b : {&h->res_xg, &h->rb_part, &h->rb_D}) b->release();
+		return TBTKX_OK;
+	};
 	tbtkx_context::BlockForms &f = c.single ? h->rb_single : h->rb_multi;
-	if ((rc = scan_models(h, c, f))) return rc;
+	if ((rc = scan_models(h, c, f))) return rc == TBTKX_ERR_OOM ? no_memory() : rc;
 	// Against the streamed step: 12 bytes per column element at 4.4 TB/s (1,048,576
 	// states x 256 columns: 732 us, measured 711), at least 5 us per launch; models of a
 	// batch share its launches. Wide rings lose: 864,000 states (96 x 100 x 90), 64
@@ -626,12 +633,13 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	// Long calls keep to the step kernels rather than to gigabytes of scratch.
 	if (part > ((size_t)1 << 30) || xg >= ((size_t)1 << 32) - 64 || phases > (1u << 30))
 		return TBTKX_OK;
-	if ((rc = exchange_buffer(h, xg, phases))) return rc;
-	if (c.doubling && (rc = h->rb_part.reserve(part))) return rc;
+	if ((rc = exchange_buffer(h, xg, phases))) return rc == kDeclined ? no_memory() : rc;
 	const size_t res_bytes = c.doubling ? D * 8 : mu * 16;
-	if ((rc = h->rb_D.reserve(res_bytes))) return rc;
+	if ((c.doubling && (rc = h->rb_part.reserve(part))) || (rc = h->rb_D.reserve(res_bytes)))
+		return rc == TBTKX_ERR_OOM ? no_memory() : rc;
 	if (c.sites) {
-		if ((rc = h->rb_sites.reserve((size_t)vectors * 8))) return rc;
+		if ((rc = h->rb_sites.reserve((size_t)vectors * 8)))
+			return rc == TBTKX_ERR_OOM ? no_memory() : rc;
 		TBTKX_CHECK_HIP(hipMemcpyAsync(h->rb_sites.ptr, c.sites, (size_t)vectors * 8,
 		                               hipMemcpyHostToDevice, h->stream));
 	}
@@ -672,8 +680,7 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 			a.epoch = h->res_epoch;
 			h->res_epoch += (uint32_t)(S[m] + 2);
 			void *args[] = {&a};
-			TBTKX_CHECK_HIP(hipLaunchCooperativeKernel(k, dim3((unsigned)(teams * s.Gt)), dim3(kT), args, 0,
-			                                           h->stream));
+			if (launch_cooperative(h, k, (unsigned)(teams * s.Gt), kT, args)) return TBTKX_OK;
 			if (!c.doubling) continue;
 			const int64_t n = (int64_t)S[m] * teams * kDots;
 			block_dots<<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, h->stream>>>(

@@ -1,0 +1,69 @@
+"""Where a resident recurrence can't run, the step kernels run instead, with their
+results: a cooperative launch that the runtime refuses, no memory for the
+scratch that only the resident path needs, and a wait given up on the device.
+Each is brought about on the host by a shim between the library and the runtime.
+"""
+import pytest
+
+from shim import run_shimmed
+
+pytestmark = pytest.mark.gpu
+
+CALLS = """
+def plain(f, n, s):
+    m = f(*n, disorder=0.5, seed=2)
+    N = m.basis_size
+    eng.set_csr(m.csr(), s)
+    return lambda: eng.moments(N // 2, [0, N // 2, N // 2 + 1, N - 1], 60)
+
+def block(flags):
+    m = L.honeycomb_ribbon(40, 997, disorder=0.5, seed=4)
+    sites = np.random.default_rng(3).integers(0, m.basis_size, 37)
+    eng.set_csr(m.csr(), 9.2)
+    return lambda: eng.moments_block(sites, 80, flags)
+
+def trace():
+    eng.set_csr(L.square(300, 301, disorder=0.5, seed=4).csr(), 5.0)
+    return lambda: eng.moments_trace(33, 11, 80)
+
+def batch():
+    specs = [L.square_spec(200, 211, disorder=0.5, seed=1), L.square_spec(170, 201, disorder=0.5, seed=2)]
+    eng.multi_set_lattices(specs, [5.0, 5.0])
+    return lambda: np.concatenate([x.ravel() for x in eng.multi_moments(
+        [np.arange(64), np.arange(40)], [120, 90], X.DOUBLING)])
+
+CASES = [("tiles", lambda: plain(L.square_spin, (173, 61), 6.0)),
+         ("wide tiles", lambda: plain(L.square_spin, (611, 613), 6.0)),
+         ("gathered block", lambda: block(0)), ("doubled block", lambda: block(X.DOUBLING)),
+         ("trace", trace), ("batch", batch)]
+"""
+
+BODY = CALLS + """
+trouble, how = value("{name}"), {how}
+for name, make in CASES:
+    eng = X.Engine(0)
+    call = make()
+    eng.set_option(X.OPT_RESIDENT, 0)
+    ref = call()
+    eng.set_option(X.OPT_RESIDENT, 1)
+    trouble.value = how
+    print(name, flush=True)
+    got = call()
+    trouble.value = 0
+    assert eng.get_option(X.OPT_RESIDENT) == 0, name
+    assert np.array_equal(got, ref), name
+    if {settled}:
+        value("shim_cooperative").value = 0
+        assert np.array_equal(call(), ref), name
+        assert value("shim_cooperative").value == 0, name
+    else:
+        call()
+        assert eng.get_option(X.OPT_RESIDENT) == 1, name
+"""
+
+
+@pytest.mark.parametrize("name,how,settled", [
+    ("shim_refuse", 1, True), ("shim_malloc_limit", 100000, False), ("shim_give_up", 1, False)])
+def test_step_kernels_take_over(tmp_path, name, how, settled):
+    """A refused launch is not tried again on the handle; memory and waits are."""
+    run_shimmed(tmp_path, BODY.format(name=name, how=how, settled=settled))
