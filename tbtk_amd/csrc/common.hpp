@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -188,7 +189,8 @@ struct tbtkx_context {
 	int64_t res_plan_key[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
 	int last_resident = 0;   // the last plain call ran resident
 	int num_cus = 0;
-	int cooperative = 0;     // cooperative launches supported and none refused yet
+	int cooperative = 0;     // the device has cooperative launches
+	std::chrono::steady_clock::time_point cooperative_again;   // not before this time
 	// What the resident blocks need of the single model and of the batch: the
 	// scan's results and the palettes on the device.
 	struct BlockForms {
@@ -348,16 +350,22 @@ inline PlainForm plain_form(const tbtkx_context *h) {
 // refused, or there is no memory for its scratch); the step kernels run instead.
 constexpr int kDeclined = -1;
 
-// Launches a resident kernel whose workgroups wait for each other; kDeclined, and
-// no further tries on this handle, when the runtime refuses it (fewer usable CUs
-// than the device reports).
+// Cooperative launches work now, as far as is known. The runtime refuses them
+// while another process has used them on the same GPU, and with fewer usable CUs than
+// the device reports. A refused try takes 80 ms, so the handle waits 10 s for the
+// next.
+inline bool cooperative_now(const tbtkx_context *h) {
+	return h->cooperative && std::chrono::steady_clock::now() >= h->cooperative_again;
+}
+// Launches a resident kernel whose workgroups wait for each other; kDeclined when
+// the runtime refuses it.
 inline int launch_cooperative(tbtkx_context *h, const void *kernel, unsigned grid,
                               unsigned threads, void **args) {
 	if (hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(threads), args, 0, h->stream) ==
 	    hipSuccess)
 		return TBTKX_OK;
 	(void)hipGetLastError();
-	h->cooperative = 0;
+	h->cooperative_again = std::chrono::steady_clock::now() + std::chrono::seconds(10);
 	return kDeclined;
 }
 

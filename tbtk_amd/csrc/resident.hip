@@ -834,7 +834,7 @@ static ResidentPlan make_plan(const tbtkx_context *h, const PlainForm &f, int cu
 		best.us = base + set * (double)((N + T - 1) / T);
 		return best;
 	}
-	if (!h->cooperative) return best;
+	if (!cooperative_now(h)) return best;
 	double limit = std::max(2.7, f.bytes / 5.5e6);
 	// Tiles of every form that fits and has no more of them than CUs.
 	auto tiles = [&](int64_t L, int64_t hq, int64_t ds) {
@@ -898,7 +898,7 @@ ResidentPlan resident_plan(tbtkx_context *h, int cus) {
 	                        f.slot + 2 * f.pal + 4 * (h->real_path && h->h_real),
 	                        (int64_t)h->use_resident + 2 * h->use_graph + 4 * h->slot_rows +
 	                            64 * h->use_patterns,
-	                        cus * 2 + (h->cooperative != 0)};
+	                        cus * 2 + cooperative_now(h)};
 	if (memcmp(key, h->res_plan_key, sizeof key) != 0) {
 		h->res_plan = make_plan(h, f, cus);
 		memcpy(h->res_plan_key, key, sizeof key);

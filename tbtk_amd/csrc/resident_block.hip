@@ -586,7 +586,7 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 		vectors += c.cols[m];
 	}
 	int rc;
-	if (!h->cooperative) return TBTKX_OK;
+	if (!cooperative_now(h)) return TBTKX_OK;
 	// No memory for this path's own scratch: the step kernels need what it holds.
 	auto no_memory = [&]() {
 		(void)hipGetLastError();

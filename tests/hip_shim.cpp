@@ -42,9 +42,11 @@ int hipMalloc(void **ptr, size_t bytes) {
 
 int hipLaunchCooperativeKernel(const void *f, Dim3 grid, Dim3 block, void **args, unsigned lds,
                                void *stream) {
-	typedef int (*F)(const void *, Dim3, Dim3, void **, unsigned, void *);
-	static F fn = (F)real("hipLaunchCooperativeKernel");
 	shim_cooperative++;
+	// An ordinary launch: only one process at a time has cooperative ones on a
+	// GPU. Grids have at most a workgroup per compute unit, and waits are bounded.
+	typedef int (*F)(const void *, Dim3, Dim3, void **, size_t, void *);
+	static F fn = (F)real("hipLaunchKernel");
 	if (!shim_refuse) return fn(f, grid, block, args, lds, stream);
 	typedef int (*Malloc)(void **, size_t);
 	static Malloc any_error = (Malloc)real("hipMalloc");

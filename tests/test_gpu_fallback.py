@@ -3,9 +3,15 @@ results: a cooperative launch that the runtime refuses, no memory for the
 scratch that only the resident path needs, and a wait given up on the device.
 Each is brought about on the host by a shim between the library and the runtime.
 """
+import subprocess
+import sys
+
+import numpy as np
 import pytest
 
-from shim import run_shimmed
+from tbtk_amd import engine as X
+from tbtk_amd import lattice as L
+from shim import ROOT, run_shimmed
 
 pytestmark = pytest.mark.gpu
 
@@ -65,5 +71,29 @@ for name, make in CASES:
 @pytest.mark.parametrize("name,how,settled", [
     ("shim_refuse", 1, True), ("shim_malloc_limit", 100000, False), ("shim_give_up", 1, False)])
 def test_step_kernels_take_over(tmp_path, name, how, settled):
-    """A refused launch is not tried again on the handle; memory and waits are."""
+    """A refused launch is not tried again at once; memory and waits are."""
     run_shimmed(tmp_path, BODY.format(name=name, how=how, settled=settled))
+
+
+def test_second_process_on_the_gpu(engine, tmp_path):
+    """Only one process at a time has cooperative launches on a GPU: another one
+    runs the step kernels, bitwise the same."""
+    m = L.square_spin(173, 61, disorder=0.5, seed=2)
+    N = m.basis_size
+    engine.set_csr(m.csr(), 6.0)
+    here = engine.moments(N // 2, [0, N // 2, N - 1], 60)
+    assert engine.get_option(X.OPT_RESIDENT) == 1
+    out = str(tmp_path / "there.npy")
+    code = f"""
+import sys
+sys.path.insert(0, {ROOT!r})
+import numpy as np
+from tbtk_amd import engine as X, lattice as L
+eng, m = X.Engine(0), L.square_spin(173, 61, disorder=0.5, seed=2)
+eng.set_csr(m.csr(), 6.0)
+N = m.basis_size
+np.save({out!r}, [eng.moments(N // 2, [0, N // 2, N - 1], 60) for _ in range(3)])
+"""
+    subprocess.run([sys.executable, "-u", "-c", code], check=True, timeout=60)
+    for there in np.load(out):
+        assert np.array_equal(there, here)
