@@ -466,6 +466,11 @@ __global__ __launch_bounds__(kThreads) void block_dots(const double *__restrict_
 	D[i] = s;
 }
 
+// Times in us of the rule in resident_block: a step of one round of 512 rows with
+// one entry beside the diagonal, a launch; the share of the streamed time to beat.
+constexpr double kRound = 0.11, kStep = 0.6;
+constexpr double kLeastStep = kStep + kRound * (1 + 2), kPerLaunch = 20.0, kWorth = 0.9;
+
 struct Shape {
 	int L = 0, hq = 0, ds = 0, A = 0, B = 0, Gt = 0, teams = 0, passes = 0, rows = 0;
 	double us = 0;   // a step of all passes
@@ -489,7 +494,7 @@ Shape shape_of(int64_t N, int ne, int layer, int reach, int64_t band, int V, int
 		if (fit < 1) return;
 		const int64_t passes = (groups + fit - 1) / fit, teams = (groups + passes - 1) / passes;
 		const double rounds = (double)((own + kT - 1) / kT);
-		double us = 0.6 + rounds * 0.11 * (ne + 2);
+		double us = kStep + rounds * kRound * (ne + 2);
 		if (Gt > 1)
 			us += 1.6 + (double)(teams * Gt * (win - own)) * 128 / 8e6 +
 			      0.7 * (double)((win - own - 1) / (2 * kT));
@@ -578,13 +583,26 @@ int scan_models(tbtkx_context *h, const BlockCall &c, tbtkx_context::BlockForms 
 int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done) {
 	*done = false;
 	h->last_resident = 0;
+	// Against the streamed step: 12 bytes per column element at 4.4 TB/s (1,048,576
+	// states x 256 columns: 732 us, measured 711), at least 5 us per launch; models of a
+	// batch share its launches. Wide rings lose: 864,000 states (96 x 100 x 90), 64
+	// columns, a ring of 4000 of 3800 rows, 270 us a step against 173.
 	int64_t vectors = 0;
 	std::vector<int> S(c.K);
+	double theirs = 0, least = 0;
+	int Smax = 0;
 	for (int m = 0; m < c.K; m++) {
 		S[m] = c.doubling ? (c.M[m] + 1) / 2 : c.M[m] - 1;
 		if (S[m] < 1) return TBTKX_OK;
 		vectors += c.cols[m];
+		theirs += (double)c.N[m] * c.cols[m] * 12 / 4.4e6 * S[m];
+		least += kLeastStep * S[m] + kPerLaunch;
+		Smax = std::max(Smax, S[m]);
 	}
+	theirs = std::max(theirs, 5.0 * Smax);
+	// A launch per model and its shortest steps cost more already: no scan, which
+	// takes 10 KB and some 50 us of the host per model (a batch of 1000 small models).
+	if (least > kWorth * theirs) return TBTKX_OK;
 	int rc;
 	if (!cooperative_now(h)) return TBTKX_OK;
 	// No memory for this path's own scratch: the step kernels need what it holds.
@@ -595,24 +613,16 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	};
 	tbtkx_context::BlockForms &f = c.single ? h->rb_single : h->rb_multi;
 	if ((rc = scan_models(h, c, f))) return rc == TBTKX_ERR_OOM ? no_memory() : rc;
-	// Against the streamed step: 12 bytes per column element at 4.4 TB/s (1,048,576
-	// states x 256 columns: 732 us, measured 711), at least 5 us per launch; models of a
-	// batch share its launches. Wide rings lose: 864,000 states (96 x 100 x 90), 64
-	// columns, a ring of 4000 of 3800 rows, 270 us a step against 173.
 	std::vector<Shape> sh(c.K);
-	double mine = 0, theirs = 0;
-	int Smax = 0;
+	double mine = 0;
 	for (int m = 0; m < c.K; m++) {
 		if (!f.ne[m]) return TBTKX_OK;
 		sh[m] = shape_of(c.N[m], f.ne[m], f.layer[m], f.reach[m], c.band[m], c.cols[m], h->num_cus);
 		if (sh[m].us == 0) return TBTKX_OK;
 		// Dots of complex vectors: 12.8 us where the model gives 9.4.
-		mine += sh[m].us * (c.phases ? 1.35 : 1.0) * S[m] + 20.0 * sh[m].passes;
-		theirs += (double)c.N[m] * c.cols[m] * 12 / 4.4e6 * S[m];
-		Smax = std::max(Smax, S[m]);
+		mine += sh[m].us * (c.phases ? 1.35 : 1.0) * S[m] + kPerLaunch * sh[m].passes;
 	}
-	theirs = std::max(theirs, 5.0 * Smax);
-	if (mine > 0.9 * theirs) return TBTKX_OK;
+	if (mine > kWorth * theirs) return TBTKX_OK;
 
 	size_t part = 0, D = 0, xg = 0, mu = 0;
 	uint32_t phases = 0;

@@ -25,3 +25,22 @@ for n, parts in ((37, 1), (65, 2), (91, 2)):
         print(n, M, count.value, flush=True)
         assert 0 < count.value <= parts * 40, (n, M, count.value)
 """)
+
+
+def test_many_small_models_are_not_scanned(tmp_path):
+    """A batch whose models could never pay for a resident launch each isn't
+    looked over for one: the first call's launches are the step path's."""
+    run_shimmed(tmp_path, """
+specs = [L.square_spec(5, 4 + i % 3, disorder=0.5, seed=i) for i in range(300)]
+count, got = value("shim_launches"), []
+for resident in (1, 0):
+    eng = X.Engine(0)
+    eng.set_option(X.OPT_RESIDENT, resident)
+    eng.multi_set_lattices(specs, [5.0] * 300)
+    count.value = 0
+    got.append(eng.multi_moments([np.arange(3)] * 300, [40] * 300, X.DOUBLING))
+    got.append(count.value)
+assert got[1] == got[3], (got[1], got[3])
+for a, b in zip(got[0], got[2]):
+    assert np.abs(a - b).max() < 1e-12
+""")
