@@ -316,8 +316,9 @@ int tbtkx_multi_moments(tbtkx_handle handle, const int *num_sites,
 
 /* Device time of the last recurrence call: total milliseconds between the
  * first and last step launch (HIP events on the handle's stream) and the
- * number of steps in it (one launch each, or all in one launch where the
- * recurrence ran resident, TBTKX_OPT_RESIDENT). */
+ * number of steps in it: one launch each, or, where TBTKX_OPT_RESIDENT reads
+ * 1, all of a start vector's, or of the columns that fit the chip at a time, in
+ * one launch. */
 int tbtkx_last_timing(tbtkx_handle handle, double *milliseconds,
                       int64_t *launches);
 
@@ -385,9 +386,13 @@ enum {
 	                           used the palette */,
 	TBTKX_OPT_MULTI = 17    /* tbtkx_moments_multi: 0 = plain recurrences or
 	                           exact FP64 blocks, whichever moves fewer bytes
-	                           (default); 1 = plain recurrences; 2 = exact
-	                           blocks. Reading it gives what the last call
-	                           ran (1 plain, 2 blocks) */,
+	                           (default), or resident recurrences where the
+	                           model fits one workgroup (TBTKX_OPT_RESIDENT);
+	                           1 = plain recurrences; 2 = exact blocks. Reading
+	                           it gives how the last call ran its from-indices:
+	                           1 = one after another, 2 = together (exact
+	                           blocks, or, where TBTKX_OPT_RESIDENT reads 1, a
+	                           workgroup each) */,
 	TBTKX_OPT_ROW_PATTERNS = 18 /* 1 = the slot-major plain step with the
 	                           palette reads one byte per row, an index into
 	                           the model's at most 255 distinct rows (column
@@ -408,13 +413,20 @@ enum {
 	                           (the rows whose pattern byte the step reads
 	                           with TBTKX_OPT_ROW_PATTERNS = 1); -1 when the
 	                           model has no row patterns */,
-	TBTKX_OPT_RESIDENT = 21 /* 1 = the plain recurrence runs all its steps in
-	                           one launch with the vectors resident on the
-	                           chip, where the model fits and that is faster
-	                           (default; not with TBTKX_OPT_GRAPH or options
-	                           that choose a form of the per-step kernel):
-	                           same moments; 0 = a launch per step. Reading it
-	                           gives 1 when the last plain call ran resident */
+	TBTKX_OPT_RESIDENT = 21 /* 1 = a recurrence runs all its steps in one
+	                           launch with the vectors resident on the chip,
+	                           where they fit and that is faster (default; not
+	                           with TBTKX_OPT_GRAPH or options that choose a
+	                           form of the per-step kernels): tbtkx_moments
+	                           and tbtkx_moments_multi with the same moments;
+	                           tbtkx_moments_block, tbtkx_moments_trace and
+	                           tbtkx_multi_moments of a real H in FP32, with the
+	                           same moments up to the order of their dot sums;
+	                           0 = a launch per step. A launch whose workgroups
+	                           wait for each other is cooperative, which the
+	                           runtime allows one process per GPU at a time: the
+	                           others run the steps. Reading it gives 1 when the
+	                           last recurrence call ran resident */
 };
 int tbtkx_set_option(tbtkx_handle handle, int option, int64_t value);
 
@@ -426,7 +438,11 @@ int tbtkx_set_option(tbtkx_handle handle, int option, int64_t value);
  * TBTKX_OPT_TILE_ROWS, when 0, gives the row groups per tile of the
  * last uneven-batch call; TBTKX_OPT_ELL gives 1 only when the
  * ELL copy exists and is enabled; TBTKX_OPT_REAL gives 1 when the last
- * recurrence call (plain, batched or uneven batch) ran in real arithmetic. */
+ * recurrence call (plain, batched or uneven batch) ran in real arithmetic.
+ * A batched call that ran resident, or its few columns at their own width, gives
+ * width 64, strip -1 and share 1 (its grid's, at its own width), one that ran
+ * partly so the rest's; an uneven batch that ran resident gives tile rows and
+ * share 0. */
 int tbtkx_get_option(tbtkx_handle handle, int option, int64_t *value);
 
 #ifdef __cplusplus

@@ -1517,8 +1517,7 @@ int run_resident(tbtkx_context *h, const ResidentPlan &plan, int nvec, const int
 	}
 	h->last_ms = ms_all;
 	h->last_launches = M > 1 ? M - 1 : 0;
-	h->last_real = h->real_path && h->h_real;
-	h->last_resident = 1;
+	report_plain(h, plain_form(h), true);
 	return TBTKX_OK;
 }
 
@@ -1607,6 +1606,7 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 	int rc = set_device(h);
 	if (rc) return rc;
 	if (flags & TBTKX_VEC_FP64) flags |= TBTKX_H_FP64;
+	h->last_resident = 0;
 	// Unit start vectors on a real H: two real vectors per complex column.
 	const int packed = mode == 0 && h->real_path && h->h_real;
 	const int per = packed ? 2 : 1, cols = (total + per - 1) / per;
@@ -1620,9 +1620,6 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 		mu.resize((size_t)total * M);
 		if ((rc = resident_block(h, c, reinterpret_cast<double *>(mu.data()), &done))) return rc;
 		if (done) {
-			// Counted as steps of 64 columns, as the step kernels' launches.
-			h->last_launches =
-			    (int64_t)((cols + 63) / 64) * ((flags & TBTKX_DOUBLING) ? (M + 1) / 2 : M - 1);
 			h->last_block_width = 64;
 			h->last_strip = -1;
 			h->last_share = h->last_rmul = 1;
@@ -1638,10 +1635,17 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 	const int wide = (cols - rest) * per;
 	mu.clear();
 	double ms = 0;
+	int64_t launches = 0;
 	if (wide > 0) {
 		if ((rc = wide_entry(h, wide, sites, mode, seed, M, flags, mu))) return rc;
 		ms = h->last_ms;
+		launches = h->last_launches;
+	} else {
+		h->last_block_width = 64;
+		h->last_strip = -1;
+		h->last_rmul = 1;
 	}
+	const int wide_share = h->last_share, tile_groups = h->last_tile_groups;
 	mu.resize((size_t)total * M);
 	for (int v = wide; v < total; v += w * per) {
 		const int n = std::min(total - v, w * per);
@@ -1649,13 +1653,12 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 		                         packed, reinterpret_cast<double *>(mu.data() + (size_t)v * M))))
 			return rc;
 		ms += h->last_ms;
+		launches += h->last_launches;
 	}
 	h->last_ms = ms;
-	const int S = (flags & TBTKX_DOUBLING) ? (M + 1) / 2 : M - 1;
-	h->last_launches = (int64_t)(wide / (128 * per) + parts) * S;
-	h->last_block_width = 64;
-	h->last_strip = -1;
-	h->last_rmul = 1;
+	h->last_launches = launches;
+	if (wide > 0) h->last_share = wide_share;
+	h->last_tile_groups = tile_groups;
 	return TBTKX_OK;
 }
 
@@ -1735,7 +1738,7 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 			if ((rc = tbtkx_moments(h, from[j], k1 - k0, to + k0, M, out + (size_t)k0 * M * 2)))
 				return rc;
 		}
-		h->last_multi_blocks = 0;
+		h->last_multi_batched = 0;
 		return TBTKX_OK;
 	}
 	// Gather entries: per from-index its distinct to-indices (a repeated
@@ -1754,7 +1757,7 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 	}
 	if (resident) {
 		if ((rc = run_resident(h, plan, num_from, from, grow, gvec, gslot, T, M, out))) return rc;
-		h->last_multi_blocks = blocks;
+		h->last_multi_batched = 1;
 		return TBTKX_OK;
 	}
 	std::vector<double2> mu;
@@ -1765,7 +1768,8 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 	memset(out, 0, (size_t)T * M * 16);
 	for (size_t l = 0; l < grow.size(); l++)
 		memcpy(out + (size_t)gslot[l] * M * 2, mu.data() + l * M, (size_t)M * 16);
-	h->last_multi_blocks = 1;
+	h->last_multi_batched = 1;
+	h->last_resident = 0;
 	return TBTKX_OK;
 }
 

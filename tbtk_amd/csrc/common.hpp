@@ -187,7 +187,7 @@ struct tbtkx_context {
 	int use_resident = 1;
 	tbtkx::ResidentPlan res_plan;   // of res_plan_key (resident_plan)
 	int64_t res_plan_key[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
-	int last_resident = 0;   // the last plain call ran resident
+	int last_resident = 0;   // the last recurrence call ran resident
 	int num_cus = 0;
 	int cooperative = 0;     // the device has cooperative launches
 	std::chrono::steady_clock::time_point cooperative_again;   // not before this time
@@ -277,7 +277,7 @@ struct tbtkx_context {
 	                       // of 4; 0 = 4)
 	int rows_in_flight = 0;   // strip step rows-in-flight multiplier (0 = tuned)
 	int multi_mode = 0;    // tbtkx_moments_multi: 0 by cost, 1 plain, 2 exact blocks
-	int last_multi_blocks = 0;   // the last tbtkx_moments_multi ran exact blocks
+	int last_multi_batched = 0;   // the last tbtkx_moments_multi ran its vectors together
 	int real_path = 1;     // real arithmetic for real H and real start vectors
 	int last_real = 0;     // the last recurrence call ran in real arithmetic
 
@@ -368,6 +368,9 @@ inline int launch_cooperative(tbtkx_context *h, const void *kernel, unsigned gri
 	h->cooperative_again = std::chrono::steady_clock::now() + std::chrono::seconds(10);
 	return kDeclined;
 }
+
+// What get_option reports of a plain recurrence (plain.hip).
+void report_plain(tbtkx_context *h, const PlainForm &f, bool resident);
 
 // The resident recurrence of this model and form (made once per model).
 ResidentPlan resident_plan(tbtkx_context *h, int cus);

@@ -514,7 +514,7 @@ int tbtkx_get_option(tbtkx_handle h, int option, int64_t *value) {
 	case TBTKX_OPT_AUTOTUNE: *value = h->autotune; return TBTKX_OK;
 	case TBTKX_OPT_MFMA_PIPE: *value = h->mfma_pipe; return TBTKX_OK;
 	case TBTKX_OPT_RESIDENT: *value = h->last_resident; return TBTKX_OK;
-	case TBTKX_OPT_MULTI: *value = h->last_multi_blocks ? 2 : 1; return TBTKX_OK;
+	case TBTKX_OPT_MULTI: *value = h->last_multi_batched ? 2 : 1; return TBTKX_OK;
 	case TBTKX_OPT_ROW_PATTERNS: *value = h->last_patterns; return TBTKX_OK;
 	case TBTKX_OPT_SLOT_ROWS: *value = h->slot_rows; return TBTKX_OK;
 	case TBTKX_OPT_PATTERN_BYTE_ROWS: *value = h->pat_ok ? h->pat_byte_rows : -1; return TBTKX_OK;

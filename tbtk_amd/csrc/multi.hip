@@ -1479,6 +1479,7 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 		TBTKX_REQUIRE(h->mm_N[m] * (width + 1) * 8 < ((int64_t)1 << 32), TBTKX_ERR_ARG,
 		              tag + "rows x (columns + 1) x 8 B must stay below 4 GiB");
 	}
+	h->last_resident = 0;
 	if (packed && h->use_resident && h->autotune && !h->use_graph && h->tile_rows == 0 &&
 	    h->grid_share == 0) {
 		int rc = set_device(h);
@@ -1490,6 +1491,7 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 		if ((rc = resident_block(h, c, out, &done))) return rc;
 		if (done) {
 			h->last_real = packed;
+			h->last_tile_groups = h->last_share = 0;
 			return TBTKX_OK;
 		}
 	}

@@ -930,6 +930,15 @@ static int noalloc_scratch(tbtkx_context *h, unsigned char **ptr) {
 	return TBTKX_OK;
 }
 
+void report_plain(tbtkx_context *h, const PlainForm &f, bool resident) {
+	h->last_real = h->real_path && h->h_real;
+	h->last_col16 = f.c16;
+	h->last_palette = f.pal;
+	h->last_plain_kernel = f.slot ? 2 : h->plain_kernel == 1 ? 1 : 0;
+	h->last_patterns = f.pat;
+	h->last_resident = resident;
+}
+
 // The plain recurrence with a launch per step: enqueues the moments of the
 // unit vector `from` at the indices of `uniq` into h->coef.
 static int stream_moments(tbtkx_context *h, int64_t from, const std::vector<int64_t> &uniq, int M,
@@ -1062,12 +1071,7 @@ extern "C" int tbtkx_moments_noalloc(tbtkx_handle h, int64_t from, int K,
 	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
 	h->last_ms = ms;
 	h->last_launches = M > 1 ? M - 1 : 0;
-	h->last_real = real;
-	h->last_col16 = c16;
-	h->last_palette = usepal;
-	h->last_plain_kernel = pform.slot ? 2 : h->plain_kernel == 1 ? 1 : 0;
-	h->last_patterns = pform.pat;
-	h->last_resident = 0;
+	report_plain(h, pform, false);
 	// A repeated to-index keeps only its last position (as tbtkx_moments).
 	for (int k = 0; k < K; k++)
 		for (int l = k + 1; l < K; l++)
@@ -1149,12 +1153,7 @@ extern "C" int tbtkx_moments(tbtkx_handle h, int64_t from, int K,
 	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
 	h->last_ms = ms;
 	h->last_launches = M > 1 ? M - 1 : 0;
-	h->last_real = real;
-	h->last_col16 = c16;
-	h->last_palette = usepal;
-	h->last_plain_kernel = pform.slot ? 2 : h->plain_kernel == 1 ? 1 : 0;
-	h->last_patterns = pform.pat;
-	h->last_resident = resident;
+	report_plain(h, pform, resident);
 
 	for (int k = 0; k < K; k++) {
 		double *o = out + (size_t)k * M * 2;

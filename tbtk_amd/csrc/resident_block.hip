@@ -582,7 +582,6 @@ int scan_models(tbtkx_context *h, const BlockCall &c, tbtkx_context::BlockForms 
 
 int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done) {
 	*done = false;
-	h->last_resident = 0;
 	// Against the streamed step: 12 bytes per column element at 4.4 TB/s (1,048,576
 	// states x 256 columns: 732 us, measured 711), at least 5 us per launch; models of a
 	// batch share its launches. Wide rings lose: 864,000 states (96 x 100 x 90), 64
@@ -615,11 +614,13 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	if ((rc = scan_models(h, c, f))) return rc == TBTKX_ERR_OOM ? no_memory() : rc;
 	std::vector<Shape> sh(c.K);
 	double mine = 0;
+	int64_t steps = 0;
 	for (int m = 0; m < c.K; m++) {
 		if (!f.ne[m]) return TBTKX_OK;
 		sh[m] = shape_of(c.N[m], f.ne[m], f.layer[m], f.reach[m], c.band[m], c.cols[m], h->num_cus);
 		if (sh[m].us == 0) return TBTKX_OK;
 		// Dots of complex vectors: 12.8 us where the model gives 9.4.
+		steps += (int64_t)S[m] * sh[m].passes;
 		mine += sh[m].us * (c.phases ? 1.35 : 1.0) * S[m] + kPerLaunch * sh[m].passes;
 	}
 	if (mine > kWorth * theirs) return TBTKX_OK;
@@ -709,7 +710,7 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	float ms = 0;
 	TBTKX_CHECK_HIP(hipEventElapsedTime(&ms, h->ev_start, h->ev_stop));
 	h->last_ms = ms;
-	h->last_launches = Smax;
+	h->last_launches = steps;
 	h->last_resident = 1;
 	*done = true;
 	if (!c.doubling) {
