@@ -1717,7 +1717,10 @@ int tbtkx_moments_multi(tbtkx_handle h, int num_from, const int64_t *from,
 	if (T == 0) return TBTKX_OK;
 	int rc = set_device(h);
 	if (!rc) rc = build_plain_forms(h);
-	if (!rc && h->plain_kernel == 2 && !(h->use_palette && h->slot_pal)) rc = build_slot_values(h);
+	// Values in slots only where the vectors may run resident, a workgroup each.
+	if (!rc && h->multi_mode == 0 && num_from > 1 && h->use_resident && h->plain_kernel == 2 &&
+	    !(h->use_palette && h->slot_pal) && h->N <= one_workgroup_rows(h))
+		rc = build_slot_values(h);
 	if (rc) return rc;
 	const int packed = h->real_path && h->h_real;
 	int B = 64;

@@ -372,6 +372,9 @@ inline int launch_cooperative(tbtkx_context *h, const void *kernel, unsigned gri
 // What get_option reports of a plain recurrence (plain.hip).
 void report_plain(tbtkx_context *h, const PlainForm &f, bool resident);
 
+// The most rows that one workgroup of the resident recurrence takes, for this
+// model's entries beside the diagonal; 0: more than the kernels have.
+int64_t one_workgroup_rows(const tbtkx_context *h);
 // The resident recurrence of this model and form (made once per model).
 ResidentPlan resident_plan(tbtkx_context *h, int cus);
 // Enqueues the moments of V start vectors (V = 1 unless plan.C covers the

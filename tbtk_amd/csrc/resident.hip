@@ -806,6 +806,14 @@ int run_res(tbtkx_context *h, const ResidentPlan &plan, int V, const int64_t *fr
 
 }  // namespace
 
+int64_t one_workgroup_rows(const tbtkx_context *h) {
+	const bool real = h->real_path && h->h_real;
+	const int H = h->slot_half;
+	if (H > 4) return 0;
+	const int64_t rows = (int64_t)kResThreads * (real ? max_rows<double, false>(H) : max_rows<Z2, false>(H));
+	return std::min<int64_t>(rows, (real ? R64<double>::kStride : R64<Z2>::kStride) - 1);
+}
+
 // The model fits one workgroup's registers and LDS, or tiles of it fit and
 // their exchanges cost less than a launch per step. Times in us, fitted to
 // (model and measured, real H, H = 2 unless said): narrow, 73,006 states k = 1 1.9
@@ -823,12 +831,11 @@ static ResidentPlan make_plan(const tbtkx_context *h, const PlainForm &f, int cu
 	const int64_t N = h->N, T = kResThreads;
 	const int64_t window = (real ? R64<double>::kStride : R64<Z2>::kStride) - 1;
 	const int64_t wide_window = kWideBytes / (real ? 8 : 16) - 1;
-	const int one = real ? max_rows<double, false>(H) : max_rows<Z2, false>(H);
 	const int many = real ? max_rows<double, true>(H) : max_rows<Z2, true>(H);
 	const int wide = !f.pal ? 0 : real ? wide_rows<double>(H) : wide_rows<Z2>(H);
 	// One round of rows (1024), and what a step takes without any.
 	const double set = (real ? 0.025 : 0.06) * (2 * H + 1), base = 0.14;
-	if (N <= (int64_t)one * T && N <= window) {
+	if (N <= one_workgroup_rows(h)) {
 		best.C = best.L = best.B = (int)N;
 		best.A = 1;
 		best.us = base + set * (double)((N + T - 1) / T);

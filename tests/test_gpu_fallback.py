@@ -97,3 +97,24 @@ np.save({out!r}, [eng.moments(N // 2, [0, N // 2, N - 1], 60) for _ in range(3)]
     subprocess.run([sys.executable, "-u", "-c", code], check=True, timeout=60)
     for there in np.load(out):
         assert np.array_equal(there, here)
+
+
+def test_exact_blocks_need_no_slot_values(tmp_path):
+    """Vectors that run in exact blocks: without the palette the plain step reads
+    values in slots (2 x 5 x 16 B a row), which aren't built for them."""
+    run_shimmed(tmp_path, """
+m = L.square(101, 97, disorder=0.5, seed=3)
+eng.set_csr(m.csr(), 5.0)
+eng.set_option(X.OPT_PALETTE, 0)
+froms = np.arange(0, 9000, 150)
+call = lambda: np.concatenate(eng.moments_multi(froms, [[int(f)] for f in froms], 30))
+eng.set_option(X.OPT_MULTI, 2)
+eng.set_option(X.OPT_PLAIN_KERNEL, 0)
+ref = call()
+eng.set_option(X.OPT_PLAIN_KERNEL, 2)
+value("shim_malloc_limit").value = 500000
+for mode in (2, 0):
+    eng.set_option(X.OPT_MULTI, mode)
+    assert np.array_equal(call(), ref)
+    assert eng.get_option(X.OPT_MULTI) == 2
+""")
