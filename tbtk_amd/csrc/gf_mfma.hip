@@ -478,10 +478,19 @@ int tbtkx_contract_mfma(tbtkx_handle h, int type, double *out) {
 		// doubles, and no pinning of the caller's pages. Contraction and result:
 		// 400 vectors x 500 moments x 1000 energies 239 us (widened on the device
 		// and copied straight out 517), 1500 x 600 x 600 664 us (1132).
-		if (!h->gf_stage) TBTKX_CHECK_HIP(hipHostMalloc(&h->gf_stage, 2 * kStageBytes, 0));
+		// Without pinned memory a pageable buffer does, at the copies' pace.
+		std::vector<float> pageable;
+		float *stage = static_cast<float *>(h->gf_stage);
+		if (!stage && hipHostMalloc(&h->gf_stage, 2 * kStageBytes, 0) == hipSuccess)
+			stage = static_cast<float *>(h->gf_stage);
+		if (!stage) {
+			(void)hipGetLastError();
+			h->gf_stage = nullptr;
+			pageable.resize(2 * kStageBytes / 4);
+			stage = pageable.data();
+		}
 		const int64_t n = (int64_t)K * E, part = kStageBytes / 8;
-		float *const half[2] = {static_cast<float *>(h->gf_stage),
-		                        static_cast<float *>(h->gf_stage) + 2 * part};
+		float *const half[2] = {stage, stage + 2 * part};
 		for (int64_t i = 0, b = 0; i < n + part; i += part, b ^= 1) {
 			TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
 			if (i < n)

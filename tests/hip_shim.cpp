@@ -23,6 +23,7 @@ int shim_launches = 0;      // kernel launches
 int shim_cooperative = 0;   // cooperative launches
 int shim_refuse = 0;        // 1: cooperative launches are refused (too large)
 int shim_malloc_limit = 0;  // > 0: no device memory for as many bytes or more
+int shim_no_pinned = 0;     // 1: no pinned host memory
 int shim_give_up = 0;       // 1: a 4-byte result copied to the host reads 1
 
 int hipLaunchKernel(const void *f, Dim3 grid, Dim3 block, void **args, size_t lds, void *stream) {
@@ -38,6 +39,12 @@ int hipMalloc(void **ptr, size_t bytes) {
 	// Refused by the runtime itself, which leaves its error behind.
 	if (shim_malloc_limit > 0 && bytes >= (size_t)shim_malloc_limit) bytes = (size_t)1 << 60;
 	return fn(ptr, bytes);
+}
+
+int hipHostMalloc(void **ptr, size_t bytes, unsigned flags) {
+	typedef int (*F)(void **, size_t, unsigned);
+	static F fn = (F)real("hipHostMalloc");
+	return fn(ptr, shim_no_pinned ? (size_t)1 << 60 : bytes, flags);
 }
 
 int hipLaunchCooperativeKernel(const void *f, Dim3 grid, Dim3 block, void **args, unsigned lds,

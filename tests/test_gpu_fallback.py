@@ -118,3 +118,16 @@ for mode in (2, 0):
     assert np.array_equal(call(), ref)
     assert eng.get_option(X.OPT_MULTI) == 2
 """)
+
+
+def test_matrix_contraction_without_pinned_memory(tmp_path):
+    """Results through a pageable buffer, bitwise, in several parts of it."""
+    run_shimmed(tmp_path, """
+rng = np.random.default_rng(2)
+eng.lut_generate(64, 1500, -5.0, 5.0, 6.0)
+eng.coeffs_upload(rng.normal(size=(900, 64)) + 1j * rng.normal(size=(900, 64)))
+value("shim_no_pinned").value = 1
+pageable = eng.contract_mfma(X.RETARDED)
+value("shim_no_pinned").value = 0
+assert np.array_equal(pageable, eng.contract_mfma(X.RETARDED))
+""")
