@@ -920,18 +920,24 @@ void launch_step(tbtkx_context *h, const Plan &p, const Phase &ph, bool first,
 #undef TBTKX_LS
 }
 
-int reserve_plan(tbtkx_context *h, const Plan &p, int ncols, int64_t mu_elems) {
+int reserve_plan(tbtkx_context *h, Plan &p, int ncols, int64_t mu_elems) {
 	int rc;
 	if ((rc = h->mm_desc.reserve(p.desc.size() * sizeof(MDesc)))) return rc;
 	if ((rc = h->mm_tab.reserve(p.tab.size() * 4))) return rc;
 	if ((rc = h->mm_x.reserve((size_t)p.vec_elems * 8))) return rc;
 	if ((rc = h->mm_y.reserve((size_t)p.vec_elems * 8))) return rc;
-	if ((rc = h->mm_part.reserve((size_t)(p.max_slots > 0 ? p.max_slots : 1) * p.ring * 2 *
-	                             kMaxWidth * 16)))
-		return rc;
-	if ((rc = h->mm_seg.reserve((size_t)(p.max_seg > 0 ? p.max_seg : 1) * p.ring * 2 *
-	                            kMaxWidth * 16)))
-		return rc;
+	auto slots = [&]() {
+		const size_t each = (size_t)p.ring * 2 * kMaxWidth * 16;
+		const int r = h->mm_part.reserve((size_t)(p.max_slots > 0 ? p.max_slots : 1) * each);
+		return r ? r : h->mm_seg.reserve((size_t)(p.max_seg > 0 ? p.max_seg : 1) * each);
+	};
+	rc = slots();
+	if (rc == TBTKX_ERR_OOM && p.ring > 1) {   // one step's slots must do
+		(void)hipGetLastError();
+		p.ring = 1;
+		rc = slots();
+	}
+	if (rc) return rc;
 	if ((rc = h->mm_D.reserve((size_t)(mu_elems > 0 ? mu_elems : 1) * 16))) return rc;
 	if ((rc = h->mm_cols.reserve((size_t)ncols * sizeof(GCol)))) return rc;
 	TBTKX_CHECK_HIP(hipMemcpyAsync(h->mm_desc.ptr, p.desc.data(),

@@ -131,3 +131,20 @@ pageable = eng.contract_mfma(X.RETARDED)
 value("shim_no_pinned").value = 0
 assert np.array_equal(pageable, eng.contract_mfma(X.RETARDED))
 """)
+
+
+def test_batch_with_little_memory_for_dot_slots(tmp_path):
+    """Memory for one step's dot slots (20 MB), not for several (266 MB): reduced
+    every step, bitwise the same sums."""
+    run_shimmed(tmp_path, """
+m = L.square(100, 200, disorder=0.5, seed=3, flux=0.01)
+got = []
+for limit in (0, 100000000):
+    eng = X.Engine(0)
+    eng.multi_set([m.csr()], [5.0])
+    eng.set_option(X.OPT_TILE_ROWS, 2)
+    value("shim_malloc_limit").value = limit
+    got.append(eng.multi_moments([np.arange(40)], [60], X.DOUBLING)[0])
+    value("shim_malloc_limit").value = 0
+assert np.array_equal(*got)
+""")
