@@ -209,3 +209,33 @@ def test_tiles_without_palette(res, oracle_mod):
     csr = cylinder(211, 190, 1, seed=4)
     res.set_option(X.OPT_PALETTE, 0)
     assert check(res, oracle_mod, csr, 5.0, 9, [0, 9, 189, 190, 40089], 60) == 1
+
+
+def test_two_handles_at_once(oracle_mod):
+    """Threads with handles of their own whose workgroups exchange, narrow tiles
+    beside wide ones and blocks: every call bitwise the handle's first."""
+    import threading
+    wrong, done = [], []
+
+    def work(make, s, call):
+        eng = X.Engine(0)
+        m = make()
+        eng.set_csr(m.csr(), s)
+        first = call(eng, m.basis_size)
+        for _ in range(20):
+            if not np.array_equal(call(eng, m.basis_size), first):
+                wrong.append(m.name)
+        done.append(eng.get_option(X.OPT_RESIDENT))
+        eng.close()
+
+    plain = lambda eng, N: eng.moments(N // 2, [0, N // 2, N - 1], 300)
+    block = lambda eng, N: eng.moments_block(np.arange(0, N, N // 37), 60, 0)
+    jobs = [(lambda: L.square_spin(173, 61, disorder=0.5, seed=2), 6.0, plain),
+            (lambda: L.square_spin(611, 613, disorder=0.5, seed=2), 6.0, plain),
+            (lambda: L.honeycomb_ribbon(40, 997, disorder=0.5, seed=4), 9.2, block)]
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert wrong == [] and done == [1, 1, 1]

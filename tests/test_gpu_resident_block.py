@@ -111,3 +111,74 @@ def test_many_values_and_zero_entries(res):
         b = res.moments_block([0, 5, n // 2, n - 1], 60, X.DOUBLING)
         res.set_option(X.OPT_RESIDENT, 1)
         close(a, b, 60)
+
+
+# The two sides hold the same FP32 values (gathered moments are equal bit for
+# bit); their dots differ in the order of N FP64 sums of products whose magnitudes
+# add to at most 1 (|T_n| <= 1), twice in 2 <n|n> - mu_0: 4 N 2^-53.
+def dots(N):
+    return 4 * N * 2.0 ** -53
+
+
+def sides(eng, call):
+    """The resident result, which must have run so, and the step kernels'."""
+    a = call()
+    assert eng.get_option(X.OPT_RESIDENT) == 1
+    eng.set_option(X.OPT_RESIDENT, 0)
+    b = call()
+    assert eng.get_option(X.OPT_RESIDENT) == 0
+    eng.set_option(X.OPT_RESIDENT, 1)
+    return a, b
+
+
+MANY = ((41, 0), (64, X.DOUBLING), (63, X.DOUBLING))
+FEW = ((3, 0), (3, X.DOUBLING), (4, X.DOUBLING))   # two steps: fewer never pay
+
+
+@pytest.mark.parametrize("name,n,cols,moments", [
+    ("square", (9, 7), 3, MANY), ("cubic", (9, 8, 7), 40, MANY), ("nambu", (31, 33), 17, MANY),
+    ("square", (64, 64), 65, MANY), ("spin", (57, 61), 37, MANY), ("honeycomb", (7, 501), 12, MANY),
+    ("nambu", (120, 131), 100, MANY), ("honeycomb", (40, 997), 37, MANY),
+    ("spin", (520, 530), 16, MANY), ("honeycomb", (500, 500), 9, MANY),
+    ("honeycomb", (32, 32), 2048, FEW), ("nambu", (32, 32), 2048, FEW),
+    ("square", (63, 65), 2041, FEW), ("spin", (1024, 500), 16, FEW)])
+def test_blocks_that_run_resident(res, name, n, cols, moments):
+    """One workgroup, tiles of few and of all rows per thread, one and two passes,
+    many steps and two."""
+    m, s = model(name, n)
+    N = m.basis_size
+    print(name, N, cols, flush=True)
+    res.set_csr(m.csr(), s)
+    sites = np.random.default_rng(3).integers(0, N, cols)
+    sites[0], sites[-1] = 0, N - 1
+    for M, flags in moments:
+        a, b = sides(res, lambda: res.moments_block(sites, M, flags))
+        if flags == 0:
+            assert np.array_equal(a, b), M
+        else:
+            assert np.abs(a - b).max() <= dots(N), M
+
+
+@pytest.mark.parametrize("name,n,R", [
+    ("square", (9, 7), 1), ("cubic", (9, 8, 7), 40), ("nambu", (120, 131), 50),
+    ("spin", (200, 211), 24), ("square", (300, 301), 33)])
+def test_random_phases_that_run_resident(res, name, n, R):
+    m, s = model(name, n)
+    N = m.basis_size
+    print(name, N, R, flush=True)
+    res.set_csr(m.csr(), s)
+    a, b = sides(res, lambda: res.moments_trace(R, 11, 50))
+    assert np.abs(a - b).max() <= dots(N) * N * R
+
+
+def test_which_matrices_run_resident(res):
+    """Bond values of more than a palette don't, few with explicit zeros do."""
+    n = 3000
+    i, d = np.arange(n - 1), np.arange(n // 2)
+    rng = np.random.default_rng(8)
+    for v, ran in ((rng.uniform(-1, 1, n - 1), 0), (np.where(i % 3 == 0, 0.0, -0.8), 1)):
+        csr = L.coo_to_csr(np.concatenate([i, i + 1, d]), np.concatenate([i + 1, i, d]),
+                           np.concatenate([v, v, rng.uniform(-1, 1, d.size)]).astype(complex), n)
+        res.set_csr(csr, 4.0)
+        res.moments_block([0, 5, n // 2, n - 1], 60, X.DOUBLING)
+        assert res.get_option(X.OPT_RESIDENT) == ran
