@@ -527,23 +527,13 @@ __device__ __forceinline__ void model_rows(
 // it leaves a model, into slot pbase[k*8+x] + its rank among the
 // wavefronts that touch the model's piece of part x (pstart: the piece's
 // first tile).
-// Batches of at most 5 ELL slots per row are held to 4 wavefronts per SIMD
-// (128 VGPRs): the doubling variants then keep 4-6 values in scratch and
-// still finish the 64-model batch 1.3% sooner than at 3 wavefronts.
 template <int WMAX, bool FIRST, bool DOTS, bool REALH>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(WMAX <= 5 ? 4 : 1))) void multi_step(
+__device__ __forceinline__ void step_tiles(
     const MDesc *__restrict__ md, const int *__restrict__ toff, int kact,
     const int *__restrict__ xpart, const int *__restrict__ pbase,
     const int *__restrict__ pstart, int G, const uint32_t *__restrict__ ecol,
     const float2 *__restrict__ ev, const float2 *__restrict__ X,
-    float2 *__restrict__ Y, double2 *__restrict__ part, int packed,
-    const GCol *__restrict__ cols, int ncols, double2 *__restrict__ mu, int nprev) {
-	// The moments of X (step nprev) ride on the launch that reads it; X is not
-	// written here.
-	if (!DOTS)
-		for (int g = blockIdx.x * kThreads + threadIdx.x; g < ncols; g += gridDim.x * kThreads)
-			gather_col(cols, g, X, mu, nprev);
+    float2 *__restrict__ Y, double2 *__restrict__ part, int packed) {
 	const int lane = threadIdx.x & 63;
 	const int x = blockIdx.x & 7;
 	const int nwx = (gridDim.x >> 3) * kWaves;                  // wavefronts per XCD
@@ -598,6 +588,28 @@ __attribute__((amdgpu_waves_per_eu(WMAX <= 5 ? 4 : 1))) void multi_step(
 		if (t >= phi) break;
 		while (toff[m + 1] <= t) m++;
 	}
+}
+
+// Batches of at most 5 ELL slots per row are held to 4 wavefronts per SIMD
+// (128 VGPRs): the doubling variants then keep 4-6 values in scratch and
+// still finish the 64-model batch 1.3% sooner than at 3 wavefronts.
+template <int WMAX, bool FIRST, bool DOTS, bool REALH>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(WMAX <= 5 ? 4 : 1))) void multi_step(
+    const MDesc *__restrict__ md, const int *__restrict__ toff, int kact,
+    const int *__restrict__ xpart, const int *__restrict__ pbase,
+    const int *__restrict__ pstart, int G, const uint32_t *__restrict__ ecol,
+    const float2 *__restrict__ ev, const float2 *__restrict__ X,
+    float2 *__restrict__ Y, double2 *__restrict__ part, int packed,
+    const GCol *__restrict__ cols, int ncols, double2 *__restrict__ mu, int nprev) {
+	step_tiles<WMAX, FIRST, DOTS, REALH>(md, toff, kact, xpart, pbase, pstart, G, ecol, ev, X, Y,
+	                                     part, packed);
+	// The moments of X (step nprev) ride on the launch that reads it; X is not
+	// written here. At the end: a store before the tiles would keep their tables
+	// out of the scalar registers (94 -> 128 VGPRs and scratch).
+	if (!DOTS)
+		for (int g = blockIdx.x * kThreads + threadIdx.x; g < ncols; g += gridDim.x * kThreads)
+			gather_col(cols, g, X, mu, nprev);
 }
 
 // Pass 1: segment s = (model, slot_lo, slot_hi) of <= 64 slots; one
