@@ -1598,8 +1598,44 @@ int wide_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 
 // Columns in blocks of 64, 128 or 256 (wide_entry), except that up to
 // kNarrowRest columns, alone or left over by blocks of 128, run at their own
-// width (narrow_moments).
+// width (narrow_moments) where narrow_pays.
 constexpr int kNarrowRest = 96;
+
+// Times in us of a call of S steps: a step moves 12 bytes per entry and 24 per
+// column element (`moved`, at 4.4 TB/s) and takes no less than its launches; with
+// dots, a full block's slots cost 3.5 ns per row and 128 columns once. One column
+// alone sums 64 rows' dots in a wavefront (+3 us a step). Model and measured, whole
+// calls: 9,800 rows, 32 columns, 100 steps, dots: 884 867 narrow, 946 880 in a block
+// of 64; 90,300 rows, 33 columns: 2200 2340 and 5070 4780; 20 columns gathered, 100
+// steps: 1130 1150 and 4530 4125; 3600 rows, 65 columns, 100 steps, dots: 1610 1540 in
+// two parts, 1030 1020 in a block of 128.
+bool narrow_pays(const tbtkx_context *h, int cols, int rest, int parts, int S, bool dots) {
+	auto moved = [&](int w) { return (double)h->N * (12 * h->ell_W + 24 * w) / 4.4e6; };
+	auto wide = [&](int c) {
+		double best = 0;
+		for (int B : {64, 128, 256}) {
+			if (B == 256 && c <= 192) continue;   // never chosen for fewer
+			const int blocks = (c + B - 1) / B;
+			const double m = B == 64 ? 1.25 * moved(B) : moved(B);
+			const double least = B == 64 ? 8.0 : B == 128 ? 9.6 : 15.8;
+			const double once = dots ? blocks * std::max(1, B / 128) * (60 + std::min(400.0, 0.0035 * h->N))
+			                         : 20.0 + 20.0 * blocks;
+			const double us = once + S * blocks * (dots ? std::max(least, 4.5 + m)
+			                                            : std::max(least - 0.5, 3.5 + m));
+			if (best == 0 || us < best) best = us;
+		}
+		return best;
+	};
+	double narrow = cols > rest ? wide(cols - rest) : 0.0;
+	for (int p = 0, left = rest; p < parts; p++) {
+		const int w = (left + parts - p - 1) / (parts - p);
+		const double m = moved(w);
+		left -= w;
+		narrow += dots ? 72 + S * (std::max(6.8 + 0.65 * m, 4 + m) + (w == 1 ? 3.0 : 0.0))
+		               : 60 + S * std::max(4.2 + 0.5 * m, 2 + 0.8 * m);
+	}
+	return narrow < wide(cols);
+}
 
 int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
                 uint64_t seed, int M, int flags, std::vector<double2> &mu) {
@@ -1630,7 +1666,9 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 	}
 	const int rest = cols % 128;
 	const int parts = rest > 64 ? 2 : 1, w = (rest + parts - 1) / parts;
-	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w))
+	const bool dots = (flags & TBTKX_DOUBLING) != 0;
+	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w) ||
+	    !narrow_pays(h, cols, rest, parts, dots ? (M + 1) / 2 : M - 1, dots))
 		return wide_entry(h, total, sites, mode, seed, M, flags, mu);
 	const int wide = (cols - rest) * per;
 	mu.clear();

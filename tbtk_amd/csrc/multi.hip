@@ -1034,16 +1034,24 @@ int64_t run_steps(const Plan &p) {
 // Autotuner: time a few steps of the first phase for each (tile groups, grid
 // share) candidate on the actual batch and keep the fastest: persistent grids
 // (share 1 or 2) with tiles of 2-16 row groups, and one tile per wavefront
-// (share 0) with tiles of 8-64 row groups.
+// (share 0) with tiles of 8-64 row groups. Narrow blocks: the first kNarrowCand,
+// whose best took at most 1.05 of the best of all 12 (8 models of 29,760 to 753,480
+// rows, 1 to 64 columns); two row groups per tile without trials where a step moves
+// less than an XCD's L2 holds (3600 to 29,760 rows: at most 1.08 of the best).
 int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<int> &S,
-             bool dots, int ncols, int64_t mu_elems, TunedShape &tuned) {
-	static const int kCand[][2] = {{1, 2}, {1, 4}, {1, 8}, {1, 16}, {2, 2},  {2, 4},
-	                               {2, 8}, {2, 16}, {0, 8}, {0, 16}, {0, 32}, {0, 64}};
-	constexpr int kTrial = 4;
+             bool dots, int ncols, int64_t mu_elems, bool narrow, TunedShape &tuned) {
+	static const int kCand[][2] = {{1, 2}, {1, 4}, {1, 16}, {2, 2},  {2, 4},  {0, 8},
+	                               {1, 8}, {2, 8}, {2, 16}, {0, 16}, {0, 32}, {0, 64}};
+	constexpr int kTrial = 4, kCands = sizeof kCand / sizeof kCand[0], kNarrowCand = 6;
 	float best = 0;
 	int bestG = 8, bestShare = 1;
-	for (const auto &cand : kCand) {
-		const int share = cand[0], G = cand[1];
+	int cands = narrow ? kNarrowCand : kCands;
+	if (narrow && (double)h->mm_N[0] * (12 * h->mm_W + 24 * width[0]) < 4e6) {
+		bestShare = bestG = 2;
+		cands = 0;
+	}
+	for (int i = 0; i < cands; i++) {
+		const int share = kCand[i][0], G = kCand[i][1];
 		{
 			Plan p;
 			int rc = make_plan(h, width, S, dots, G, share, p);
@@ -1089,7 +1097,7 @@ int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<
 // What the tuned shape of a narrow block depends on: the lanes of a row, which
 // set the rows of a row group, and whether a lane moves two columns; rows that
 // fill a group by themselves in two halves. The steps don't matter, and a class
-// per width would tune up to 64 times per model (about 12 x 5 steps each).
+// per width would tune up to 64 times per model (6 x 5 steps each).
 int narrow_class(int w, int W) {
 	const int pairs = use_pairs(w, W) ? 1 : 0;
 	const int lanes = pairs ? (w + 1) / 2 : w;
@@ -1136,7 +1144,7 @@ int run_batch(tbtkx_context *h, const int *num_sites, const int64_t *sites, cons
 			int64_t mu_elems = 0;
 			for (int m = 0; m < K; m++)
 				mu_elems += dots ? (int64_t)S[m] * 2 * width[m] : out_off[m + 1] - out_off[m];
-			if ((rc = autotune(h, width, S, dots, ncols, mu_elems, tuned))) return rc;
+			if ((rc = autotune(h, width, S, dots, ncols, mu_elems, narrow, tuned))) return rc;
 			memcpy(tuned.key, key, sizeof key);
 		}
 		G = tuned.g;

@@ -70,7 +70,7 @@ def test_steps_of_resident_blocks(eng, doubling, S):
 def test_steps_and_shape_of_blocks_with_a_narrow_rest(eng):
     """128 columns in full blocks and 65 in two parts: the steps of each, and the
     shape of the full blocks. The uneven batch's tile is not a narrow block's."""
-    flux = L.square(19, 23, disorder=0.5, seed=4, flux=0.03)
+    flux = L.square(300, 301, disorder=0.5, seed=4, flux=0.03)
     eng.multi_set([flux.csr()] * 2, [5.0] * 2)
     eng.multi_moments([np.arange(40)] * 2, [40] * 2, X.DOUBLING)
     tile = eng.get_option(X.OPT_TILE_ROWS)
