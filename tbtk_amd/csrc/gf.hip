@@ -194,7 +194,7 @@ __global__ __launch_bounds__(64) void contract_few(
 		// The chunk's rows. A row takes a scalar add, a scalar minimum and one load,
 		// where a lone wavefront pays every instruction in full. Rows read ahead of
 		// the chunk's end repeat its last. Offsets stay in 32 bits: contract_launch
-		// comes here with at most 16 x 5 energies per CU (20,480), 16 B each, and r
+		// comes here with at most 16 x 4 energies per CU (16,384), 16 B each, and r
 		// runs to 512 + 3 kAhead rows.
 		const __amdgpu_buffer_rsrc_t tab = __builtin_amdgcn_make_buffer_rsrc(
 		    const_cast<char *>(reinterpret_cast<const char *>(L)) + (int64_t)r0 * rowb, 0,
@@ -376,8 +376,9 @@ __global__ __launch_bounds__(kThreads) void contract_each(
 // Contracts the K vectors in h->gf_in with the array L into h->gf_out.
 // contract_many with 8 vectors per wavefront where that gives every SIMD a
 // wavefront (4 per CU), with 4 where it gives every CU three; contract_few up to
-// about 5 wavefronts per CU; contract_each between. Whole calls at 1000 energies
-// and moments, Retarded, in us:
+// one wavefront per SIMD (beyond, some SIMDs run two: 800 energies, 777 moments, 48
+// vectors, 1224 wavefronts: 145 us, contract_each 119; 40 vectors, 1020: 105, 109);
+// contract_each between. Whole calls at 1000 energies and moments, Retarded, in us:
 //   vectors           1    9   37*   64  128  200  256  600   (* 777 x 801)
 //   contract_few     67   78  106   206  389  625
 //   contract_each    92   98  114   171  288  488  553 1315
@@ -397,7 +398,7 @@ int contract_launch(tbtkx_context *h, const double *L, const double *den, int K,
 	else if (tiles * ((K + 3) / 4) >= 3 * cus)
 		contract_many<TYPE, DIRECT, 4>
 		    <<<groups(4), kThreads, 0, h->stream>>>(L, C, den, G, K, M, E, s);
-	else if (((E + 15) / 16) * (int64_t)((K + 1) / 2) <= 5 * cus)
+	else if (((E + 15) / 16) * (int64_t)((K + 1) / 2) <= 4 * cus)
 		contract_few<TYPE, DIRECT>
 		    <<<dim3((unsigned)((E + 15) / 16), (unsigned)((K + 1) / 2)), 64, 0, h->stream>>>(
 		        L, C, den, G, K, M, E, s);

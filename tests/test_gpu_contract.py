@@ -35,9 +35,9 @@ def test_contraction_bitwise(engine, oracle_mod, K, M, E, gtype):
 @pytest.mark.parametrize("K,M", [(1, 1), (2, 2), (1, 18), (2, 49), (1, 513), (1, 530)])
 def test_few_vectors_widest_rows(engine, oracle_mod, K, M, gtype):
     """Few vectors at the most energies the few-vector kernel takes on 256 compute
-    units (16 x 5 x 256), where the rows it reads ahead of the last one would
+    units (16 x 4 x 256), where the rows it reads ahead of the last one would
     lie farthest beyond the array: bitwise the oracle."""
-    E, s, lo, hi = 20480, 6.0, -5.7, 5.8
+    E, s, lo, hi = 16384, 6.0, -5.7, 5.8
     rng = np.random.default_rng(M)
     c = rng.normal(size=(K, M)) + 1j * rng.normal(size=(K, M))
     engine.lut_generate(M, E, lo, hi, s)
@@ -53,3 +53,19 @@ def test_few_vectors_widest_rows(engine, oracle_mod, K, M, gtype):
         assert np.array_equal(direct[k], oracle_mod.gf_direct(gtype, c[k], lo, hi, E, s)), k
         # The generated table: a few ulp of acos, times n up to M, per term.
         assert np.abs(got[k] - ref).max() <= 1e-13 * M * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("K", [32, 33, 34])
+def test_beside_one_wavefront_per_simd(engine, oracle_mod, K):
+    """1000 energies: 1008 wavefronts of the few-vector kernel with 32 vectors, and 1071
+    with 33, beyond its line at 4 per compute unit."""
+    M, E, s, lo, hi = 37, 1000, 6.0, -5.7, 5.8
+    rng = np.random.default_rng(K)
+    c = rng.normal(size=(K, M)) + 1j * rng.normal(size=(K, M))
+    table = oracle_mod.lookup_table(M, E, lo, hi, s)
+    engine.lut_upload(table)
+    for gtype in range(4):
+        got = engine.contract(c, gtype)
+        for k in (0, 31, K - 1):
+            assert np.array_equal(got[k], oracle_mod.gf_lookup(gtype, table, c[k]))
+    engine.lut_destroy()
