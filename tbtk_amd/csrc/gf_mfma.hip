@@ -492,7 +492,7 @@ int tbtkx_contract_mfma(tbtkx_handle h, int type, double *out) {
 		const int64_t n = (int64_t)K * E, part = kStageBytes / 8;
 		float *const half[2] = {stage, stage + 2 * part};
 		for (int64_t i = 0, b = 0; i < n + part; i += part, b ^= 1) {
-			TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
+			if (i > 0) TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
 			if (i < n)
 				TBTKX_CHECK_HIP(hipMemcpyAsync(half[b], G + i, (size_t)std::min(part, n - i) * 8,
 				                               hipMemcpyDeviceToHost, h->stream));
