@@ -1598,7 +1598,7 @@ int wide_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 
 // Columns in blocks of 64, 128 or 256 (wide_entry), except that up to
 // kNarrowRest columns, alone or left over by blocks of 128, run at their own
-// width (narrow_moments) where narrow_pays.
+// width (narrow_moments) where that is faster (split_columns).
 constexpr int kNarrowRest = 96;
 
 // Times in us of a call of S steps: a step moves 12 bytes per entry and 24 per
@@ -1609,32 +1609,48 @@ constexpr int kNarrowRest = 96;
 // of 64; 90,300 rows, 33 columns: 2200 2340 and 5070 4780; 20 columns gathered, 100
 // steps: 1130 1150 and 4530 4125; 3600 rows, 65 columns, 100 steps, dots: 1610 1540 in
 // two parts, 1030 1020 in a block of 128.
-bool narrow_pays(const tbtkx_context *h, int cols, int rest, int parts, int S, bool dots) {
-	auto moved = [&](int w) { return (double)h->N * (12 * h->ell_W + 24 * w) / 4.4e6; };
-	auto wide = [&](int c) {
-		double best = 0;
-		for (int B : {64, 128, 256}) {
-			if (B == 256 && c <= 192) continue;   // never chosen for fewer
-			const int blocks = (c + B - 1) / B;
-			const double m = B == 64 ? 1.25 * moved(B) : moved(B);
-			const double least = B == 64 ? 8.0 : B == 128 ? 9.6 : 15.8;
-			const double once = dots ? blocks * std::max(1, B / 128) * (60 + std::min(400.0, 0.0035 * h->N))
-			                         : 20.0 + 20.0 * blocks;
-			const double us = once + S * blocks * (dots ? std::max(least, 4.5 + m)
-			                                            : std::max(least - 0.5, 3.5 + m));
-			if (best == 0 || us < best) best = us;
-		}
-		return best;
-	};
-	double narrow = cols > rest ? wide(cols - rest) : 0.0;
-	for (int p = 0, left = rest; p < parts; p++) {
-		const int w = (left + parts - p - 1) / (parts - p);
-		const double m = moved(w);
-		left -= w;
-		narrow += dots ? 72 + S * (std::max(6.8 + 0.65 * m, 4 + m) + (w == 1 ? 3.0 : 0.0))
-		               : 60 + S * std::max(4.2 + 0.5 * m, 2 + 0.8 * m);
+double moved_us(const tbtkx_context *h, int w) { return (double)h->N * (12 * h->ell_W + 24 * w) / 4.4e6; }
+double wide_us(const tbtkx_context *h, int cols, int S, bool dots) {
+	double best = 0;
+	for (int B : {64, 128, 256}) {
+		if (B == 256 && cols <= 192) continue;   // never chosen for fewer
+		const int blocks = (cols + B - 1) / B;
+		const double m = B == 64 ? 1.25 * moved_us(h, B) : moved_us(h, B);
+		const double least = B == 64 ? 8.0 : B == 128 ? 9.6 : 15.8;
+		const double once = dots ? blocks * std::max(1, B / 128) * (60 + std::min(400.0, 0.0035 * h->N))
+		                         : 20.0 + 20.0 * blocks;
+		const double us = once + (double)S * blocks * (dots ? std::max(least, 4.5 + m)
+		                                                    : std::max(least - 0.5, 3.5 + m));
+		if (best == 0 || us < best) best = us;
 	}
-	return narrow < wide(cols);
+	return best;
+}
+double narrow_us(const tbtkx_context *h, int cols, int parts, int S, bool dots) {
+	double us = 0;
+	for (int p = 0, left = cols; p < parts; p++) {
+		const int w = (left + parts - p - 1) / (parts - p);
+		const double m = moved_us(h, w);
+		left -= w;
+		us += dots ? 72 + S * (std::max(6.8 + 0.65 * m, 4 + m) + (w == 1 ? 3.0 : 0.0))
+		           : 60 + S * std::max(4.2 + 0.5 * m, 2 + 0.8 * m);
+	}
+	return us;
+}
+
+// How a block's columns run: full blocks, then `rest` columns in `parts` narrow
+// blocks of `w` (parts = 0: none); and the time of it.
+struct Split {
+	int rest, parts, w;
+	double us;
+};
+Split split_columns(const tbtkx_context *h, int flags, int cols, int S) {
+	const bool dots = (flags & TBTKX_DOUBLING) != 0;
+	Split s{0, 0, 0, wide_us(h, cols, S, dots)};
+	const int rest = cols % 128, parts = rest > 64 ? 2 : 1, w = (rest + parts - 1) / parts;
+	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w)) return s;
+	const double us =
+	    narrow_us(h, rest, parts, S, dots) + (cols > rest ? wide_us(h, cols - rest, S, dots) : 0.0);
+	return us < s.us ? Split{rest, parts, w, us} : s;
 }
 
 int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
@@ -1646,12 +1662,14 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 	// Unit start vectors on a real H: two real vectors per complex column.
 	const int packed = mode == 0 && h->real_path && h->h_real;
 	const int per = packed ? 2 : 1, cols = (total + per - 1) / per;
+	const int S = (flags & TBTKX_DOUBLING) ? (M + 1) / 2 : M - 1;
+	const Split split = split_columns(h, flags, cols, S);
 	if (h->use_resident && h->real_path && h->h_real && narrow_fits(h, flags, 1)) {
 		const int real_cols = mode == 0 ? total : 2 * total;
 		const int64_t zero = 0;
 		BlockCall c{1, h->ell_col.as<uint32_t>(), h->ell_v2f.as<double>(), &h->N, &zero, &h->band,
 		            &h->ell_W, h->csr_gen, true, &real_cols, mode == 0 ? sites : nullptr, mode != 0,
-		            seed, &M, (flags & TBTKX_DOUBLING) != 0};
+		            seed, &M, (flags & TBTKX_DOUBLING) != 0, split.us};
 		bool done = false;
 		mu.resize((size_t)total * M);
 		if ((rc = resident_block(h, c, reinterpret_cast<double *>(mu.data()), &done))) return rc;
@@ -1664,13 +1682,8 @@ int block_entry(tbtkx_context *h, int total, const int64_t *sites, int mode,
 		}
 		mu.clear();
 	}
-	const int rest = cols % 128;
-	const int parts = rest > 64 ? 2 : 1, w = (rest + parts - 1) / parts;
-	const bool dots = (flags & TBTKX_DOUBLING) != 0;
-	if (rest == 0 || rest > kNarrowRest || !narrow_fits(h, flags, w) ||
-	    !narrow_pays(h, cols, rest, parts, dots ? (M + 1) / 2 : M - 1, dots))
-		return wide_entry(h, total, sites, mode, seed, M, flags, mu);
-	const int wide = (cols - rest) * per;
+	if (split.parts == 0) return wide_entry(h, total, sites, mode, seed, M, flags, mu);
+	const int w = split.w, wide = (cols - split.rest) * per;
 	mu.clear();
 	double ms = 0;
 	int64_t launches = 0;

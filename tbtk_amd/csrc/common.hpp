@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstdint>
@@ -102,6 +103,14 @@ struct TunedShape {
 	int g = 0, share = 0;
 };
 
+// Tiles and teams of the resident blocks (resident_block.hip): Gt workgroups per
+// team with tiles of A layers x B rows, `rounds` of 512 rows; us: a step of all passes,
+// 0: the model doesn't fit.
+struct BlockShape {
+	int L = 0, hq = 0, ds = 0, A = 0, B = 0, Gt = 0, teams = 0, passes = 0, rounds = 0;
+	double us = 0;
+};
+
 // The plain recurrence in one launch, the vectors resident on the chip
 // (resident.hip): C rows per workgroup (the whole model: one workgroup per start
 // vector), else G tiles of A layers x B rows with k steps between exchanges;
@@ -196,6 +205,7 @@ struct tbtkx_context {
 	struct BlockForms {
 		int64_t gen = -1;
 		std::vector<int> ne, layer, reach;   // per model; ne 0: not for this path
+		std::map<std::pair<int, int>, tbtkx::BlockShape> shapes;   // by model and columns
 		tbtkx::DevBuf scan;
 	} rb_single, rb_multi;
 	tbtkx::DevBuf rb_sites, rb_part, rb_D;
@@ -423,6 +433,7 @@ struct BlockCall {
 	uint64_t seed;
 	const int *M;
 	bool doubling;
+	double theirs;       // us of the call in the step kernels
 };
 int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done);
 

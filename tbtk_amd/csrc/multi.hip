@@ -1317,6 +1317,23 @@ struct SingleModel {
 	}
 };
 
+// The time in us of a batch of real models in the step kernels: 12 bytes per entry
+// and 24 per column element at 4.4 TB/s, at least a launch (and with dots a share of
+// two reductions) per step of the longest model. Model and measured: 8 models of
+// 10,000 to 24,000 rows, 64 sites, 109 steps gathered 2300 2000; one of 90,000 rows,
+// 20 sites, 39 steps gathered 320 300; 3 models of 900 to 360,000 rows, 64 sites, 2 to 12
+// steps with dots 470 524.
+double batch_us(const tbtkx_context *h, const int *num_sites, const int *num_moments, bool dots) {
+	double moved = 0;
+	int longest = 0;
+	for (int m = 0; m < h->mm_K; m++) {
+		const int S = dots ? (num_moments[m] + 1) / 2 : num_moments[m] - 1;
+		moved += (double)S * h->mm_N[m] * (12 * h->mm_Wm[m] + 24 * ((num_sites[m] + 1) / 2)) / 4.4e6;
+		longest = std::max(longest, S);
+	}
+	return 70 + std::max(moved, (dots ? 6.5 : 4.2) * longest);
+}
+
 }  // namespace
 
 bool narrow_fits(const tbtkx_context *h, int flags, int cols) {
@@ -1512,7 +1529,8 @@ int tbtkx_multi_moments(tbtkx_handle h, const int *num_sites, const int64_t *sit
 		if (rc) return rc;
 		BlockCall c{K, h->mm_ecol.as<uint32_t>(), h->mm_ev2.as<double>(), h->mm_N.data(),
 		            h->mm_e0.data(), h->mm_band.data(), h->mm_Wm.data(), h->mm_gen, false, num_sites,
-		            sites, false, 0, num_moments, (flags & TBTKX_DOUBLING) != 0};
+		            sites, false, 0, num_moments, (flags & TBTKX_DOUBLING) != 0,
+		            batch_us(h, num_sites, num_moments, (flags & TBTKX_DOUBLING) != 0)};
 		bool done = false;
 		if ((rc = resident_block(h, c, out, &done))) return rc;
 		if (done) {

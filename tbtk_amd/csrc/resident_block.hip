@@ -467,14 +467,17 @@ __global__ __launch_bounds__(kThreads) void block_dots(const double *__restrict_
 }
 
 // Times in us of the rule in resident_block: a step of one round of 512 rows with
-// one entry beside the diagonal, a launch; the share of the streamed time to beat.
+// one entry beside the diagonal; a call, a cooperative launch, a launch's setup per
+// round (entries and codes), the sum of its dots per workgroup of a team; and
+// the share of the step kernels' time to beat. Model and measured, whole calls: 1,024,000
+// states, 64 columns in 8 passes, 2 steps gathered 520 509, 4 with dots 1270 1290; 159,520
+// states, 37 columns, 30 steps with dots 350 343; 1800 states, 64 columns, 20 steps
+// with dots 137 116.
 constexpr double kRound = 0.11, kStep = 0.6;
-constexpr double kLeastStep = kStep + kRound * (1 + 2), kPerLaunch = 20.0, kWorth = 0.9;
+constexpr double kLeastStep = kStep + kRound * (1 + 2);
+constexpr double kCall = 50, kLaunch = 17, kSetup = 3, kSumDots = 0.3, kWorth = 0.9;
 
-struct Shape {
-	int L = 0, hq = 0, ds = 0, A = 0, B = 0, Gt = 0, teams = 0, passes = 0, rows = 0;
-	double us = 0;   // a step of all passes
-};
+typedef BlockShape Shape;
 
 // The tiles and teams of the least time for V columns of a model; us = 0: none.
 // Time of a step in us: rounds of 512 rows, the ring's bytes and its passes; model
@@ -503,7 +506,7 @@ Shape shape_of(int64_t N, int ne, int layer, int reach, int64_t band, int V, int
 			best.L = (int)L, best.hq = (int)hq, best.ds = (int)ds;
 			best.A = (int)A, best.B = (int)B, best.Gt = (int)Gt;
 			best.teams = (int)teams, best.passes = (int)passes;
-			best.rows = (int)((own + kT - 1) / kT);
+			best.rounds = (int)((own + kT - 1) / kT);
 			best.us = us;
 		}
 	};
@@ -545,6 +548,7 @@ int scan_models(tbtkx_context *h, const BlockCall &c, tbtkx_context::BlockForms 
 	if (f.gen == c.gen && (int)f.ne.size() == c.K) return TBTKX_OK;
 	int rc;
 	f.gen = -1;
+	f.shapes.clear();
 	const size_t at = (size_t)c.K * sizeof(Scan);
 	if ((rc = f.scan.reserve(at + (size_t)c.K * sizeof(ScanModel)))) return rc;
 	std::vector<ScanModel> sm(c.K);
@@ -582,26 +586,22 @@ int scan_models(tbtkx_context *h, const BlockCall &c, tbtkx_context::BlockForms 
 
 int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done) {
 	*done = false;
-	// Against the streamed step: 12 bytes per column element at 4.4 TB/s (1,048,576
-	// states x 256 columns: 732 us, measured 711), at least 5 us per launch; models of a
-	// batch share its launches. Wide rings lose: 864,000 states (96 x 100 x 90), 64
-	// columns, a ring of 4000 of 3800 rows, 270 us a step against 173.
+	// Against the step kernels. Wide rings lose: 864,000 states (96 x 100 x 90), 64
+	// columns, a ring of 4000 of 3800 rows, 270 us a step against 173; and so do many passes
+	// of few steps: 1,024,000 states, 64 columns in 8 passes, 4 steps with dots 1287 us
+	// against 833, 10 steps 1668 against 1920.
 	int64_t vectors = 0;
 	std::vector<int> S(c.K);
-	double theirs = 0, least = 0;
-	int Smax = 0;
+	double least = kCall;
 	for (int m = 0; m < c.K; m++) {
 		S[m] = c.doubling ? (c.M[m] + 1) / 2 : c.M[m] - 1;
 		if (S[m] < 1) return TBTKX_OK;
 		vectors += c.cols[m];
-		theirs += (double)c.N[m] * c.cols[m] * 12 / 4.4e6 * S[m];
-		least += kLeastStep * S[m] + kPerLaunch;
-		Smax = std::max(Smax, S[m]);
+		least += kLeastStep * S[m] + kLaunch + kSetup;
 	}
-	theirs = std::max(theirs, 5.0 * Smax);
 	// A launch per model and its shortest steps cost more already: no scan, which
 	// takes 10 KB and some 50 us of the host per model (a batch of 1000 small models).
-	if (least > kWorth * theirs) return TBTKX_OK;
+	if (least > kWorth * c.theirs) return TBTKX_OK;
 	int rc;
 	if (!cooperative_now(h)) return TBTKX_OK;
 	// No memory for this path's own scratch: the step kernels need what it holds.
@@ -613,17 +613,25 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 	tbtkx_context::BlockForms &f = c.single ? h->rb_single : h->rb_multi;
 	if ((rc = scan_models(h, c, f))) return rc == TBTKX_ERR_OOM ? no_memory() : rc;
 	std::vector<Shape> sh(c.K);
-	double mine = 0;
+	double mine = kCall;
 	int64_t steps = 0;
 	for (int m = 0; m < c.K; m++) {
 		if (!f.ne[m]) return TBTKX_OK;
-		sh[m] = shape_of(c.N[m], f.ne[m], f.layer[m], f.reach[m], c.band[m], c.cols[m], h->num_cus);
+		const auto key = std::make_pair(m, c.cols[m]);
+		auto known = f.shapes.find(key);
+		if (known == f.shapes.end()) {
+			if (f.shapes.size() >= 4096) f.shapes.clear();
+			known = f.shapes.emplace(key, shape_of(c.N[m], f.ne[m], f.layer[m], f.reach[m], c.band[m],
+			                                       c.cols[m], h->num_cus)).first;
+		}
+		sh[m] = known->second;
 		if (sh[m].us == 0) return TBTKX_OK;
 		// Dots of complex vectors: 12.8 us where the model gives 9.4.
 		steps += (int64_t)S[m] * sh[m].passes;
-		mine += sh[m].us * (c.phases ? 1.35 : 1.0) * S[m] + kPerLaunch * sh[m].passes;
+		mine += sh[m].us * (c.phases ? 1.35 : 1.0) * S[m] +
+		        sh[m].passes * (kLaunch + kSetup * sh[m].rounds + (c.doubling ? kSumDots * sh[m].Gt : 0.0));
 	}
-	if (mine > kWorth * theirs) return TBTKX_OK;
+	if (mine > kWorth * c.theirs) return TBTKX_OK;
 
 	size_t part = 0, D = 0, xg = 0, mu = 0;
 	uint32_t phases = 0;
@@ -682,9 +690,9 @@ int resident_block(tbtkx_context *h, const BlockCall &c, double *out, bool *done
 		a.xg = h->res_xg.ptr;
 		a.xg_bytes = (uint32_t)xg;
 		a.err = h->res_err.as<uint32_t>();
-		const void *k = c.phases      ? kernel_of<2>(f.ne[m], s.rows)
-		                : c.doubling ? kernel_of<1>(f.ne[m], s.rows)
-		                             : kernel_of<0>(f.ne[m], s.rows);
+		const void *k = c.phases      ? kernel_of<2>(f.ne[m], s.rounds)
+		                : c.doubling ? kernel_of<1>(f.ne[m], s.rounds)
+		                             : kernel_of<0>(f.ne[m], s.rounds);
 		for (int p = 0; p < s.passes; p++) {
 			a.col0 = p * s.teams * kCols;
 			const int left = (c.cols[m] - a.col0 + kCols - 1) / kCols, teams = std::min(s.teams, left);

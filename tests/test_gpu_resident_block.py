@@ -132,7 +132,7 @@ def sides(eng, call):
 
 
 MANY = ((41, 0), (64, X.DOUBLING), (63, X.DOUBLING))
-FEW = ((3, 0), (3, X.DOUBLING), (4, X.DOUBLING))   # two steps: fewer never pay
+FEW = ((3, 0), (3, X.DOUBLING), (4, X.DOUBLING))   # two steps
 
 
 @pytest.mark.parametrize("name,n,cols,moments", [
@@ -141,7 +141,7 @@ FEW = ((3, 0), (3, X.DOUBLING), (4, X.DOUBLING))   # two steps: fewer never pay
     ("nambu", (120, 131), 100, MANY), ("honeycomb", (40, 997), 37, MANY),
     ("spin", (520, 530), 16, MANY), ("honeycomb", (500, 500), 9, MANY),
     ("honeycomb", (32, 32), 2048, FEW), ("nambu", (32, 32), 2048, FEW),
-    ("square", (63, 65), 2041, FEW), ("spin", (1024, 500), 16, FEW)])
+    ("square", (63, 65), 2041, FEW), ("spin", (1024, 500), 16, ((11, 0), (21, X.DOUBLING)))])
 def test_blocks_that_run_resident(res, name, n, cols, moments):
     """One workgroup, tiles of few and of all rows per thread, one and two passes,
     many steps and two."""
@@ -182,3 +182,16 @@ def test_which_matrices_run_resident(res):
         res.set_csr(csr, 4.0)
         res.moments_block([0, 5, n // 2, n - 1], 60, X.DOUBLING)
         assert res.get_option(X.OPT_RESIDENT) == ran
+
+
+def test_calls_that_would_lose_keep_the_steps(res):
+    """Eight passes of four steps with dots, and a batch whose steps are fewer than
+    its launches are worth."""
+    m, s = model("spin", (1024, 500))
+    res.set_csr(m.csr(), s)
+    res.moments_block(np.arange(64), 8, X.DOUBLING)
+    assert res.get_option(X.OPT_RESIDENT) == 0
+    specs = [L.square_spec(*z, disorder=0.5, seed=i) for i, z in enumerate([(600, 600), (500, 400), (30, 30)])]
+    res.multi_set_lattices(specs, [5.0] * 3)
+    res.multi_moments([np.arange(64)] * 3, [3, 13, 23], X.DOUBLING)
+    assert res.get_option(X.OPT_RESIDENT) == 0
