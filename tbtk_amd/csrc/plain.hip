@@ -1126,8 +1126,9 @@ extern "C" int tbtkx_moments(tbtkx_handle h, int64_t from, int K,
 	const PlainForm pform = plain_form(h);
 	const bool c16 = pform.c16, usepal = pform.pal;
 	std::vector<double> dense((size_t)U * M * 2);
+	// The first moment needs no step: 39 us a call, 72-90 through a cooperative launch.
 	const ResidentPlan plan = resident_plan(h, h->num_cus);
-	bool resident = plan.C > 0;
+	bool resident = plan.C > 0 && (plan.G == 1 || M > 1);
 	if (resident) {
 		const int toff[2] = {0, U};
 		TBTKX_CHECK_HIP(hipEventRecord(h->ev_start, h->stream));

@@ -98,3 +98,12 @@ def test_shape_of_a_resident_batch(eng):
         assert eng.get_option(X.OPT_RESIDENT) == resident
         assert (eng.get_option(X.OPT_TILE_ROWS) == 0) == bool(resident)
     assert eng.get_option(X.OPT_GRID_SHARE) == 0
+
+
+def test_first_moment_alone_takes_no_cooperative_launch(eng):
+    m = L.square_spin(173, 61, disorder=0.5, seed=2)
+    eng.set_csr(m.csr(), 6.0)
+    assert np.array_equal(eng.moments(7, [3, 7], 1)[:, 0], [0, 1])
+    assert eng.get_option(X.OPT_RESIDENT) == 0
+    eng.moments(7, [3, 7], 20)
+    assert eng.get_option(X.OPT_RESIDENT) == 1
