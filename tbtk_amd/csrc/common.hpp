@@ -166,6 +166,7 @@ struct tbtkx_context {
 	// slot_W slots per row, 16-bit column offsets from the row, palette codes
 	// (slot_pal) or H/s, 2H/s values (complex, and real for a real H).
 	tbtkx::DevBuf scol, scode, sv1, sv2, sv1r, sv2r;
+	tbtkx::DevBuf offset_scan;
 	int slot_ok = 0, slot_pal = 0, slot_vals = 0, slot_W = 0;
 	int slot_half = 0;   // most entries on either side of a row's diagonal
 	// Rows per layer of the slot form's lattice view and the farthest column
@@ -319,7 +320,7 @@ int build_col16(tbtkx_context *h);
 
 // Builds the slot-major ELL form of the plain kernel from the resident CSR
 // and palette (plain.hip); `rowptr` is a host copy of the row pointer.
-int build_slots(tbtkx_context *h, const uint32_t *rowptr, const uint32_t *col);
+int build_slots(tbtkx_context *h, const uint32_t *rowptr);
 // Adds H/s and 2H/s values to the slots (for calls without the palette).
 int build_slot_values(tbtkx_context *h);
 // Builds the palette, the row patterns and the slot form of a device-built

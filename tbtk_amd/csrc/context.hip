@@ -200,7 +200,7 @@ int tbtkx_destroy(tbtkx_handle h) {
 	for (DevBuf *b : {&h->rowptr, &h->col, &h->v1, &h->v2, &h->v1f, &h->v2f,
 	                  &h->v1r, &h->v2r, &h->lat_terms, &h->lat_onsite, &h->lat_count,
 	                  &h->lat_part, &h->lat_tmp, &h->rblk, &h->col16, &h->col16_flag,
-	                  &h->pcode, &h->pal, &h->palr, &h->pdiag, &h->pdiagr, &h->scol, &h->scode, &h->sv1, &h->sv2, &h->sv1r, &h->sv2r, &h->ppid, &h->ptoff, &h->ptcode, &h->pchunk, &h->vec_a, &h->vec_b, &h->coef, &h->to,
+	                  &h->pcode, &h->pal, &h->palr, &h->pdiag, &h->pdiagr, &h->scol, &h->offset_scan, &h->scode, &h->sv1, &h->sv2, &h->sv1r, &h->sv2r, &h->ppid, &h->ptoff, &h->ptcode, &h->pchunk, &h->vec_a, &h->vec_b, &h->coef, &h->to,
 	                  &h->res_in, &h->res_xg, &h->res_err,
 	                  &h->lut, &h->gf_in, &h->gf_out, &h->dfac, &h->dden, &h->blk_x, &h->blk_y,
 	                  &h->blk_mu, &h->blk_sites, &h->blk_part, &h->blk_grow, &h->blk_gvec, &h->cplanes,
@@ -371,7 +371,7 @@ int tbtkx_set_csr(tbtkx_handle h, int64_t N, int64_t Z, const uint32_t *rowptr,
 	if ((rc = build_col16(h))) return rc;
 	h->forms_pending = 0;
 	if ((rc = build_palette(h, N, Z, rowptr, col, v1.data(), v2.data()))) return rc;
-	return build_slots(h, rowptr, col);
+	return build_slots(h, rowptr);
 }
 
 int tbtkx_last_timing(tbtkx_handle h, double *ms, int64_t *launches) {

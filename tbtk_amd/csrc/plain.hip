@@ -650,34 +650,82 @@ void layer_stride(int64_t N, const std::vector<uint8_t> &seen, int *layer, int *
 	}
 }
 
-int build_slots(tbtkx_context *h, const uint32_t *rowptr, const uint32_t *col) {
+// The column offsets that occur (bit offset + 32768 of seen, those that fit) and the
+// most entries on either side of a row's first diagonal entry.
+struct OffsetScan {
+	uint32_t seen[2048], half;
+};
+static __global__ __launch_bounds__(kThreads) void offset_scan(const uint32_t *__restrict__ rowptr,
+                                                               const uint32_t *__restrict__ col,
+                                                               int64_t N, OffsetScan *out) {
+	__shared__ uint32_t seen[2048], half;
+	for (int i = threadIdx.x; i < 2048; i += kThreads) seen[i] = 0;
+	if (threadIdx.x == 0) half = 0;
+	__syncthreads();
+	uint32_t most = 0;
+	for (int64_t r = (int64_t)blockIdx.x * kThreads + threadIdx.x; r < N;
+	     r += (int64_t)gridDim.x * kThreads) {
+		uint32_t before = 0, after = 0;
+		bool diag = false;
+		for (uint32_t k = rowptr[r]; k < rowptr[r + 1]; k++) {
+			const int64_t d = (int64_t)col[k] - r;
+			if (d == 0 && !diag) diag = true;
+			else if (diag) after++;
+			else before++;
+			if (d < -32768 || d > 32767) continue;
+			const uint32_t o = (uint32_t)(d + 32768), bit = 1u << (o & 31);
+			if (!(*(volatile uint32_t *)&seen[o >> 5] & bit)) atomicOr(&seen[o >> 5], bit);
+		}
+		const uint32_t m = before > after ? before : after;
+		most = m > most ? m : most;
+	}
+	if (most) atomicMax(&half, most);
+	__syncthreads();
+	for (int i = threadIdx.x; i < 2048; i += kThreads)
+		if (seen[i]) atomicOr(&out->seen[i], seen[i]);
+	if (threadIdx.x == 0) atomicMax(&out->half, half);
+}
+static __global__ __launch_bounds__(kThreads) void offset_scan_clear(OffsetScan *out) {
+	for (int i = threadIdx.x; i < 2048; i += kThreads) out->seen[i] = 0;
+	if (threadIdx.x == 0) out->half = 0;
+}
+
+// offset_scan of the resident CSR; seen[offset + 32768]. A loop over the host's CSR
+// took 1 to 5% of tbtkx_set_csr.
+static int scan_offsets(tbtkx_context *h, std::vector<uint8_t> &seen, int *half) {
+	int rc;
+	if ((rc = h->offset_scan.reserve(sizeof(OffsetScan)))) return rc;
+	OffsetScan *dev = h->offset_scan.as<OffsetScan>(), host;
+	offset_scan_clear<<<1, kThreads, 0, h->stream>>>(dev);
+	offset_scan<<<(unsigned)std::min<int64_t>(1024, (h->N + kThreads - 1) / kThreads), kThreads, 0,
+	              h->stream>>>(h->rowptr.as<uint32_t>(), h->col.as<uint32_t>(), h->N, dev);
+	TBTKX_CHECK_HIP(hipGetLastError());
+	TBTKX_CHECK_HIP(hipMemcpyAsync(&host, dev, sizeof host, hipMemcpyDeviceToHost, h->stream));
+	TBTKX_CHECK_HIP(hipStreamSynchronize(h->stream));
+	seen.resize(65536);
+	for (int o = 0; o < 65536; o++) seen[o] = host.seen[o >> 5] >> (o & 31) & 1;
+	*half = (int)host.half;
+	return TBTKX_OK;
+}
+
+int build_slots(tbtkx_context *h, const uint32_t *rowptr) {
 	h->tile_L = h->tile_ds = 0;
 	h->slot_ok = 0;
 	h->slot_pal = 0;
 	h->slot_vals = 0;
 	h->slot_W = 0;
 	int64_t maxrow = 0;
-	int half = 0;
-	std::vector<uint8_t> seen(65536, 0);   // column offsets of the matrix, + 32768
-	for (int64_t r = 0; r < h->N; r++) {
-		int before = 0, after = 0;
-		bool diag = false;
-		for (uint32_t k = rowptr[r]; k < rowptr[r + 1]; k++) {
-			const int64_t d = (int64_t)col[k] - r + 32768;
-			if (d >= 0 && d < 65536) seen[(size_t)d] = 1;
-			if ((int64_t)col[k] == r && !diag) diag = true;
-			else ++(diag ? after : before);
-		}
+	for (int64_t r = 0; r < h->N; r++)
 		maxrow = std::max<int64_t>(maxrow, rowptr[r + 1] - rowptr[r]);
-		half = std::max(half, std::max(before, after));
-	}
 	if (h->N <= 0 || maxrow > 8) return TBTKX_OK;
+	int rc;
+	std::vector<uint8_t> seen;
+	if ((rc = scan_offsets(h, seen, &h->slot_half))) return rc;
 	h->slot_W = maxrow < 4 ? 4 : (int)maxrow;
-	h->slot_half = half;
 	h->slot_ok = 1;
 	layer_stride(h->N, seen, &h->tile_L, &h->tile_ds);
 	const bool pal = h->palette_ok != 0;
-	int rc = make_slot_arrays(h, pal, !pal);
+	rc = make_slot_arrays(h, pal, !pal);
 	if (rc || !h->slot_ok) return rc;
 	h->slot_pal = pal;
 	h->slot_vals = !pal;
@@ -698,7 +746,7 @@ int build_plain_forms(tbtkx_context *h) {
 	}
 	int rc = build_palette(h, N, Z, hrp.data(), hcol.data(), hv1.data(), hv2.data());
 	if (rc) return rc;
-	if ((rc = build_slots(h, hrp.data(), hcol.data()))) return rc;
+	if ((rc = build_slots(h, hrp.data()))) return rc;
 	h->forms_pending = 0;
 	return TBTKX_OK;
 }
