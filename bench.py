@@ -25,7 +25,7 @@ of the same workload on this host, on one core and in one process per core
 (the throughput mode), with the GPU/CPU ratios beside it.
 
 Further objects on the same line: "uneven_batch" (64 models of uneven size
-in one launch per step), "stochastic_dos" (128^3 cubic, 512
+in one call), "stochastic_dos" (128^3 cubic, 512
 random-phase vectors, M=4096) and "contraction_mfma" (1e5 x 4096 x 8192
 split-BF16 Green's-function GEMM), each with its own roofline fraction and
 error against the FP64 path.
@@ -58,6 +58,7 @@ from tbtk_amd import lattice as L  # noqa: E402
 
 METRIC = "LDOS sites/s + SpMV GB/s, batched FP32 vs plain FP64 at fixed error"
 HBM_PEAK_GBPS = 8000.0
+LDS_PEAK_GBPS = 256 * 128 * 2.4   # 256 CUs x 128 B a cycle at 2.4 GHz
 BF16_PEAK_TFLOPS = 2500.0
 
 # Default workload
@@ -321,6 +322,7 @@ def batched_comparison(eng):
     t0 = time.perf_counter()
     mu = eng.moments_block(sites, M_BATCH, X.DOUBLING)
     ms_rec, launches = eng.last_timing()
+    resident = eng.get_option(X.OPT_RESIDENT) == 1
     ld_batched = contract(mu)
     t_batched = time.perf_counter() - t0
 
@@ -335,6 +337,7 @@ def batched_comparison(eng):
         plain_ms += eng.last_timing()[0]
         ref.append(c[0])
     plain_bytes, plain_form = plain_step_bytes(eng, N, Z)
+    plain_resident = eng.get_option(X.OPT_RESIDENT) == 1
     ld_plain = contract(np.array(ref))
     t_plain = (time.perf_counter() - t0) / PLAIN_CMP_SITES
 
@@ -346,8 +349,24 @@ def batched_comparison(eng):
     shape = {"block_width": B, "strip_rows": eng.get_option(X.OPT_STRIP_ROWS),
              "grid_share": eng.get_option(X.OPT_GRID_SHARE),
              "rows_in_flight_x": eng.get_option(X.OPT_ROWS_IN_FLIGHT)}
-    step_bytes = 12 * Z + 4 * N + 24 * B * N
-    per_step = ms_rec * 1e-3 / launches
+    # Steps of full blocks stream H and three blocks of vectors. Resident, a step of
+    # all columns reads a value per entry and column from LDS, and the vector
+    # two steps back, and writes one; nothing streams from HBM.
+    if resident:
+        steps = (M_BATCH + 1) // 2
+        per_step = ms_rec * 1e-3 / steps
+        step_bytes = 4 * B_SITES * (Z + 2 * N)
+        rate = {"spmm_GBps": None, "spmm_hbm_frac": None,
+                "spmm_lds_GBps": step_bytes / per_step / 1e9,
+                "spmm_lds_frac": step_bytes / per_step / 1e9 / LDS_PEAK_GBPS,
+                "spmm_launches": launches // steps}
+    else:
+        per_step = ms_rec * 1e-3 / launches
+        step_bytes = 12 * Z + 4 * N + 24 * B * N
+        rate = {"spmm_GBps": step_bytes / per_step / 1e9,
+                "spmm_hbm_frac": step_bytes / per_step / 1e9 / HBM_PEAK_GBPS,
+                "spmm_block_width": B, "vectors_per_block": 2 * B if packed else B,
+                "spmm_shape": shape}
     sps_b = B_SITES / t_batched
     sps_p = 1.0 / t_plain
     return {
@@ -365,18 +384,17 @@ def batched_comparison(eng):
         "batched_dtype": ("fp32 vectors; real H as one fp64 value per 8-byte entry, fp64 row "
                           "sums; fp64 moments, doubling"
                           + (", real H: two real vectors per complex column" if packed else "")),
-        "spmm_block_width": B,
-        "vectors_per_block": 2 * B if packed else B,
-        "spmm_shape": shape,
+        "spmm_path": ("resident: all steps of 8 columns per team of workgroups in one launch"
+                      if resident else "a launch per step and block"),
         "spmm_step_ms": per_step * 1e3,
-        "spmm_GBps": step_bytes / per_step / 1e9,
-        "spmm_hbm_frac": step_bytes / per_step / 1e9 / HBM_PEAK_GBPS,
+        **rate,
+        "plain_path": "resident" if plain_resident else "a launch per step",
         "plain_arithmetic": "real fp64" if plain_real else "complex fp64",
         "plain_form": ("slot-major, wave-uniform row patterns" if plain_form["uniform"] else
                        "slot-major, row patterns" if plain_form["patterns"] else
                        "slot-major" if plain_form["slot"] else "row blocks"),
         "plain_step_us": plain_ms * 1e3 / (PLAIN_CMP_SITES * (M_BATCH - 1)),
-        "plain_spmv_GBps": plain_bytes
+        "plain_spmv_GBps": None if plain_resident else plain_bytes
         / (plain_ms * 1e-3 / (PLAIN_CMP_SITES * (M_BATCH - 1))) / 1e9,
     }
 
@@ -384,8 +402,10 @@ def batched_comparison(eng):
 def uneven_batch(eng, graph=True, moments_div=1, tile_rows=0, grid_share=0):
     """64 independent models of uneven size (honeycomb ribbons and square
     lattices, 20k-1M states, 1-64 sites and 500-8000 moments each, seed 4) in
-    one launch per recurrence step: FP32 storage, FP64 moments,
-    doubling, autotuned launch shape, replayed as hipGraphs. The models
+    one call: FP32 storage, FP64 moments, doubling. Timed: the default call
+    (resident where that is faster), and the step kernels replayed as
+    hipGraphs (one launch per recurrence step, autotuned shape), whose rate is
+    the streamed one. The models
     are built on the device from their lattice descriptions
     (tbtkx_multi_set_lattices). For counter runs, moments_div > 1 divides
     every model's moment count (at least 50: the same phases, a tenth of the
@@ -413,29 +433,36 @@ def uneven_batch(eng, graph=True, moments_div=1, tile_rows=0, grid_share=0):
     # rounded up to a kernel width: 4, 5, 6 or 8)
     W = np.array([min(w for w in (4, 5, 6, 8) if w >= sp.max_row_entries()) for sp in specs],
                  dtype=np.int64)
-    # 1: autotune + direct launches; 2: hipGraph capture; 3: graph replay (timed)
+    # 1: first call; 2: the default call again (timed); 3: hipGraph capture (with
+    # the autotuner); 4: graph replay (timed)
     t0 = time.perf_counter()
     mu = eng.multi_moments(sites, Ms, X.DOUBLING)
     t_first = time.perf_counter() - t0
+    t0 = time.perf_counter()
+    mu = eng.multi_moments(sites, Ms, X.DOUBLING)
+    t_direct = time.perf_counter() - t0
     ms_direct, launches = eng.last_timing()
-    shape = {"tile_row_groups": eng.get_option(X.OPT_TILE_ROWS),
-             "grid_share": eng.get_option(X.OPT_GRID_SHARE)}
+    resident = eng.get_option(X.OPT_RESIDENT) == 1
     # complex columns per model: two real vectors per column for a real batch
     packed = eng.get_option(X.OPT_REAL) == 1
     cols = (B + 1) // 2 if packed else B
     step_bytes_total = float(((12 * W * N + 24 * cols * N) * S).sum())
-    # graph=False (--no-graph): a second direct run is timed instead of the
-    # graph replay (for profilers that do not follow graph launches)
+    # graph=False (--no-graph): a direct run of the step kernels is timed instead
+    # of the graph replay (for profilers that do not follow graph launches)
     eng.set_option(X.OPT_GRAPH, 1 if graph else 0)
+    eng.set_option(X.OPT_RESIDENT, 0)
     try:
         if graph:
             eng.multi_moments(sites, Ms, X.DOUBLING)
         t0 = time.perf_counter()
         mu_g = eng.multi_moments(sites, Ms, X.DOUBLING)
         t_graph = time.perf_counter() - t0
-        ms_graph, _ = eng.last_timing()
+        ms_graph, steps = eng.last_timing()
+        shape = {"tile_row_groups": eng.get_option(X.OPT_TILE_ROWS),
+                 "grid_share": eng.get_option(X.OPT_GRID_SHARE)}
     finally:
         eng.set_option(X.OPT_GRAPH, 0)
+        eng.set_option(X.OPT_RESIDENT, 1)
     graph_diff = max(float(np.abs(a - b).max()) for a, b in zip(mu, mu_g))
     # error against the plain FP64 path: the two smallest and the two
     # largest models, their first and last sites
@@ -471,17 +498,21 @@ def uneven_batch(eng, graph=True, moments_div=1, tile_rows=0, grid_share=0):
         "dtype": ("fp32 vectors; real H as one fp64 value per 8-byte entry, fp64 row sums; "
                   "fp64 moments, doubling"
                   + (", real H: two real vectors per complex column" if packed else "")),
-        "timed_run": "hipGraph replay" if graph else "direct launches (--no-graph)",
-        "sites_per_s": float(B.sum()) / (t_graph),
-        "device_s": dev_s,
-        "direct_device_s": ms_direct * 1e-3,
-        "first_call_s_incl_autotune": t_first,
-        "graph_replay_wall_s": t_graph,
-        "step_launches": int(launches),
-        "algorithmic_bytes": step_bytes_total,
-        "GBps": step_bytes_total / dev_s / 1e9,
-        "hbm_frac": step_bytes_total / dev_s / 1e9 / HBM_PEAK_GBPS,
-        "graph_vs_direct_max_abs_diff": graph_diff,
+        "timed_run": "default call" + (", resident" if resident else ""),
+        "sites_per_s": float(B.sum()) / t_direct,
+        "wall_s": t_direct,
+        "device_s": ms_direct * 1e-3,
+        "first_call_s": t_first,
+        "steps": int(launches),
+        "streamed": {
+            "run": "hipGraph replay" if graph else "direct launches (--no-graph)",
+            "device_s": dev_s, "wall_s": t_graph, "steps": int(steps),
+            "sites_per_s": float(B.sum()) / t_graph,
+            "algorithmic_bytes": step_bytes_total,
+            "GBps": step_bytes_total / dev_s / 1e9,
+            "hbm_frac": step_bytes_total / dev_s / 1e9 / HBM_PEAK_GBPS,
+        },
+        "streamed_vs_default_max_abs_diff": graph_diff,
         "max_ldos_rel_err_vs_fp64": max(e[0] for e in errs),
         "max_ldos_pointwise_rel_err_vs_fp64": max(e[1] for e in errs),
         "error_sites_compared": len(errs),
@@ -745,12 +776,13 @@ def main():
         slot, patterns, uniform = form["slot"], form["patterns"], form["uniform"]
         byte_rows = form["byte_rows"]
         avg_kernel_s = kernel_ms * 1e-3 / launches
-        # All steps in one launch with the vectors on the chip: LDS bounds a step
-        # (per row 4 neighbours, 4 palette values and the row's own write).
+        # All steps in one launch with the vectors on the chip: a step's bytes are
+        # LDS bytes, four neighbours and the row's own write (the palette's values
+        # are broadcast).
         resident = eng.get_option(X.OPT_RESIDENT) == 1
-        peak = 256 * 128 * 2.4 if resident else HBM_PEAK_GBPS
+        peak = LDS_PEAK_GBPS if resident else HBM_PEAK_GBPS
         if resident:
-            step_bytes = 9 * (8 if real else 16) * N
+            step_bytes = 5 * (8 if real else 16) * N
         achieved = step_bytes / avg_kernel_s / 1e9
         dE = (WINDOW[1] - WINDOW[0]) / (E_PTS - 1)
         out.update({
@@ -775,6 +807,7 @@ def main():
             },
             "physical_sites_per_s": value / 2,
             "spmv_GBps": achieved,
+            "spmv_memory": "lds (the vectors stay on the chip)" if resident else "hbm",
             "roofline": {
                 "kernel": "resident_wide (all steps in one launch, vectors in LDS and "
                           "registers; per-step figures)" if resident else
@@ -817,7 +850,7 @@ def main():
         log("batched comparison (512x512 Nambu, 256 sites)")
         out["batched"] = batched_comparison(eng)
     if "uneven" in parts:
-        log("uneven batch (64 models, one launch per step)")
+        log("uneven batch (64 models)")
         out["uneven_batch"] = uneven_batch(eng, graph=not args.no_graph,
                                            moments_div=args.uneven_moments_div,
                                            tile_rows=args.uneven_tile_rows,
