@@ -454,7 +454,8 @@ __global__ __launch_bounds__(kResThreads) void resident_recurrence(ResArgs<S> a)
 // rows 2.7 us, where a launch per step took 11.9 (50 MB of vectors and 18 MB
 // of matrix from the cache beyond L2); 1,048,576 states (512 x 512 x 4) 1.9 us;
 // 864,000 states (96 x 100 x 90) 4.1 us, a frame of 2800 of 4000 rows there. Bound by
-// LDS reads (8 per row and step) and the exchange.
+// VALU issue (62% of the SIMDs' cycles at 2,097,152 states: 8 FP64 and 12 integer
+// instructions per row and step), the exchange, and LDS (busy 42% of the time).
 // Large models (palette only): up to 8192 real rows per workgroup, one step per
 // exchange. LDS holds one window of x_n, which is overwritten after a
 // barrier; a row's entries are 16-bit window elements and 8-bit palette codes in
