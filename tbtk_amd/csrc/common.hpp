@@ -101,6 +101,7 @@ struct GraphCache {
 struct TunedShape {
 	int64_t key[3] = {-1, -1, -1};
 	int g = 0, share = 0;
+	bool all = false;   // of every shape, not of the first few
 };
 
 // Tiles and teams of the resident blocks (resident_block.hip): Gt workgroups per

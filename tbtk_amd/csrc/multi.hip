@@ -1031,21 +1031,24 @@ int64_t run_steps(const Plan &p) {
 	return n;
 }
 
+constexpr int kLongRun = 128;   // steps of a run that repays trials of every shape
+
 // Autotuner: time a few steps of the first phase for each (tile groups, grid
 // share) candidate on the actual batch and keep the fastest: persistent grids
 // (share 1 or 2) with tiles of 2-16 row groups, and one tile per wavefront
-// (share 0) with tiles of 8-64 row groups. Narrow blocks: the first kNarrowCand,
-// whose best took at most 1.05 of the best of all 12 (8 models of 29,760 to 753,480
-// rows, 1 to 64 columns); two row groups per tile without trials where a step moves
+// (share 0) with tiles of 8-64 row groups. Narrow blocks of fewer than kLongRun steps:
+// the first kNarrowCand, whose best took at most 1.05 of the best of all 12 (8 models of
+// 29,760 to 753,480 rows, 1 to 64 columns; 864,000 rows, 32 columns, 256 steps: 45.5 ms
+// against 44.5, where the other trials take 6 ms once); two row groups per tile without trials where a step moves
 // less than an XCD's L2 holds (3600 to 29,760 rows: at most 1.08 of the best).
 int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<int> &S,
-             bool dots, int ncols, int64_t mu_elems, bool narrow, TunedShape &tuned) {
+             bool dots, int ncols, int64_t mu_elems, bool narrow, bool all, TunedShape &tuned) {
 	static const int kCand[][2] = {{1, 2}, {1, 4}, {1, 16}, {2, 2},  {2, 4},  {0, 8},
 	                               {1, 8}, {2, 8}, {2, 16}, {0, 16}, {0, 32}, {0, 64}};
 	constexpr int kTrial = 4, kCands = sizeof kCand / sizeof kCand[0], kNarrowCand = 6;
 	float best = 0;
 	int bestG = 8, bestShare = 1;
-	int cands = narrow ? kNarrowCand : kCands;
+	int cands = all ? kCands : kNarrowCand;
 	if (narrow && (double)h->mm_N[0] * (12 * h->mm_W + 24 * width[0]) < 4e6) {
 		bestShare = bestG = 2;
 		cands = 0;
@@ -1134,18 +1137,20 @@ int run_batch(tbtkx_context *h, const int *num_sites, const int64_t *sites, cons
 	const int cls = narrow ? narrow_class(width[0], h->mm_W) : 0;
 	TunedShape &tuned = narrow ? h->nb_tuned[cls * 4 + mode] : h->mm_tuned;
 	const int64_t key[3] = {h->mm_gen, mode, narrow ? cls : hw};
+	const bool all = !narrow || Smax >= kLongRun;
 	int G = 8, share = 1;
 	if (h->tile_rows > 0) {
 		G = std::max(kRpi, (h->tile_rows + kRpi - 1) / kRpi * kRpi);
 		share = h->grid_share;
 	} else if (h->autotune && Smax > 0) {
-		if (memcmp(key, tuned.key, sizeof key) != 0) {
+		if (memcmp(key, tuned.key, sizeof key) != 0 || (all && !tuned.all)) {
 			// Output sizes are needed to reserve buffers for the trial runs.
 			int64_t mu_elems = 0;
 			for (int m = 0; m < K; m++)
 				mu_elems += dots ? (int64_t)S[m] * 2 * width[m] : out_off[m + 1] - out_off[m];
-			if ((rc = autotune(h, width, S, dots, ncols, mu_elems, narrow, tuned))) return rc;
+			if ((rc = autotune(h, width, S, dots, ncols, mu_elems, narrow, all, tuned))) return rc;
 			memcpy(tuned.key, key, sizeof key);
+			tuned.all = all;
 		}
 		G = tuned.g;
 		share = tuned.share;
