@@ -208,7 +208,9 @@ int tbtkx_moments_block(tbtkx_handle handle, int num_sites,
  * from-index or exact FP64 blocks of 64-256 start vectors through one SpMM
  * per step (CSR order, no fused multiply-add: every column reproduces the
  * plain recurrence bit for bit; two real vectors per column for a real H),
- * whichever moves fewer bytes (TBTKX_OPT_MULTI). This batches the
+ * whichever moves fewer bytes (TBTKX_OPT_MULTI), or, for a model that fits one
+ * workgroup, a resident recurrence per from-index, all in one launch
+ * (TBTKX_OPT_RESIDENT). This batches the
  * reference's sequential per-index recurrences of
  * PropertyExtractor::ChebyshevExpander::calculateGreensFunction (pattern
  * form) and calculateLDOS (Lib/src/PropertyExtractor/ChebyshevExpander.cpp:
@@ -296,8 +298,8 @@ int tbtkx_multi_set_lattices(tbtkx_handle handle, int num_models,
                              const tbtkx_lattice *lattices, const double *const *onsite,
                              const double *scales);
 
-/* Diagonal moments of every uploaded model in one launch per
- * recurrence step: model m gets num_sites[m] (1..64) unit start vectors at
+/* Diagonal moments of every uploaded model in one call, resident
+ * (TBTKX_OPT_RESIDENT) or in one launch per recurrence step: model m gets num_sites[m] (1..64) unit start vectors at
  * its local basis indices (consecutive in sites) and num_moments[m] moments.
  * out holds, model after model, num_sites[m] x num_moments[m] complex values
  * (site-major), as tbtkx_moments_block would give per model. FP32 storage,
