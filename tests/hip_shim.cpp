@@ -23,6 +23,7 @@ int shim_launches = 0;      // kernel launches
 int shim_cooperative = 0;   // cooperative launches
 int shim_refuse = 0;        // 1: cooperative launches are refused (too large)
 int shim_malloc_limit = 0;  // > 0: no device memory for as many bytes or more
+int shim_drop = 0;          // 1: cooperative launches lack their last workgroup
 int shim_no_pinned = 0;     // 1: no pinned host memory
 int shim_give_up = 0;       // 1: a 4-byte result copied to the host reads 1
 
@@ -54,6 +55,7 @@ int hipLaunchCooperativeKernel(const void *f, Dim3 grid, Dim3 block, void **args
 	// GPU. Grids have at most a workgroup per compute unit, and waits are bounded.
 	typedef int (*F)(const void *, Dim3, Dim3, void **, size_t, void *);
 	static F fn = (F)real("hipLaunchKernel");
+	if (shim_drop) grid.x--;
 	if (!shim_refuse) return fn(f, grid, block, args, lds, stream);
 	typedef int (*Malloc)(void **, size_t);
 	static Malloc any_error = (Malloc)real("hipMalloc");

@@ -69,9 +69,12 @@ for name, make in CASES:
 
 
 @pytest.mark.parametrize("name,how,settled", [
-    ("shim_refuse", 1, True), ("shim_malloc_limit", 100000, False), ("shim_give_up", 1, False)])
+    ("shim_refuse", 1, True), ("shim_malloc_limit", 100000, False), ("shim_give_up", 1, False),
+    ("shim_drop", 1, False)])
 def test_step_kernels_take_over(tmp_path, name, how, settled):
-    """A refused launch is not tried again at once; memory and waits are."""
+    """A refused launch is not tried again at once; memory and waits are. Without
+    its last workgroup (shim_drop) a launch's waits for that one's rows end after a
+    second, the others' when they see it, and every workgroup leaves the kernel."""
     run_shimmed(tmp_path, BODY.format(name=name, how=how, settled=settled))
 
 
