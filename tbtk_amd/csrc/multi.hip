@@ -1039,8 +1039,9 @@ constexpr int kLongRun = 128;   // steps of a run that repays trials of every sh
 // (share 0) with tiles of 8-64 row groups. Narrow blocks of fewer than kLongRun steps:
 // the first kNarrowCand, whose best took at most 1.05 of the best of all 12 (8 models of
 // 29,760 to 753,480 rows, 1 to 64 columns; 864,000 rows, 32 columns, 256 steps: 45.5 ms
-// against 44.5, where the other trials take 6 ms once); two row groups per tile without trials where a step moves
-// less than an XCD's L2 holds (3600 to 29,760 rows: at most 1.08 of the best).
+// against 44.5, where the other trials take 6 ms once). Two row groups per tile
+// without trials where a step moves less than an XCD's L2 holds (3600 to 29,760 rows:
+// at most 1.08 of the best).
 int autotune(tbtkx_context *h, const std::vector<int> &width, const std::vector<int> &S,
              bool dots, int ncols, int64_t mu_elems, bool narrow, bool all, TunedShape &tuned) {
 	static const int kCand[][2] = {{1, 2}, {1, 4}, {1, 16}, {2, 2},  {2, 4},  {0, 8},

@@ -18,8 +18,8 @@
 // where no row's sums take registers. Bound by VALU issue (51% of the SIMDs' cycles on
 // the first model below, 37% of it conversions between FP32 and FP64) at two
 // wavefronts per SIMD that wait half of the time, and by the exchange; LDS is busy 23%
-// of the time (32 bytes per entry, row and step). Two workgroups of 4 columns per CU spilled at 8
-// rows (46 us for 16 columns of the first model below against 24).
+// of the time (32 bytes per entry, row and step). Two workgroups of 4 columns per CU
+// spilled at 8 rows (46 us for 16 columns of the first model below against 24).
 // A model too large for one pass takes several launches, 8 columns per team each.
 //
 // Measured per step, the step kernels and this one (dots):
